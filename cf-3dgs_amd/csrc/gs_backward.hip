@@ -8,20 +8,18 @@
 //                    the sequence can be captured in a graph)
 //   k_render_bwd     one chunk per workgroup (16x16 pixels), back to front.
 //                    A chunk that is not the tile's last starts from the
-//                    forward's checkpoint at its end: T_b, and the suffix sums
-//                    (C_final - C_b) / T_b that the back-to-front recurrence
-//                    would have accumulated, so heavy tiles spread over many
-//                    workgroups instead of serialising in one.  T is then
-//                    recovered by division as in the forward's algebra.  The
-//                    10 per-(pixel, Gaussian) terms are summed over the
-//                    wave with permlane swaps + DPP (wave_sum12), the wave
-//                    sums go to LDS accumulators, and each Gaussian of the
-//                    chunk receives one global atomic per term.
-//                    Deterministic mode: each wave keeps its own LDS
-//                    partials (summed in wave order), and the chunk writes one
-//                    10-float partial per (Gaussian, tile) pair into a slot
-//                    of its own (the Gaussian's offset in the Gaussian-order
-//                    tile prefix + the tile's rank in its rect) -- no atomics;
+//                    forward's checkpoint at its end: T_b, and the sum of what
+//                    lies behind it, C_final - C_b, so heavy tiles spread over
+//                    many workgroups instead of serialising in one.  Within
+//                    the chunk 16 entries x 4 pixels go through a wave at a
+//                    time, T and the sum behind each entry by scans over the
+//                    entries (render_bwd_item).  The sums of the Gaussian's 10
+//                    terms over the pixels go to LDS, one set per wave, and
+//                    leave as one global atomic per term.
+//                    Deterministic mode: the chunk writes one 10-float partial
+//                    per (Gaussian, tile) pair into a slot of its own (the
+//                    Gaussian's offset in the Gaussian-order tile prefix + the
+//                    tile's rank in its rect) -- no atomics;
 //   k_det_gather     deterministic mode: per Gaussian, its partials summed in
 //                    rect order (the pose-only backward sums its 5-term
 //                    partials the same way inside k_preprocess_bwd);
@@ -39,10 +37,11 @@
 
 namespace gs {
 
-// render-gradient record: m2x m2y ca cb cc opac r g b depth - -, where ca and
-// cc are the conic gradients times -2: their factor -0.5 is applied to the
-// Gaussian's sum instead of to every pixel's term (a power of two, so the
-// sums and their rounding are exactly the same)
+// render-gradient record, sums over the pixels a Gaussian blends into, with
+// g = G dL/dalpha and (dx, dy) = centre - pixel:
+//   g dx, g dy, g dx^2, g dx dy, g dy^2, g, w dL/dr, w dL/dg, w dL/db,
+//   w dL/ddepth, -, -
+// (k_preprocess_bwd applies the opacity and the conic to the sums)
 constexpr int kRG = 12;
 
 struct RBArgs {
@@ -58,7 +57,7 @@ struct RBArgs {
   const float* ckpt;          // [..][5][256] forward state at batch boundaries
   const uint32_t* ckpt_base;  // [nt + 1]
   const uint32_t* tile_maxc;  // [nt]
-  const uint32_t* items;      // [0] count, then (tile, chunk) pairs, longest estimated first
+  const uint32_t* items;      // [0] count, then from word 4 (tile, chunk, list start, last contributor), longest estimated first
   const uint32_t* item_log;   // the blend's item records: [0] count, then (tile, chunk << 6 | class)
   const float* dL_dcolor;
   const float* dL_ddepth;
@@ -81,7 +80,8 @@ struct RBArgs {
 // the LDS atomics give: no result depends on the order of items
 // (deterministic mode writes one slot per pair; the atomic mode is
 // order-dependent in any case).
-__device__ __forceinline__ void bwd_items(const uint32_t* item_log, uint32_t* items) {
+__device__ __forceinline__ void bwd_items(const uint32_t* item_log, const uint32_t* ranges, const uint32_t* tile_maxc,
+                                          uint32_t* items) {
   __shared__ uint32_t s_cls[64];
   const int t = threadIdx.x;
   const uint32_t n = item_log[0];
@@ -104,8 +104,7 @@ __device__ __forceinline__ void bwd_items(const uint32_t* item_log, uint32_t* it
   for (uint32_t i = t; i < n; i += 1024) {
     const uint32_t tile = item_log[1 + 2 * i], cc = item_log[2 + 2 * i];
     const uint32_t pos = atomicAdd(&s_cls[cc & 63u], 1u);
-    items[1 + 2 * pos] = tile;
-    items[2 + 2 * pos] = cc >> 6;
+    reinterpret_cast<uint4*>(items)[1 + pos] = make_uint4(tile, cc >> 6, ranges[2 * tile], tile_maxc[tile]);
   }
   if (t == 0) items[0] = n;
 }
@@ -121,6 +120,8 @@ struct BwdPrep {
   float* zp;
   long long zn;
   const uint32_t* item_log;
+  const uint32_t* ranges;
+  const uint32_t* tile_maxc;
   uint32_t* items;
   const uint32_t* counters;
   int terms;
@@ -130,7 +131,7 @@ struct BwdPrep {
 __device__ __forceinline__ void bwd_prepare_block(const BwdPrep& p, int bid, int nblocks) {
   const int first = p.items ? 1 : 0;
   if (first && bid == 0) {
-    bwd_items(p.item_log, p.items);
+    bwd_items(p.item_log, p.ranges, p.tile_maxc, p.items);
     return;
   }
   long long zn = p.zn;
@@ -193,293 +194,347 @@ __device__ __forceinline__ void wave_sum12(const float v[12], float w[3]) {
   }
 }
 
-// wave_sum12 of v[0..9] with v[10] = v[11] = 0 (the render backward's 10
-// terms): the last stage-1 sum is the literal 0, not a swap of two zeros.
-__device__ __forceinline__ void wave_sum10(const float v[10], float w[3]) {
-  float u[6];
+// ---- scans over the 16 lanes of each DPP row, four independent chains -------
+// Lane e of a row holds entry e of a group, and the four chains are the four
+// pixels the lane works on.  A DPP operand needs two wait states after the
+// instruction that wrote it, and a transcendental's result one: the leading
+// s_nop covers what came before, and the other three chains' instructions lie
+// between two steps of one chain.  row_shl:n reads lane e + n; lanes past the
+// row's end keep their value.
+#define GS_ROW4(op, n)                                                     \
+  op " %0, %0, %0 row_shl:" #n " row_mask:0xf bank_mask:0xf\n\t"           \
+  op " %1, %1, %1 row_shl:" #n " row_mask:0xf bank_mask:0xf\n\t"           \
+  op " %2, %2, %2 row_shl:" #n " row_mask:0xf bank_mask:0xf\n\t"           \
+  op " %3, %3, %3 row_shl:" #n " row_mask:0xf bank_mask:0xf\n\t"
+// p[q] of lane e = product of the lanes >= e; t_out = t_in times it; t_in then
+// takes the row's whole product.
+__device__ __forceinline__ void row_suffix_product4(float (&p)[4], float (&t)[4], float (&t_out)[4]) {
+  asm("s_nop 1\n\t" GS_ROW4("v_mul_f32_dpp", 1) GS_ROW4("v_mul_f32_dpp", 2) GS_ROW4("v_mul_f32_dpp", 4)
+          GS_ROW4("v_mul_f32_dpp", 8)
+      "v_mul_f32 %8, %0, %4\n\t"
+      "v_mul_f32 %9, %1, %5\n\t"
+      "v_mul_f32 %10, %2, %6\n\t"
+      "v_mul_f32 %11, %3, %7\n\t"
+      "v_mul_f32_dpp %4, %0, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mul_f32_dpp %5, %1, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mul_f32_dpp %6, %2, %6 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_mul_f32_dpp %7, %3, %7 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "+v"(p[0]), "+v"(p[1]), "+v"(p[2]), "+v"(p[3]), "+v"(t[0]), "+v"(t[1]), "+v"(t[2]), "+v"(t[3]),
+        "=&v"(t_out[0]), "=&v"(t_out[1]), "=&v"(t_out[2]), "=&v"(t_out[3]));
+}
+// after[q] of lane e = r[q] + the sum of x[q] over the lanes > e; r then adds
+// the row's whole sum.
+__device__ __forceinline__ void row_suffix_sum4(float (&x)[4], float (&r)[4], float (&after)[4]) {
+  asm("s_nop 1\n\t" GS_ROW4("v_add_f32_dpp", 1) GS_ROW4("v_add_f32_dpp", 2) GS_ROW4("v_add_f32_dpp", 4)
+          GS_ROW4("v_add_f32_dpp", 8)
+      "v_add_f32_dpp %8, %0, %4 row_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_add_f32_dpp %9, %1, %5 row_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_add_f32_dpp %10, %2, %6 row_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_add_f32_dpp %11, %3, %7 row_shl:1 row_mask:0xf bank_mask:0xf bound_ctrl:0\n\t"
+      "v_add_f32_dpp %4, %0, %4 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %5, %1, %5 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %6, %2, %6 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "v_add_f32_dpp %7, %3, %7 row_newbcast:0 row_mask:0xf bank_mask:0xf\n\t"
+      "s_nop 1"
+      : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(r[0]), "+v"(r[1]), "+v"(r[2]), "+v"(r[3]),
+        "=&v"(after[0]), "=&v"(after[1]), "=&v"(after[2]), "=&v"(after[3]));
+}
+#undef GS_ROW4
+
+// The four row values of v[0..N-1] summed over the rows (lanes 16 and 32
+// apart), a reduce-scatter: lane e of row q of w[m] gets value
+// 4 m + {0, 2, 1, 3}[q] of its entry.  Every value is formed as
+// (row 0 + row 2) + (row 1 + row 3), wherever it stands, so the pose-only
+// terms have the same bits with and without the others.
+template <int N>
+__device__ __forceinline__ void rows_reduce(const float (&v)[N], float (&w)[(N + 3) / 4]) {
+  constexpr int M = (N + 3) / 4;
+  float u[2 * M];
 #pragma unroll
-  for (int i = 0; i < 5; ++i) swap_add32(v[2 * i], v[2 * i + 1], u[i]);
-  u[5] = 0.0f;
-#pragma unroll
-  for (int m = 0; m < 3; ++m) {
-    swap_add16(u[2 * m], u[2 * m + 1], w[m]);
-    w[m] = row_sum16(w[m]);
+  for (int i = 0; i < 2 * M; ++i) {
+    if (2 * i + 1 < N) swap_add32(v[2 * i], v[2 * i + 1], u[i]);
+    else if (2 * i < N) swap_add32(v[2 * i], 0.0f, u[i]);
+    else u[i] = 0.0f;
   }
-  // keep the last row step with the reduction: the sums are consumed only
-  // by the storing lanes, and an add sunk into that branch would leave its
-  // DPP permutation as a separate move
-  asm volatile("" : : "v"(w[0]), "v"(w[1]), "v"(w[2]));
+#pragma unroll
+  for (int m = 0; m < M; ++m) swap_add16(u[2 * m], u[2 * m + 1], w[m]);
 }
 
-// DEP: the frame has a depth or an alpha cotangent.  Without one (a colour
-// loss, as in the training step and the pose solve) the depth and alpha
-// terms, their running sums and the depth gradient are identically zero and
-// are not computed.
-// wave_sum10 restricted to v[0..4] (the pose-only backward's terms): each of
-// these five sums is formed by the same operations, in the same lanes, as in
-// wave_sum10, so the two give the same bits.  w[0] rows hold values
-// {0, 2, 1, 3}, row 0 of w[1] value 4.
-__device__ __forceinline__ void wave_sum5(const float v[5], float w[2]) {
-  float u[3];
-  swap_add32(v[0], v[1], u[0]);
-  swap_add32(v[2], v[3], u[1]);
-  swap_add32(v[4], 0.0f, u[2]);
-  swap_add16(u[0], u[1], w[0]);
-  w[0] = row_sum16(w[0]);
-  swap_add16(u[2], 0.0f, w[1]);
-  w[1] = row_sum16(w[1]);
-  asm volatile("" : : "v"(w[0]), "v"(w[1]));  // as in wave_sum10
-}
-
-template <bool B>
-struct BoolTag {
-  static constexpr bool value = B;
-};
-
+// One 256-entry chunk of one tile's list, back to front, by 256 threads.
+//
+// What bounds it is VALU issue: the exact exponential and the gradient of
+// every (pixel, splat) pair.  Three choices keep the instructions per pair low.
+//  * Work is listed per 4 x 4-pixel cell (splat_cells).  On the 500k-Gaussian
+//    training scene 72% of the (pixel, splat) slots of such lists blend, on a
+//    480 x 270 pose frame 45%; on 8 x 8 quadrants it was 48% and 23%.
+//  * A wave takes 16 entries x 4 pixels at a time: lane 16 k + e is entry e at
+//    column k of the cell, and the four rows of the cell are four independent
+//    chains in its registers.  What runs along the list -- the transmittance
+//    and the colour behind an entry -- is a scan over the 16 lanes of a DPP
+//    row, 4 instructions for 64 pairs.  So each entry's gradient terms stay in
+//    its own lanes over the cell's 16 pixels and are summed over the 4 rows of
+//    lanes once per group (rows_reduce), where one entry at a time on 64
+//    pixels needs a 30-instruction wave reduction for every entry.
+//  * Only sums over pixels are formed here: with g = G dL/dalpha the moments
+//    of g in (dx, dy) up to the second order, and w dL/dcolour.  What is
+//    constant per splat (its opacity, its conic) is applied to the sums in
+//    k_preprocess_bwd.
+// The colour recurrence is carried as one number per pixel: with d = colour .
+// dL/dcolour (+ depth and alpha terms), dL/dalpha_k = T_k d_k - R_k / (1 -
+// alpha_k), R_k = the sum of w d over the later entries plus T_final times
+// background . dL/dcolour.
 template <bool DET, bool DEP, bool PO>
 __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) {
   // PO (pose-only, fixed-order, colour cotangent only): the caller wants only
   // the pose gradient, which at active SH degree 0 depends on a splat's
-  // screen position and conic alone, so only those five terms are summed and
+  // screen position and conic alone, so only those five sums are formed and
   // stored per (Gaussian, tile) pair.  Their arithmetic is the full path's,
   // term for term, so the pose gradient has the same bits either way.
   static_assert(!PO || (DET && !DEP), "the pose-only backward is fixed-order and colour-only");
   constexpr int kTerms = PO ? 5 : 10;
-  constexpr int kParts = DET ? 4 : 1;  // LDS partial sets: one per wave when deterministic
-  // The item's 256-entry chunk is staged 128 entries at a time (back half
-  // first): half the LDS per workgroup, so twice as many workgroups fit on a
-  // CU (deterministic mode: 5 instead of 2).  The pixel state carries over.
-  constexpr int kSub = 128;
-  __shared__ uint32_t s_id[kSub];
-  __shared__ float4 s_a[kSub];
-  __shared__ float4 s_b[kSub];
-  __shared__ float4 s_c[kSub];
-  __shared__ uint32_t s_mask[kSub];    // quadrants each staged splat can reach (splat_quads)
-  __shared__ uint8_t s_list[4][kSub];  // per wave: the staged splats that reach its pixels
-  __shared__ float s_acc[kTerms * kParts][kSub];
+  constexpr int kVals = PO ? 5 : (DEP ? 10 : 9);  // (without a depth cotangent its sum is 0)
+  constexpr int kSub = 256;                       // entries of a chunk
+  // LDS sizes decide how many workgroups share a CU: 53 KB for the colour
+  // gradient, so three; 37 KB for the pose-only form, four.
+  __shared__ float4 s_a[kSub];  // x, y, conic a, conic b
+  __shared__ float4 s_b[kSub];  // conic c, opacity, r, g
+  __shared__ float s_c[DEP ? 2 : 1][kSub];  // b, depth
+  __shared__ uint16_t s_mask[kSub];    // cells each staged splat can reach (splat_cells)
+  __shared__ __align__(4) uint8_t s_list[4][kSub];  // per wave: the staged splats that reach the cell at hand
+  // per pixel, cell by cell: T and R at the chunk's end, last contributor, the cotangents
+  __shared__ float2 s_tr[256];
+  __shared__ uint32_t s_last[256];
+  __shared__ float s_d[DEP ? 5 : 3][256];
+  // every wave sums into rows of its own with plain reads and writes: float
+  // adds to LDS from 64 lanes took ~100 cycles each and held the kernel
+  __shared__ float s_acc[4][kSub * kVals];  // [wave][entry][sum]
   if (item >= a.items[0]) return;
-  const int tile = (int)a.items[1 + 2 * item];
-  const uint32_t chunk = a.items[2 + 2 * item];
-  const uint32_t maxc = a.tile_maxc[tile];
+  const uint4 rec = reinterpret_cast<const uint4*>(a.items)[1 + item];
+  const int tile = __builtin_amdgcn_readfirstlane((int)rec.x);
+  const uint32_t chunk = __builtin_amdgcn_readfirstlane((int)rec.y), r0 = __builtin_amdgcn_readfirstlane((int)rec.z);
+  const uint32_t maxc = __builtin_amdgcn_readfirstlane((int)rec.w);
   const uint32_t nchunk = (maxc + 255) / 256;
   const uint32_t cstart = chunk * 256;
   const uint32_t cend = min(cstart + 256, maxc);
   const int tx = tile % a.gx, ty = tile / a.gx;
-  int pdx, pdy;
-  tile_pixel(threadIdx.x, pdx, pdy);
-  const int px = tx * kBX + pdx, py = ty * kBY + pdy;
-  const bool inside = px < a.W && py < a.H;
-  const int pix = py * a.W + px;
-  const int HW = a.W * a.H;
-  const float pfx = (float)px, pfy = (float)py;
-  const uint32_t r0 = a.ranges[2 * tile];
-  const float T_fin = inside ? a.final_T[pix] : 0.0f;
-  const uint32_t last = inside ? a.n_contrib[pix] : 0u;
-  float dpix0 = 0.f, dpix1 = 0.f, dpix2 = 0.f, dD = 0.f, dA = 0.f;
-  // per-pixel state at position cend (the end of this chunk)
-  float T = T_fin;
-  float acc0 = 0.f, acc1 = 0.f, acc2 = 0.f, acc_d = 0.f, acc_a = 0.f;
-  if (inside && last > cstart) {
-    dpix0 = a.dL_dcolor[pix];
-    dpix1 = a.dL_dcolor[HW + pix];
-    dpix2 = a.dL_dcolor[2 * HW + pix];
-    if constexpr (DEP) {
-      if (a.dL_ddepth) dD = a.dL_ddepth[pix];
-      if (a.dL_dalpha) dA = a.dL_dalpha[pix];
-    }
-    if (chunk + 1 < nchunk) {
-      // suffix sums from the forward's state at the boundary: sum_{k >= b} c_k a_k T_k = C_final - C_b
-      const float* ck = a.ckpt + (size_t)(a.ckpt_base[tile] + chunk) * 5 * 256 + threadIdx.x;
-      const float Tb = ck[0];
-      const float inv = 1.0f / Tb;
-      T = Tb;
-      acc0 = (a.accum[pix] - ck[256]) * inv;
-      acc1 = (a.accum[HW + pix] - ck[512]) * inv;
-      acc2 = (a.accum[2 * HW + pix] - ck[768]) * inv;
+  const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  {
+    int pdx, pdy;
+    tile_pixel(threadIdx.x, pdx, pdy);
+    const int px = tx * kBX + pdx, py = ty * kBY + pdy;
+    const bool inside = px < a.W && py < a.H;
+    const int pix = py * a.W + px;
+    const int HW = a.W * a.H;
+    const uint32_t last = inside ? a.n_contrib[pix] : 0u;
+    float T = 0.f, R = 0.f, d0 = 0.f, d1 = 0.f, d2 = 0.f, dD = 0.f, dA = 0.f;
+    if (last > cstart) {
+      d0 = a.dL_dcolor[pix];
+      d1 = a.dL_dcolor[HW + pix];
+      d2 = a.dL_dcolor[2 * HW + pix];
       if constexpr (DEP) {
-        acc_d = (a.accum[3 * HW + pix] - ck[1024]) * inv;
-        acc_a = 1.0f - T_fin * inv;
+        if (a.dL_ddepth) dD = a.dL_ddepth[pix];
+        if (a.dL_dalpha) dA = a.dL_dalpha[pix];
+      }
+      const float T_fin = a.final_T[pix];
+      T = T_fin;
+      R = T_fin * ((a.bg[0] * d0 + a.bg[1] * d1) + a.bg[2] * d2);
+      if (chunk + 1 < nchunk) {
+        // the forward's state at the chunk's end: sum_{k >= b} w_k c_k = C_final - C_b
+        const float* ck = a.ckpt + (size_t)(a.ckpt_base[tile] + chunk) * 5 * 256 + threadIdx.x;
+        T = ck[0];
+        R += (a.accum[pix] - ck[256]) * d0;
+        R += (a.accum[HW + pix] - ck[512]) * d1;
+        R += (a.accum[2 * HW + pix] - ck[768]) * d2;
+        if constexpr (DEP) {
+          R += (a.accum[3 * HW + pix] - ck[1024]) * dD;
+          R += (T - T_fin) * dA;
+        }
+      }
+    }
+    const int slot = ((pdy >> 2) * 4 + (pdx >> 2)) * 16 + (pdy & 3) * 4 + (pdx & 3);
+    s_tr[slot] = make_float2(T, R);
+    s_last[slot] = last;
+    s_d[0][slot] = d0;
+    s_d[1][slot] = d1;
+    s_d[2][slot] = d2;
+    if constexpr (DEP) {
+      s_d[3][slot] = dD;
+      s_d[4][slot] = dA;
+    }
+  }
+  const float a_min = 1.0f / 255.0f;
+  const int e = lane & 15, k = lane >> 4;
+  uint32_t g = 0;   // the thread's entry: its Gaussian
+  int radius = 0;
+  {
+    const uint32_t q = cstart + threadIdx.x;
+    uint32_t m = 0u;
+    if (q < cend) {
+      g = a.list[r0 + q] & a.id_mask;
+      const float4 sa = a.splat[3 * g], sb = a.splat[3 * g + 1], sc = a.splat[3 * g + 2];
+      radius = __float_as_int(sc.w);
+      s_a[threadIdx.x] = sa;
+      s_b[threadIdx.x] = make_float4(sb.x, sb.y, sc.x, sc.y);
+      s_c[0][threadIdx.x] = sc.z;
+      if constexpr (DEP) s_c[1][threadIdx.x] = sb.z;
+      m = splat_cells(sa.x, sa.y, sa.z, sa.w, sb.x, skip_threshold(sb.y), (float)(tx * kBX), (float)(ty * kBY));
+    }
+    s_mask[threadIdx.x] = (uint16_t)m;
+  }
+  for (int i = threadIdx.x; i < 4 * kVals * kSub / 4; i += 256)
+    reinterpret_cast<float4*>(&s_acc[0][0])[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  __syncthreads();
+  uint32_t hits[kSub / 64];
+#pragma unroll
+  for (int c = 0; c < kSub / 64; ++c) hits[c] = s_mask[c * 64 + lane];
+  // The wave's four cells, one in each row and column of the tile's 4 x 4 (a
+  // dense patch of the image then loads all four waves).
+#pragma unroll 1
+  for (int cy = 0; cy < 4; ++cy) {
+    const int cx = (wv + cy) & 3, cell = 4 * cy + cx;
+    float T[4], R[4], dc0[4], dc1[4], dc2[4], dD[4], dA[4];
+    uint32_t last[4];
+    uint32_t cl = 0;  // the cell's last contributor
+#pragma unroll
+    for (int q = 0; q < 4; ++q) {
+      const int at = cell * 16 + 4 * q + k;
+      const float2 tr = s_tr[at];
+      T[q] = tr.x;
+      R[q] = tr.y;
+      last[q] = s_last[at];
+      dc0[q] = s_d[0][at];
+      dc1[q] = s_d[1][at];
+      dc2[q] = s_d[2][at];
+      if constexpr (DEP) {
+        dD[q] = s_d[3][at];
+        dA[q] = s_d[4][at];
+      }
+      cl = max(cl, last[q]);
+    }
+    cl = max(cl, (uint32_t)__shfl_xor((int)cl, 16, 64));
+    cl = max(cl, (uint32_t)__shfl_xor((int)cl, 32, 64));
+    const int lim = cl > cstart ? (int)min(cl - cstart, (uint32_t)kSub) : 0;
+    int n = 0;
+#pragma unroll
+    for (int c = 0; c < kSub / 64; ++c) {
+      const bool hit = c * 64 + lane < lim && ((hits[c] >> cell) & 1u);
+      const uint64_t bal = __ballot(hit);
+      if (hit) s_list[wv][n + __popcll(bal & lanemask_lt())] = (uint8_t)(c * 64 + lane);
+      n += __popcll(bal);
+    }
+    n = __builtin_amdgcn_readfirstlane(n);
+    if (n == 0) continue;
+    __builtin_amdgcn_wave_barrier();
+    const float pfx = (float)(tx * kBX + 4 * cx + k), pfy = (float)(ty * kBY + 4 * cy);
+    for (int i0 = (n - 1) & ~15; i0 >= 0; i0 -= 16) {
+      // What decides which pairs contribute -- the power (blend_power's
+      // operations), spec_expf and the product alpha = o G -- is exactly the
+      // forward's; the forward's pre-test is implied by alpha < 1/255.
+      const bool have = i0 + e < n;
+      const int j = s_list[wv][have ? i0 + e : n - 1];  // (lanes past the list repeat its last entry, inactive)
+      const uint32_t pos = have ? cstart + (uint32_t)j : 0xffffffffu;  // 0-based list position
+      const float4 ga = s_a[j], gb = s_b[j];
+      const float cb = s_c[0][j];
+      const float dx = ga.x - pfx;
+      const float ax = ga.z * dx, bx = ga.w * dx;
+      float dy[4], alpha[4], G[4], d[4], inv[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        dy[q] = ga.y - (pfy + (float)q);
+        const float power = fmaf(-0.5f, fmaf(ax, dx, (gb.x * dy[q]) * dy[q]), -(bx * dy[q]));
+        const float Graw = spec_expf(power);
+        const float araw = fminf(0.99f, gb.y * Graw);
+        const bool active = pos < last[q] && !(power > 0.0f) && !(araw < a_min);
+        alpha[q] = active ? araw : 0.0f;
+        G[q] = active ? Graw : 0.0f;
+        inv[q] = __builtin_amdgcn_rcpf(1.0f - alpha[q]);
+        d[q] = fmaf(cb, dc2[q], fmaf(gb.w, dc1[q], gb.z * dc0[q]));
+        if constexpr (DEP) d[q] = fmaf(s_c[1][j], dD[q], d[q]) + dA[q];
+      }
+      // T before each entry from T after the group, and the sum behind it
+      float Q[4], Tb[4], w[4], X[4], S[4];
+#pragma unroll
+      for (int q = 0; q < 4; ++q) Q[q] = inv[q];
+      row_suffix_product4(Q, T, Tb);
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        w[q] = alpha[q] * Tb[q];
+        X[q] = w[q] * d[q];
+      }
+      row_suffix_sum4(X, R, S);
+      float m0 = 0.f, m1 = 0.f, m2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
+#pragma unroll
+      for (int q = 0; q < 4; ++q) {
+        const float g = G[q] * fmaf(Tb[q], d[q], -(S[q] * inv[q]));
+        const float gy = g * dy[q];
+        m0 += g;
+        m1 += gy;
+        m2 = fmaf(gy, dy[q], m2);
+        if constexpr (!PO) {
+          c0 = fmaf(w[q], dc0[q], c0);
+          c1 = fmaf(w[q], dc1[q], c1);
+          c2 = fmaf(w[q], dc2[q], c2);
+          if constexpr (DEP) c3 = fmaf(w[q], dD[q], c3);
+        }
+      }
+      const float mx = dx * m0;
+      float v[kVals], o[(kVals + 3) / 4];
+      v[0] = mx;
+      v[1] = m1;
+      v[2] = dx * mx;
+      v[3] = dx * m1;
+      v[4] = m2;
+      if constexpr (!PO) {
+        v[5] = m0;
+        v[6] = c0;
+        v[7] = c1;
+        v[8] = c2;
+        if constexpr (DEP) v[9] = c3;
+      }
+      rows_reduce<kVals>(v, o);
+      const int val = k == 1 ? 2 : (k == 2 ? 1 : k);
+#pragma unroll
+      for (int m = 0; m < (kVals + 3) / 4; ++m) {
+        const int t = 4 * m + val;
+        if (have && t < kVals) s_acc[wv][j * kVals + t] += o[m];  // (the entries of a group differ)
       }
     }
   }
-  const float bg_dot = (a.bg[0] * dpix0 + a.bg[1] * dpix1) + a.bg[2] * dpix2;
-  const bool bg_black = a.bg[0] == 0.0f && a.bg[1] == 0.0f && a.bg[2] == 0.0f;
-  const float ddelx = 0.5f * (float)a.W, ddely = 0.5f * (float)a.H;
-  const float a_min = 1.0f / 255.0f;
-  const int lane = threadIdx.x & 63;
-  const int wv = threadIdx.x >> 6;
-  // entries at or past the last contributor of every pixel of the wave are
-  // inactive on every lane
-  const uint32_t wlast = wave_max_u32(last);
-#pragma unroll 1
-  for (int sb = 1; sb >= 0; --sb) {
-    const uint32_t sbase = cstart + (uint32_t)(sb * kSub);
-    if (sbase >= cend) continue;  // (uniform) a chunk of at most 128 entries
-    const uint32_t send = min(sbase + (uint32_t)kSub, cend);
-    __syncthreads();  // the previous half's staged data has been flushed
-    if (threadIdx.x < kSub) {
-      const uint32_t q = sbase + threadIdx.x;
-      uint32_t m = 0u;
-      if (q < send) {
-        const uint32_t g = a.list[r0 + q] & a.id_mask;
-        s_id[threadIdx.x] = g;
-        const float4 sa = a.splat[3 * g];
-        s_a[threadIdx.x] = sa;
-        float4 b = a.splat[3 * g + 1];
-        b.w = skip_threshold(b.y);
-        s_b[threadIdx.x] = b;
-        s_c[threadIdx.x] = a.splat[3 * g + 2];
-        m = splat_quads(sa.x, sa.y, sa.z, sa.w, b.x, b.w, (float)(tx * kBX), (float)(ty * kBY));
-      }
-      s_mask[threadIdx.x] = m;
+  __syncthreads();
+  // The chunk's sums leave with consecutive threads on consecutive words of an
+  // entry's record, so an instruction touches a record's cache line once (one
+  // thread per entry sends every word of a wave's 64 records on its own, and
+  // the atomics of the 500k-Gaussian training scene then held the kernel).
+  const uint32_t ne = cend - cstart;
+  uint32_t* s_to = reinterpret_cast<uint32_t*>(&s_list[0][0]);  // per entry: where its sums go
+  if (threadIdx.x < ne) {
+    uint32_t to = g;
+    if constexpr (DET) {
+      // slot of this (Gaussian, tile) pair: the Gaussian's first slot in the
+      // Gaussian-order prefix of tiles touched + the tile's row-major rank in
+      // its rect (every pair of the list has exactly one chunk)
+      int x0, y0, x1, y1;
+      const float4 sa = s_a[threadIdx.x];
+      tile_rect(sa.x, sa.y, radius, a.gx, a.gy, x0, y0, x1, y1);
+      const uint32_t w = (uint32_t)(x1 - x0);
+      const uint32_t ntg = w * (uint32_t)(y1 - y0);
+      to = a.block_excl[g >> 8] + a.local_incl[g] - ntg + (uint32_t)(ty - y0) * w + (uint32_t)(tx - x0);
     }
-    for (int k = threadIdx.x; k < kTerms * kParts * kSub; k += 256) (&s_acc[0][0])[k] = 0.0f;
-    __syncthreads();
-    // the wave's own list: splats that miss its 8 x 8 pixels are ones no lane would use
-    const int lim = wlast > sbase ? (int)min(wlast - sbase, (uint32_t)kSub) : 0;
-    // (a sum of ballot counts, so wave-uniform; read from the first lane so
-    // that the pair loop below counts in a scalar register)
-    const int nw = __builtin_amdgcn_readfirstlane(compact_wave_list<kSub / 64>(s_mask, s_list[wv], wv, lane, lim));
-    // Branch-free per pair: masked lanes cost a SIMD as much as active ones,
-    // so every lane evaluates the pair; the only branches are wave-uniform
-    // skips when no lane is active.  An inactive lane runs with alpha = G = 0,
-    // which leaves its state unchanged (T / (1 - 0) = T, 0 c + 1 acc = acc) and
-    // makes each of its gradient terms 0, so no per-lane selects are needed.
-    // The running sums acc = sum_{k > current} c_k alpha_k T_k / T_{current+1}
-    // are advanced right after each splat (the reference advances them
-    // lazily at the next one, from last_alpha / last_color; same expression,
-    // same rounding).
-    // The pair loop in two forms: a black background (the reference's
-    // default) adds nothing to dL/dalpha -- its term is a signed zero -- so
-    // that form leaves the term out (the choice is wave-uniform).
-    auto pair_loop = [&](auto bg_on) {
-      for (int i = nw - 1; i >= 0; --i) {
-        // Gradient arithmetic may fuse multiply-adds (the library is built
-        // without contraction for the forward's bit-exactness).  What decides
-        // which pairs contribute -- blend_power, spec_expf and the single
-        // product alpha = o G -- is outside this scope or has no add, so it
-        // stays exactly the forward's.
-  #pragma clang fp contract(fast)
-        const int j = s_list[wv][i];
-        const uint32_t q = sbase + j;  // 0-based list position; contributor index q + 1
-        const float4 ga = s_a[j];
-        const float4 gb = s_b[j];
-        const float dx = ga.x - pfx, dy = ga.y - pfy;
-        const float power = blend_power(ga.z, ga.w, gb.x, dx, dy);
-        // gb.w: alpha < 1/255 for sure below it.  (q < last implies inside:
-        // last is 0 outside the image.)  The wave-uniform skips test the
-        // product of one ballot per compare, which is the ballot of the
-        // conjunction: a ballot of a single compare is that compare's lane mask.
-        const bool in_list = q < last, p_le0 = !(power > 0.0f), p_ge = !(power < gb.w);
-        uint64_t live = __builtin_amdgcn_ballot_w64(in_list) & __builtin_amdgcn_ballot_w64(p_le0) &
-                        __builtin_amdgcn_ballot_w64(p_ge);
-        if (live == 0ull) continue;
-        const float Graw = spec_expf(power);
-        const float alpha_raw = fminf(0.99f, gb.y * Graw);
-        const bool a_ok = !(alpha_raw < a_min);
-        live &= __builtin_amdgcn_ballot_w64(a_ok);
-        if (live == 0ull) continue;
-        const bool active = in_list && p_le0 && p_ge && a_ok;
-        const float G = active ? Graw : 0.0f;
-        const float alpha = active ? alpha_raw : 0.0f;
-        const float4 gc = s_c[j];
-        // T before this splat; the gradient tolerates the 1-ulp reciprocal
-        const float inv_1ma = __builtin_amdgcn_rcpf(1.0f - alpha);
-        const float Tn = T * inv_1ma;
-        const float w = alpha * Tn;
-        float dL_da = (gc.x - acc0) * dpix0;
-        dL_da += (gc.y - acc1) * dpix1;
-        dL_da += (gc.z - acc2) * dpix2;
-        if constexpr (DEP) {
-          dL_da += (gb.z - acc_d) * dD;
-          dL_da += (1.0f - acc_a) * dA;
-        }
-        dL_da *= Tn;
-        if constexpr (decltype(bg_on)::value) dL_da += (-T_fin * inv_1ma) * bg_dot;
-        const float dL_dG = gb.y * dL_da;
-        const float gdx = G * dx, gdy = G * dy;
-        const float dG_dx = -gdx * ga.z - gdy * ga.w;
-        const float dG_dy = -gdy * gb.x - gdx * ga.w;
-        float v[10];
-        v[0] = dL_dG * dG_dx * ddelx;
-        v[1] = dL_dG * dG_dy * ddely;
-        v[2] = gdx * dx * dL_dG;  // times -0.5 in k_preprocess_bwd
-        v[3] = -gdx * dy * dL_dG;
-        v[4] = gdy * dy * dL_dG;  // times -0.5 in k_preprocess_bwd
-        if constexpr (!PO) {
-          v[5] = G * dL_da;
-          v[6] = w * dpix0;
-          v[7] = w * dpix1;
-          v[8] = w * dpix2;
-          v[9] = DEP ? w * dD : 0.0f;
-        }
-        T = Tn;
-        const float oma = 1.0f - alpha;
-        acc0 = alpha * gc.x + oma * acc0;
-        acc1 = alpha * gc.y + oma * acc1;
-        acc2 = alpha * gc.z + oma * acc2;
-        if constexpr (DEP) {
-          acc_d = alpha * gb.z + oma * acc_d;
-          acc_a = alpha + oma * acc_a;
-        }
-        if constexpr (PO) {
-          float w2[2];
-          wave_sum5(v, w2);
-          if ((lane & 15) == 0) {
-            const int q = lane >> 4;
-            const int o = q == 1 ? 2 : (q == 2 ? 1 : q);
-            s_acc[wv * kTerms + o][j] = w2[0];
-            if (q == 0) s_acc[wv * kTerms + 4][j] = w2[1];
-          }
-        } else {
-          float w[3];
-          wave_sum10(v, w);
-          if ((lane & 15) == 0) {
-            const int q = lane >> 4;
-            const int o = q == 1 ? 2 : (q == 2 ? 1 : q);  // value of row q: 4m + {0, 2, 1, 3}[q]
-  #pragma unroll
-            for (int m = 0; m < 3; ++m) {
-              const int k = 4 * m + o;
-              if (k < (DEP ? 10 : 9)) {
-                if constexpr (DET) {
-                  s_acc[wv * 10 + k][j] = w[m];
-                } else {
-                  atomicAdd(&s_acc[k][j], w[m]);  // (a zero adds nothing; testing for it costs more)
-                }
-              }
-            }
-          }
-        }
-      }
-    };
-    if (bg_black) pair_loop(BoolTag<false>{});
-    else pair_loop(BoolTag<true>{});
-    __syncthreads();
-    const uint32_t t = threadIdx.x;
-    if (t < send - sbase) {
-      if constexpr (DET) {
-        // slot of this (Gaussian, tile) pair: the Gaussian's first slot in the
-        // Gaussian-order prefix of tiles touched + the tile's row-major rank in
-        // its rect (every pair of the list has exactly one chunk)
-        const uint32_t g = s_id[t];
-        int x0, y0, x1, y1;
-        tile_rect(s_a[t].x, s_a[t].y, __float_as_int(s_c[t].w), a.gx, a.gy, x0, y0, x1, y1);
-        const uint32_t w = (uint32_t)(x1 - x0);
-        const uint32_t ntg = w * (uint32_t)(y1 - y0);
-        const uint32_t slot =
-            a.block_excl[g >> 8] + a.local_incl[g] - ntg + (uint32_t)(ty - y0) * w + (uint32_t)(tx - x0);
-        float* dst = a.part + (size_t)slot * kTerms;
-#pragma unroll
-        for (int k = 0; k < kTerms; ++k)
-          dst[k] = ((s_acc[k][t] + s_acc[kTerms + k][t]) + s_acc[2 * kTerms + k][t]) + s_acc[3 * kTerms + k][t];
-      } else {
-        float* dst = a.g_render + (size_t)s_id[t] * kRG;
-#pragma unroll
-        for (int k = 0; k < 10; ++k) {
-          const float s = s_acc[k][t];
-          if (s != 0.0f) unsafeAtomicAdd(dst + k, s);
-        }
-      }
+    s_to[threadIdx.x] = to;
+  }
+  __syncthreads();
+  for (uint32_t i = threadIdx.x; i < ne * kTerms; i += 256) {
+    const uint32_t en = i / kTerms, t = i - en * kTerms;
+    float sum = 0.0f;
+    if (t < kVals) {
+      const uint32_t at = en * kVals + t;
+      sum = ((s_acc[0][at] + s_acc[1][at]) + s_acc[2][at]) + s_acc[3][at];
+    }
+    if constexpr (DET) {
+      a.part[(size_t)s_to[en] * kTerms + t] = sum;
+    } else {
+      if (sum != 0.0f) unsafeAtomicAdd(a.g_render + (size_t)s_to[en] * kRG + t, sum);
     }
   }
 }
@@ -714,7 +769,7 @@ __device__ __forceinline__ void preprocess_bwd_block(const PBArgs& a, int bid, f
   if (a.pose) make_pose(a.pose, ps);
   if (i < a.P) {
     const bool vis = a.radii[i] > 0;
-    float4 rA, rB, rC;  // m2x m2y ca cb | cc opac r g | b depth - -
+    float4 rA, rB, rC;  // the render-gradient record, then m2x m2y ca cb | cc opac r g | b depth - -
     if (a.part5) {
       // the sums k_det_gather<5> forms, in its order (terms 5..9 are zero)
       float acc[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
@@ -735,6 +790,18 @@ __device__ __forceinline__ void preprocess_bwd_block(const PBArgs& a, int bid, f
       rA = reinterpret_cast<const float4*>(rg)[0];
       rB = reinterpret_cast<const float4*>(rg)[1];
       rC = reinterpret_cast<const float4*>(rg)[2];
+    }
+    if (vis) {
+      // the record's moments times the splat's constants: dL/dG = o g, dG/ddx =
+      // -G (a dx + b dy) and dG/ddy = -G (c dy + b dx) with a pixel's
+      // displacement in NDC units, dG/da = -G dx^2 / 2, dG/db = -G dx dy,
+      // dG/dc = -G dy^2 / 2 (the factors -0.5 stay out: ca and cc are -2x)
+      const float4 s0 = a.splat[3 * i], s1 = a.splat[3 * i + 1];
+      const float gx = s1.y * rA.x, gy = s1.y * rA.y;
+      const float mx = -(s0.z * gx + s0.w * gy) * (0.5f * (float)a.W);
+      const float my = -(s1.x * gy + s0.w * gx) * (0.5f * (float)a.H);
+      rA = make_float4(mx, my, s1.y * rA.z, -(s1.y * rA.w));
+      rB.x = s1.y * rB.x;
     }
     // (every per-Gaussian output is optional: a pose-only solve asks for none)
     if (a.dL_dmeans2D) {
@@ -1231,6 +1298,8 @@ static BwdPrep bwd_prep_of(const gs_frame_t* f, int P, long long capacity, const
   // binning workspace)
   p.item_log = r.item_log;
   p.items = capacity > 0 && P > 0 ? (uint32_t*)r.items : nullptr;
+  p.ranges = r.ranges;
+  p.tile_maxc = r.tile_maxc;
   const long long nzb = (p.zn + 1023) / 1024;
   *grid = (unsigned)((nzb < 2048 ? nzb : 2048) + (p.items ? 1 : 0));
   return p;

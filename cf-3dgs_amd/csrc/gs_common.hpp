@@ -472,6 +472,62 @@ __device__ __forceinline__ uint32_t splat_quads(float x, float y, float a, float
   return m;
 }
 
+// The 4 x 4-pixel cells of the tile at (x0, y0) that a splat at (x, y) with
+// conic (a, b, c) and pre-test threshold thr can reach: bit 4 cy + cx for the
+// cell whose first pixel is (x0 + 4 cx, y0 + 4 cy).  A pixel outside the
+// returned cells has power < thr, so every kernel skips the pair there.
+//
+// With (u, v) the pixel's offset from the centre the reach is the ellipse
+// Q = a u^2 + 2 b u v + c v^2 <= L, L = -2 thr.  A cell row is the band
+// v in [vlo, vlo + 3]; on the band the ellipse spans
+// u in [(-b v - s(v)) / a, (-b v + s(v)) / a], s(v) = sqrt(a L - det v^2), at
+// its widest where v is nearest the ellipse's own extreme, so two evaluations
+// per row give the columns (16 separate cell tests cost several times more).
+// L is padded for every rounding here and in the kernels' per-pixel power:
+// 0.01 in the exponent, 1e-3 relative and absolute, and 1e-6 a c / det
+// relative -- the terms a u^2 and c v^2 reach L a c / det on the ellipse and
+// cancel against the cross term, so that is the scale the power rounds on.
+// det is formed with its product's rounding error added back, since for a
+// long thin splat a c and b^2 agree in their leading digits; past a c / det =
+// 1e5 (300 times longer than wide) the power itself has no digits to spare and
+// every cell is returned.  The square
+// roots and reciprocals are the 1-ulp instructions; the spans get 2e-3 pixel
+// and 1e-5 of the ellipse's half-width on top.  thr NaN, a conic that is not
+// positive definite or an infinite reach return every cell too; thr >= 0.01
+// returns none.
+__device__ __forceinline__ uint32_t splat_cells(float x, float y, float a, float b, float c, float thr, float x0,
+                                                float y0) {
+  const float L0 = -2.0f * (thr - 0.01f);
+  if (!(L0 > 0.0f)) return thr != thr ? 0xffffu : 0u;
+  const float bb = b * b;
+  const float det = fmaf(a, c, -bb) - fmaf(b, b, -bb);
+  if (!(a > 0.0f) || !(c > 0.0f) || !(a * c < 1e5f * det)) return 0xffffu;
+  const float idet = __builtin_amdgcn_rcpf(det), ia = __builtin_amdgcn_rcpf(a);
+  const float L = fmaf(L0, fmaf(1e-6f * a * c, idet, 1.001f), 1e-3f);
+  if (!(L * a * idet < 1e30f) || !(L * c * idet < 1e30f)) return 0xffffu;
+  const float aL = a * L;
+  const float V = __builtin_amdgcn_sqrtf(aL * idet) * 1.0001f + 2e-3f;  // half-height
+  const float U = __builtin_amdgcn_sqrtf(L * c * idet);                 // half-width
+  const float vs = -(b * U) * __builtin_amdgcn_rcpf(c);                 // v of the right-hand extreme
+  const float pad = fmaf(U, 1e-5f, 2e-3f);
+  const float bx = x - x0, by = y - y0, bia = b * ia;
+  uint32_t m = 0u;
+#pragma unroll
+  for (int r = 0; r < 4; ++r) {
+    const float lo = fmaxf((float)(4 * r) - by, -V), hi = fminf((float)(4 * r + 3) - by, V);
+    const float vr = fminf(hi, fmaxf(lo, vs)), vl = fminf(hi, fmaxf(lo, -vs));
+    const float sr = __builtin_amdgcn_sqrtf(fmaxf(fmaf(-det * vr, vr, aL), 0.0f)) * ia;
+    const float sl = __builtin_amdgcn_sqrtf(fmaxf(fmaf(-det * vl, vl, aL), 0.0f)) * ia;
+    const float right = bx + fmaf(-bia, vr, sr) + pad, left = bx + fmaf(-bia, vl, -sl) - pad;
+    // first cell with 4 cx + 3 >= left, one past the last with 4 cx <= right
+    const int c0 = (int)ceilf(fminf(fmaxf((left - 3.0f) * 0.25f, 0.0f), 4.0f));
+    const int c1 = (int)floorf(fminf(fmaxf(right * 0.25f, -1.0f), 3.0f)) + 1;
+    const uint32_t row = (0xfu << c0) & ((1u << c1) - 1u) & 0xfu;
+    m |= lo <= hi ? row << (4 * r) : 0u;
+  }
+  return m;
+}
+
 // The wave's own list of the staged splats that meet its pixels: positions j
 // < limit (ascending) with bit `wv` set in s_mask[j]; returns the count
 // (wave-uniform).  Needs all 64 lanes active.

@@ -134,10 +134,12 @@ typedef struct gs_binning_layout {
   size_t ckpt;                 /* float[capacity/256 + 1][5][256] blend state at list batch boundaries */
   size_t bweight;              /* uint32[capacity/256 + 2 n_tiles + 2] per (tile, list batch): the blend's
                                   longest per-wave list, the backward's estimate of that chunk's cost */
-  size_t items;                /* uint32[1 + 2 (capacity/256 + n_tiles + 1)] backward work items:
-                                  count, then (tile, chunk) pairs, longest estimated first */
-  size_t item_log;             /* same size: the blend's record of the work items, in completion
-                                  order: count, then (tile, chunk << 6 | cost class) */
+  size_t items;                /* uint32[4 (1 + capacity/256 + n_tiles + 1)] backward work items: count,
+                                  then from word 4 (tile, chunk, list start, last contributor),
+                                  longest estimated first */
+  size_t item_log;             /* uint32[1 + 2 (capacity/256 + n_tiles + 1)] the blend's record of the
+                                  work items, in completion order: count, then
+                                  (tile, chunk << 6 | cost class) */
   size_t total;
 } gs_binning_layout_t;
 

@@ -1,0 +1,43 @@
+"""Tile lists whose lengths fall on the edges of the blend's and the render
+backward's steps (16-entry groups, 256-entry chunks), on an image whose last
+tiles are cut off: images bit for bit and every gradient against the fp32
+oracle, with atomics and in the fixed-order mode.  Tolerances are those of
+test_gpu_forward.py and test_gpu_backward.py."""
+import numpy as np
+import pytest
+import torch
+
+from gpu_helpers import np_, run_gpu, run_oracle
+from gs_hip import scenes
+from test_gpu_backward import _check
+
+pytestmark = pytest.mark.gpu
+
+
+def _stack(n, small):
+    """n faint Gaussians in front of a 21 x 18 image: wide ones that reach
+    every cell of every tile, or small ones that reach a few cells each."""
+    sc = scenes.plain_scene(seed=50 + n, P=n, W=21, H=18)
+    g = torch.Generator().manual_seed(n)
+    sc["means"] = torch.cat([(torch.rand((n, 2), generator=g) - 0.5) * 2.0, 2.0 + 2.0 * torch.rand((n, 1), generator=g)], 1)
+    sc["scales"] = torch.full((n, 3), 0.1 if small else 1.5) * (0.5 + torch.rand((n, 3), generator=g))
+    sc["opacities"] = 0.01 + 0.01 * torch.rand((n, 1), generator=g)
+    sc["bg"] = torch.tensor([0.2, 0.0, 0.7])
+    return sc
+
+
+@pytest.mark.parametrize("small", [False, True], ids=["wide", "small"])
+@pytest.mark.parametrize("n", [1, 15, 16, 17, 63, 65, 255, 256, 257, 512, 529])
+def test_list_lengths(n, small):
+    print("list length", n, "small" if small else "wide", flush=True)
+    sc = _stack(n, small)
+    g = run_gpu(sc, 1)
+    _, _, o = run_oracle(sc, 1)
+    if not small:
+        assert o["num_rendered"] == 4 * n
+    np.testing.assert_array_equal(np_(g["views"]["n_contrib"]), o["n_contrib"])
+    np.testing.assert_array_equal(np_(g["views"]["final_T"]), o["final_T"])
+    for k in ("color", "depth", "alpha"):
+        np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
+    _check(sc, 1, seed=n)
+    _check(sc, 1, seed=n, deterministic=True)
