@@ -314,7 +314,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
   const int tile = __builtin_amdgcn_readfirstlane((int)rec.x);
   const uint32_t chunk = __builtin_amdgcn_readfirstlane((int)rec.y), r0 = __builtin_amdgcn_readfirstlane((int)rec.z);
   const uint32_t maxc = __builtin_amdgcn_readfirstlane((int)rec.w);
-  const uint32_t nchunk = (maxc + 255) / 256;
   const uint32_t cstart = chunk * 256;
   const uint32_t cend = min(cstart + 256, maxc);
   const int tx = tile % a.gx, ty = tile / a.gx;
@@ -339,7 +338,7 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
       const float T_fin = a.final_T[pix];
       T = T_fin;
       R = T_fin * ((a.bg[0] * d0 + a.bg[1] * d1) + a.bg[2] * d2);
-      if (chunk + 1 < nchunk) {
+      if (last > cend) {
         // the forward's state at the chunk's end: sum_{k >= b} w_k c_k = C_final - C_b
         const float* ck = a.ckpt + (size_t)(a.ckpt_base[tile] + chunk) * 5 * 256 + threadIdx.x;
         T = ck[0];
@@ -378,7 +377,7 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
       s_b[threadIdx.x] = make_float4(sb.x, sb.y, sc.x, sc.y);
       s_c[0][threadIdx.x] = sc.z;
       if constexpr (DEP) s_c[1][threadIdx.x] = sb.z;
-      m = splat_cells(sa.x, sa.y, sa.z, sa.w, sb.x, skip_threshold(sb.y), (float)(tx * kBX), (float)(ty * kBY));
+      m = splat_cells(sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, (float)(tx * kBX), (float)(ty * kBY));
     }
     s_mask[threadIdx.x] = (uint16_t)m;
   }

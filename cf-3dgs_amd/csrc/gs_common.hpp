@@ -46,17 +46,6 @@ __device__ __forceinline__ float blend_power(float a, float b, float c, float dx
   return fmaf(-0.5f, q, -((b * dx) * dy));
 }
 
-// Exponent below which o * exp(power) < 1/255 for certain: ln(1/(255 o)) less
-// a 1e-3 margin that covers the rounding of logf, of spec_expf (a few ulp)
-// and of the product.  A Gaussian skipped by `power < threshold` is one the
-// exact test (alpha < 1/255) skips too, so results are unchanged; the test
-// only spares the exponential.  o = 0 gives +inf (always skipped, as the
-// exact test does); o < 0 or NaN give NaN (never skipped here, left to the
-// exact test).
-__device__ __forceinline__ float skip_threshold(float o) {
-  return logf(1.0f / (255.0f * o)) - 1e-3f;
-}
-
 // Saturating float -> int (NaN -> 0).
 __device__ __forceinline__ int sat_i(float f) {
   if (f != f) return 0;
@@ -392,29 +381,6 @@ __device__ __forceinline__ uint64_t lanemask_lt() {
   return lane == 0 ? 0ull : (~0ull >> (64 - lane));
 }
 
-// Pixel-independent form of the same test: an axis-aligned box around the
-// splat centre outside which power < thr - 0.01 everywhere.  The set
-// {power >= thr - 0.01} is the ellipse {Q <= L}, Q = a dx^2 + 2 b dx dy + c dy^2,
-// L = -2 (thr - 0.01), whose bounding box has half-extents sqrt(L c / det) and
-// sqrt(L a / det), det = a c - b^2.  The 0.01 in the exponent, the relative
-// 1e-4 and the absolute 1e-3 pixel on the extents cover the rounding of the
-// per-pixel power and of this computation by orders of magnitude, so a pixel
-// outside the box is one the per-pixel test skips as well.  Returned as
-// (x0, x1, y0, y1); thr NaN or a non-positive-definite conic give an infinite
-// box (never skipped), thr >= 0.01 an empty one (power <= 0 < thr anyway).
-__device__ __forceinline__ float4 splat_box(float x, float y, float a, float b, float c, float thr) {
-  const float inf = __builtin_inff();
-  if (thr != thr) return make_float4(-inf, inf, -inf, inf);
-  const float L = -2.0f * (thr - 0.01f);
-  if (!(L > 0.0f)) return make_float4(inf, -inf, inf, -inf);
-  const float det = a * c - b * b;
-  if (!(det > 0.0f)) return make_float4(-inf, inf, -inf, inf);
-  const float ex = sqrtf(L * c / det) * 1.0001f + 1e-3f;
-  const float ey = sqrtf(L * a / det) * 1.0001f + 1e-3f;
-  if (!(ex == ex) || !(ey == ey)) return make_float4(-inf, inf, -inf, inf);
-  return make_float4(x - ex, x + ex, y - ey, y + ey);
-}
-
 // Pixel (dx, dy) of thread t inside a 16 x 16 tile: wave w = t / 64 takes the
 // 8 x 8 quadrant (w & 1, w >> 1), lane l the pixel (l & 7, l >> 3) in it.  A
 // small splat covers more lanes of an 8 x 8 block than of a 16 x 4 strip.
@@ -424,65 +390,18 @@ __device__ __forceinline__ void tile_pixel(int t, int& dx, int& dy) {
   dy = ((w >> 1) << 3) + (l >> 3);
 }
 
-// Bit w set when the box meets the 8 x 8 pixels of quadrant w of the tile whose
-// first pixel is (x0, y0).
-__device__ __forceinline__ uint32_t wave_quads_hit(float4 bx, float x0, float y0) {
-  uint32_t m = 0u;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    const float qx = x0 + (float)((w & 1) << 3), qy = y0 + (float)((w >> 1) << 3);
-    if (!(bx.y < qx || bx.x > qx + 7.0f || bx.w < qy || bx.z > qy + 7.0f)) m |= 1u << w;
-  }
-  return m;
+// The thread tile_pixel maps to pixel (dx, dy).
+__device__ __forceinline__ int tile_thread(int dx, int dy) {
+  return ((((dy >> 3) << 1) + (dx >> 3)) << 6) + ((dy & 7) << 3) + (dx & 7);
 }
 
-// Quadrants of the tile at (x0, y0) that a splat at (x, y) with conic (a, b, c)
-// and pre-test threshold thr can reach: the box test of wave_quads_hit, then,
-// per quadrant, the exact minimum over its pixel rectangle of
-// Q = a dx^2 + 2 b dx dy + c dy^2 (dx = x - px, dy = y - py): 0 when the centre
-// lies inside, else the least of the four edge minima (a 1-D quadratic each,
-// its vertex clamped to the edge).  A quadrant whose minimum exceeds
-// L = -2 (thr - 0.01), padded by 1e-3 relative + 1e-3, has power below the
-// pre-test threshold at every pixel and is dropped.
-__device__ __forceinline__ float edge_min_q(float a, float b, float c, float u, float vlo, float vhi) {
-  // min over v in [vlo, vhi] of a u^2 + 2 b u v + c v^2 (c > 0)
-  const float v = fminf(vhi, fmaxf(vlo, -(b * u) / c));
-  return a * u * u + 2.0f * b * u * v + c * v * v;
-}
-__device__ __forceinline__ uint32_t splat_quads(float x, float y, float a, float b, float c, float thr, float x0,
-                                                float y0) {
-  uint32_t m = wave_quads_hit(splat_box(x, y, a, b, c, thr), x0, y0);
-  if (m == 0u || thr != thr) return m;
-  const float L = -2.0f * (thr - 0.01f);
-  if (!(a > 0.0f) || !(c > 0.0f) || !(a * c - b * b > 0.0f)) return m;
-  const float lim = L * 1.001f + 1e-3f;
-#pragma unroll
-  for (int w = 0; w < 4; ++w) {
-    if (!((m >> w) & 1u)) continue;
-    const float qx = x0 + (float)((w & 1) << 3), qy = y0 + (float)((w >> 1) << 3);
-    const float dxlo = x - (qx + 7.0f), dxhi = x - qx;
-    const float dylo = y - (qy + 7.0f), dyhi = y - qy;
-    if (dxlo <= 0.0f && dxhi >= 0.0f && dylo <= 0.0f && dyhi >= 0.0f) continue;  // centre inside
-    float q = edge_min_q(a, b, c, dxlo, dylo, dyhi);
-    q = fminf(q, edge_min_q(a, b, c, dxhi, dylo, dyhi));
-    q = fminf(q, edge_min_q(c, b, a, dylo, dxlo, dxhi));
-    q = fminf(q, edge_min_q(c, b, a, dyhi, dxlo, dxhi));
-    if (q > lim) m &= ~(1u << w);
-  }
-  return m;
-}
-
-// The 4 x 4-pixel cells of the tile at (x0, y0) that a splat at (x, y) with
-// conic (a, b, c) and pre-test threshold thr can reach: bit 4 cy + cx for the
-// cell whose first pixel is (x0 + 4 cx, y0 + 4 cy).  A pixel outside the
-// returned cells has power < thr, so every kernel skips the pair there.
-//
-// With (u, v) the pixel's offset from the centre the reach is the ellipse
-// Q = a u^2 + 2 b u v + c v^2 <= L, L = -2 thr.  A cell row is the band
-// v in [vlo, vlo + 3]; on the band the ellipse spans
+// Where a splat at (x, y) with conic (a, b, c) and opacity o can have alpha >=
+// 1/255: the ellipse Q = a u^2 + 2 b u v + c v^2 <= L around its centre, (u, v)
+// the pixel's offset and L = 2 ln(255 o).  On a band of rows the ellipse spans
 // u in [(-b v - s(v)) / a, (-b v + s(v)) / a], s(v) = sqrt(a L - det v^2), at
 // its widest where v is nearest the ellipse's own extreme, so two evaluations
-// per row give the columns (16 separate cell tests cost several times more).
+// give the columns it reaches on the band.  A pixel outside is one that every
+// kernel skips.
 // L is padded for every rounding here and in the kernels' per-pixel power:
 // 0.01 in the exponent, 1e-3 relative and absolute, and 1e-6 a c / det
 // relative -- the terms a u^2 and c v^2 reach L a c / det on the ellipse and
@@ -490,60 +409,72 @@ __device__ __forceinline__ uint32_t splat_quads(float x, float y, float a, float
 // det is formed with its product's rounding error added back, since for a
 // long thin splat a c and b^2 agree in their leading digits; past a c / det =
 // 1e5 (300 times longer than wide) the power itself has no digits to spare and
-// every cell is returned.  The square
-// roots and reciprocals are the 1-ulp instructions; the spans get 2e-3 pixel
-// and 1e-5 of the ellipse's half-width on top.  thr NaN, a conic that is not
-// positive definite or an infinite reach return every cell too; thr >= 0.01
-// returns none.
-__device__ __forceinline__ uint32_t splat_cells(float x, float y, float a, float b, float c, float thr, float x0,
+// the splat counts as reaching everything.  So does one with o < 0 or NaN, a
+// conic that is not positive definite or an infinite reach.  The logarithm,
+// square roots and reciprocals are the 1-ulp instructions; the spans get 2e-3
+// pixel and 1e-5 of the ellipse's half-width on top.
+struct SplatReach {
+  bool none, all;
+  float bia, ia, mdet, aL, vs, V, pad;
+  __device__ __forceinline__ SplatReach(float a, float b, float c, float o) {
+    const float L0 = 2.0f * (0.693147182f * __builtin_amdgcn_logf(255.0f * o) + 0.01f);
+    const float bb = b * b;
+    const float det = fmaf(a, c, -bb) - fmaf(b, b, -bb);
+    const float idet = __builtin_amdgcn_rcpf(det);
+    const float L = fmaf(L0, fmaf(1e-6f * a * c, idet, 1.001f), 1e-3f);
+    none = L0 <= 0.0f;
+    ia = __builtin_amdgcn_rcpf(a);
+    aL = a * L;
+    const float cL = c * L;
+    all = !(L0 > 0.0f) || !(a > 0.0f) || !(c > 0.0f) || !(a * c < 1e5f * det) || !(aL * idet < 1e30f) ||
+          !(cL * idet < 1e30f);
+    mdet = -det;
+    bia = b * ia;
+    V = __builtin_amdgcn_sqrtf(aL * idet) * 1.0001f + 2e-3f;  // half-height
+    const float U = __builtin_amdgcn_sqrtf(cL * idet);        // half-width
+    vs = -(b * U) * __builtin_amdgcn_rcpf(c);                 // v of the right-hand extreme
+    pad = fmaf(U, 1e-5f, 2e-3f);
+  }
+  // columns [left, right] relative to the centre on the rows [lo, hi]; false: none
+  __device__ __forceinline__ bool band(float lo, float hi, float& left, float& right) const {
+    lo = fmaxf(lo, -V);
+    hi = fminf(hi, V);
+    const float vr = fminf(hi, fmaxf(lo, vs)), vl = fminf(hi, fmaxf(lo, -vs));
+    right = fmaf(-bia, vr, __builtin_amdgcn_sqrtf(fmaxf(fmaf(mdet * vr, vr, aL), 0.0f)) * ia) + pad;
+    left = fmaf(-bia, vl, -(__builtin_amdgcn_sqrtf(fmaxf(fmaf(mdet * vl, vl, aL), 0.0f)) * ia)) - pad;
+    return lo <= hi;
+  }
+};
+
+// Whether the splat can reach the w x h pixels whose first is (x0, y0).
+__device__ __forceinline__ bool splat_reaches(float x, float y, float a, float b, float c, float o, float x0, float y0,
+                                              float w, float h) {
+  const SplatReach r(a, b, c, o);
+  const float u = x0 - x, v = y0 - y;
+  float left, right;
+  const bool hit = r.band(v, v + (h - 1.0f), left, right) && left <= u + (w - 1.0f) && right >= u;
+  return !r.none && (r.all || hit);
+}
+
+// The 4 x 4-pixel cells of the tile at (x0, y0) that the splat can reach: bit
+// 4 cy + cx for the cell whose first pixel is (x0 + 4 cx, y0 + 4 cy).  One
+// band per cell row (16 separate cell tests cost several times more).
+__device__ __forceinline__ uint32_t splat_cells(float x, float y, float a, float b, float c, float o, float x0,
                                                 float y0) {
-  const float L0 = -2.0f * (thr - 0.01f);
-  if (!(L0 > 0.0f)) return thr != thr ? 0xffffu : 0u;
-  const float bb = b * b;
-  const float det = fmaf(a, c, -bb) - fmaf(b, b, -bb);
-  if (!(a > 0.0f) || !(c > 0.0f) || !(a * c < 1e5f * det)) return 0xffffu;
-  const float idet = __builtin_amdgcn_rcpf(det), ia = __builtin_amdgcn_rcpf(a);
-  const float L = fmaf(L0, fmaf(1e-6f * a * c, idet, 1.001f), 1e-3f);
-  if (!(L * a * idet < 1e30f) || !(L * c * idet < 1e30f)) return 0xffffu;
-  const float aL = a * L;
-  const float V = __builtin_amdgcn_sqrtf(aL * idet) * 1.0001f + 2e-3f;  // half-height
-  const float U = __builtin_amdgcn_sqrtf(L * c * idet);                 // half-width
-  const float vs = -(b * U) * __builtin_amdgcn_rcpf(c);                 // v of the right-hand extreme
-  const float pad = fmaf(U, 1e-5f, 2e-3f);
-  const float bx = x - x0, by = y - y0, bia = b * ia;
+  const SplatReach e(a, b, c, o);
+  const float bx = x - x0, v0 = y0 - y;
   uint32_t m = 0u;
 #pragma unroll
   for (int r = 0; r < 4; ++r) {
-    const float lo = fmaxf((float)(4 * r) - by, -V), hi = fminf((float)(4 * r + 3) - by, V);
-    const float vr = fminf(hi, fmaxf(lo, vs)), vl = fminf(hi, fmaxf(lo, -vs));
-    const float sr = __builtin_amdgcn_sqrtf(fmaxf(fmaf(-det * vr, vr, aL), 0.0f)) * ia;
-    const float sl = __builtin_amdgcn_sqrtf(fmaxf(fmaf(-det * vl, vl, aL), 0.0f)) * ia;
-    const float right = bx + fmaf(-bia, vr, sr) + pad, left = bx + fmaf(-bia, vl, -sl) - pad;
+    float left, right;
+    const bool hit = e.band(v0 + (float)(4 * r), v0 + (float)(4 * r + 3), left, right);
     // first cell with 4 cx + 3 >= left, one past the last with 4 cx <= right
-    const int c0 = (int)ceilf(fminf(fmaxf((left - 3.0f) * 0.25f, 0.0f), 4.0f));
-    const int c1 = (int)floorf(fminf(fmaxf(right * 0.25f, -1.0f), 3.0f)) + 1;
+    const int c0 = (int)ceilf(fminf(fmaxf((left + bx - 3.0f) * 0.25f, 0.0f), 4.0f));
+    const int c1 = (int)floorf(fminf(fmaxf((right + bx) * 0.25f, -1.0f), 3.0f)) + 1;
     const uint32_t row = (0xfu << c0) & ((1u << c1) - 1u) & 0xfu;
-    m |= lo <= hi ? row << (4 * r) : 0u;
+    m |= hit ? row << (4 * r) : 0u;
   }
-  return m;
-}
-
-// The wave's own list of the staged splats that meet its pixels: positions j
-// < limit (ascending) with bit `wv` set in s_mask[j]; returns the count
-// (wave-uniform).  Needs all 64 lanes active.
-template <int NC = 4>  // staged entries: NC * 64
-__device__ __forceinline__ int compact_wave_list(const uint32_t* s_mask, uint8_t* s_list, int wv, int lane,
-                                                 int limit = NC * 64) {
-  int n = 0;
-#pragma unroll
-  for (int c = 0; c < NC; ++c) {
-    const int idx = c * 64 + lane;
-    const bool hit = idx < limit && ((s_mask[idx] >> wv) & 1u);
-    const uint64_t bal = __ballot(hit);
-    if (hit) s_list[n + __popcll(bal & lanemask_lt())] = (uint8_t)idx;
-    n += __popcll(bal);
-  }
-  return n;
+  return e.none ? 0u : (e.all ? 0xffffu : m);
 }
 
 // Block id -> logical id so that each of the 8 XCDs (dispatch is round-robin

@@ -14,14 +14,16 @@
 //   (the depth-first schedule instead sorts the Gaussians by depth, expands
 //   them into tile ids in that order (k_df_*), sorts on the tile bits alone,
 //   and records the tile ranges in that sort's last pass)
-//   k_blend        one 16x16 tile per 256-thread workgroup; splats staged in
-//                  LDS 256 at a time, each wave keeping its own list of the
-//                  staged splats whose alpha can reach 1/255 on its 8 x 8
-//                  pixels (splat_box); block-wide vote ends the tile early
-//                  once every pixel is saturated; XCD-aware tile order.
+//   k_blend        single-wave workgroups, each one block of a 16x16 tile's
+//                  pixels: 8 x 8, or 4 x 4 with four list entries at a time
+//                  per pixel where the launch is small; the wave streams the
+//                  tile's list, keeps the splats whose alpha can reach 1/255
+//                  on its block and stops when its pixels are saturated; a
+//                  tile's waves share an XCD.
 #include "gs_common.hpp"
 #include "gs_internal.hpp"
 
+#include <type_traits>
 #include <vector>
 
 namespace gs {
@@ -583,161 +585,297 @@ struct BlendArgs {
   const uint32_t* ckpt_base;
   float* ckpt;
   uint32_t* tile_maxc;
+  uint32_t* tile_done;
   const uint32_t* tile_order;  // the tiles, longest list first (k_tile_ckpt_scan)
   float* accum;
-  // per (tile, batch) at ckpt_base[tile] + tile + batch: the longest
-  // per-wave list of the batch, the backward's cost estimate for that chunk
+  // per (tile, batch) at ckpt_base[tile] + tile + batch: the entries the tile's
+  // waves kept of the batch, the backward's cost estimate for that chunk
   uint32_t* bweight;
   // the backward's work items, appended as tiles finish: [0] count, then
-  // (tile, chunk << 6 | cost class) -- cleared by k_tile_ckpt_scan
+  // (tile, chunk << 6 | cost class)
+  // (these, tile_maxc and tile_done, the waves that are through with the
+  // tile, are cleared by k_tile_ckpt_scan)
   uint32_t* item_log;
 };
 
-__device__ __forceinline__ void blend_tile(const BlendArgs& a, uint32_t tile) {
-  __shared__ float4 s_a[256];  // x, y, conic a, conic b
-  __shared__ float4 s_b[256];  // conic c, opacity, depth, -
-  __shared__ float4 s_c[256];  // r, g, b, -
-  __shared__ uint32_t s_mask[256];    // wave rows each staged splat can reach (splat_box)
-  __shared__ __align__(4) uint8_t s_list[4][256];  // per wave: the staged splats that reach its 8 x 8 pixels
-  __shared__ uint32_t s_maxc;
-  __shared__ uint32_t s_bw;  // longest per-wave list of the current batch
+// spec_expf of four values, instruction by instruction side by side.  A wave
+// issues a dependent instruction every ~10 clocks and an independent one every
+// ~6, and a SIMD takes one every 2, so four chains after one another leave a
+// launch of few waves waiting; the compiler's scheduler does not mix them.
+__device__ __forceinline__ void spec_expf4(const float (&x)[4], float (&p)[4]) {
+  float r[4], k[4];
+  const float c6 = 1.38888892e-03f;
+#define GS_X4(i0, i1, i2, i3) i0 "\n\t" i1 "\n\t" i2 "\n\t" i3 "\n\t"
+  asm(GS_X4("v_max_f32 %4, 0xc2a00000, %12", "v_max_f32 %5, 0xc2a00000, %13", "v_max_f32 %6, 0xc2a00000, %14",
+            "v_max_f32 %7, 0xc2a00000, %15")
+      GS_X4("v_mul_f32 %8, 0x3fb8aa3b, %4", "v_mul_f32 %9, 0x3fb8aa3b, %5", "v_mul_f32 %10, 0x3fb8aa3b, %6",
+            "v_mul_f32 %11, 0x3fb8aa3b, %7")
+      GS_X4("v_rndne_f32 %8, %8", "v_rndne_f32 %9, %9", "v_rndne_f32 %10, %10", "v_rndne_f32 %11, %11")
+      GS_X4("v_fmac_f32 %4, 0xbf317000, %8", "v_fmac_f32 %5, 0xbf317000, %9", "v_fmac_f32 %6, 0xbf317000, %10",
+            "v_fmac_f32 %7, 0xbf317000, %11")
+      GS_X4("v_fmac_f32 %4, 0xb805fdf4, %8", "v_fmac_f32 %5, 0xb805fdf4, %9", "v_fmac_f32 %6, 0xb805fdf4, %10",
+            "v_fmac_f32 %7, 0xb805fdf4, %11")
+      GS_X4("v_fmamk_f32 %0, %4, 0x39500d01, %16", "v_fmamk_f32 %1, %5, 0x39500d01, %16",
+            "v_fmamk_f32 %2, %6, 0x39500d01, %16", "v_fmamk_f32 %3, %7, 0x39500d01, %16")
+      GS_X4("v_fmaak_f32 %0, %0, %4, 0x3c088889", "v_fmaak_f32 %1, %1, %5, 0x3c088889",
+            "v_fmaak_f32 %2, %2, %6, 0x3c088889", "v_fmaak_f32 %3, %3, %7, 0x3c088889")
+      GS_X4("v_fmaak_f32 %0, %0, %4, 0x3d2aaaab", "v_fmaak_f32 %1, %1, %5, 0x3d2aaaab",
+            "v_fmaak_f32 %2, %2, %6, 0x3d2aaaab", "v_fmaak_f32 %3, %3, %7, 0x3d2aaaab")
+      GS_X4("v_fmaak_f32 %0, %0, %4, 0x3e2aaaab", "v_fmaak_f32 %1, %1, %5, 0x3e2aaaab",
+            "v_fmaak_f32 %2, %2, %6, 0x3e2aaaab", "v_fmaak_f32 %3, %3, %7, 0x3e2aaaab")
+      GS_X4("v_fma_f32 %0, %0, %4, 0.5", "v_fma_f32 %1, %1, %5, 0.5", "v_fma_f32 %2, %2, %6, 0.5",
+            "v_fma_f32 %3, %3, %7, 0.5")
+      GS_X4("v_cvt_i32_f32 %8, %8", "v_cvt_i32_f32 %9, %9", "v_cvt_i32_f32 %10, %10", "v_cvt_i32_f32 %11, %11")
+      GS_X4("v_fma_f32 %0, %0, %4, 1.0", "v_fma_f32 %1, %1, %5, 1.0", "v_fma_f32 %2, %2, %6, 1.0",
+            "v_fma_f32 %3, %3, %7, 1.0")
+      GS_X4("v_fma_f32 %0, %0, %4, 1.0", "v_fma_f32 %1, %1, %5, 1.0", "v_fma_f32 %2, %2, %6, 1.0",
+            "v_fma_f32 %3, %3, %7, 1.0")
+      GS_X4("v_ldexp_f32 %0, %0, %8", "v_ldexp_f32 %1, %1, %9", "v_ldexp_f32 %2, %2, %10", "v_ldexp_f32 %3, %3, %11")
+      : "=&v"(p[0]), "=&v"(p[1]), "=&v"(p[2]), "=&v"(p[3]), "=&v"(r[0]), "=&v"(r[1]), "=&v"(r[2]), "=&v"(r[3]),
+        "=&v"(k[0]), "=&v"(k[1]), "=&v"(k[2]), "=&v"(k[3])
+      : "v"(x[0]), "v"(x[1]), "v"(x[2]), "v"(x[3]), "v"(c6));
+#undef GS_X4
+}
+
+// One block of 64 / E pixels of a tile by one wave: 8 x 8 pixels (E = 1) or 4 x
+// 4 (4); block `part` of the tile's 4 E.
+//
+// Lane E p + e looks at entries e, E + e, .. of 4 E at pixel p of the block.  A
+// pixel's alphas are evaluated at once -- they do not depend on each other --
+// and applied in list order by its E lanes together: all carry T, each the sums
+// of 4 / E of the channels r, g, b, depth.  A pixel that saturates needs no
+// branch: T only falls, so an entry counts while T after it is at least 1e-4.
+// A (64-pixel, entry) step costs about 42 or 56 instructions.
+//
+// A wave streams the tile's list on its own, 64 entries at a time, with the ids
+// of window w + 2 and the splats of window w + 1 in flight while window w is
+// blended, keeps the entries that reach its block (splat_reaches) and stops
+// when its own pixels are opaque.  With the list staged for the whole tile, a
+// batch of 256 entries took two barriers and a chain of two dependent loads,
+// and the heaviest tiles' nine batches set the launch's length: 162 us at
+// 500 000 Gaussians and 960 x 540, 150 at 60 000 and 479 x 270, 318 at 1 200 000
+// and 1920 x 1080; now 107, 50 and 270, bound by instructions (the first and the
+// last) and by the longest wave's chain (the second).
+// Workgroups of one wave, so that a wave that is done leaves its place to the
+// next (with eight waves a workgroup, half of the wave slots stood empty).
+//
+// A smaller block wastes fewer lanes (on the training scene 48% of the lanes
+// of an 8 x 8 block blend, 72% of a 4 x 4 block's; on a 480 x 270 pose frame 23%
+// and 45%) and makes the wave's chain shorter, but every wave reads and tests
+// the whole list, ~130 instructions per 64 entries.
+template <int E>
+__device__ __forceinline__ void blend_block(const BlendArgs& a, uint32_t tile, int part) {
+  constexpr int kBlocks = 4 * E, kCh = 4 / E, kGroup = 4 * E;
+  constexpr int kBW = E == 4 ? 4 : 8, kBH = kBW;  // the block's pixels
+  constexpr int kSlots = 64 + 2 * kGroup;  // 64 new entries, those left over and the last group past them
+  __shared__ float4 s_geo[kSlots];   // x, y, conic a, conic b
+  __shared__ float2 s_op[kSlots];    // conic c, opacity
+  __shared__ float4 s_ch[kSlots];    // r, g, b, depth
+  __shared__ uint32_t s_pos[kSlots]; // position in the list + 1
   const int tx = tile % a.gx, ty = tile / a.gx;
-  int pdx, pdy;
-  tile_pixel(threadIdx.x, pdx, pdy);
-  const int px = tx * kBX + pdx, py = ty * kBY + pdy;
+  const int lane = threadIdx.x & 63;
+  const int p = lane / E, e = lane % E;
+  const int bx = (part % (kBX / kBW)) * kBW, by = (part / (kBX / kBW)) * kBH;
+  const int dx = bx + p % kBW, dy = by + p / kBW;
+  const int px = tx * kBX + dx, py = ty * kBY + dy;
   const bool inside = px < a.W && py < a.H;
   const float pfx = (float)px, pfy = (float)py;
-  const int wv = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const uint32_t r0 = a.ranges[2 * tile], r1 = a.ranges[2 * tile + 1];
+  const uint32_t r0 = a.ranges[2 * tile], n = a.ranges[2 * tile + 1] - r0;
+  const uint32_t* list = a.list + r0;
+  const uint32_t base = a.ckpt_base[tile];
   bool done = !inside;
-  float T = 1.0f, C0 = 0.0f, C1 = 0.0f, C2 = 0.0f, D = 0.0f;
+  float T = 1.0f, C[kCh];
+#pragma unroll
+  for (int c = 0; c < kCh; ++c) C[c] = 0.0f;
   uint32_t last = 0;
-  const float a_min = 1.0f / 255.0f;
-  if (threadIdx.x == 0) s_maxc = 0;
-  uint32_t batch = 0;
-  for (uint32_t base = r0; base < r1; base += 256, ++batch) {
-    if (batch > 0 && inside) {
-      float* ck = a.ckpt + (size_t)(a.ckpt_base[tile] + batch - 1) * 5 * 256 + threadIdx.x;
-      ck[0] = T;
-      ck[256] = C0;
-      ck[512] = C1;
-      ck[768] = C2;
-      ck[1024] = D;
+  const float a_min = 1.0f / 255.0f, t_min = 0.0001f;
+  // value v of lane k of this lane's pixel
+  auto of_lane = [](float v, int k) {
+    if constexpr (E == 1) return v;
+    if constexpr (E == 4) return k == 0 ? dpp<0x00>(v) : (k == 1 ? dpp<0x55>(v) : (k == 2 ? dpp<0xAA>(v) : dpp<0xFF>(v)));
+  };
+  if (n > 0 && __ballot(inside)) {
+    const uint32_t nwin = (n + 63u) / 64u;
+    auto id_at = [&](uint32_t w) { return list[min(w * 64u + (uint32_t)lane, n - 1u)] & a.id_mask; };
+    uint32_t id = id_at(0);
+    float4 sa = a.splat[3 * id], sb = a.splat[3 * id + 1], sc = a.splat[3 * id + 2];
+    id = id_at(1);
+    uint32_t have = 0;   // entries in the slots
+    uint32_t count = 0;  // entries kept of this 256-entry batch
+    uint32_t w = 0;
+    for (; w < nwin; ++w) {
+      const float4 ea = sa, eb = sb, ec = sc;
+      sa = a.splat[3 * id];
+      sb = a.splat[3 * id + 1];
+      sc = a.splat[3 * id + 2];
+      id = id_at(w + 2);
+      if ((w & 3u) == 0 && w > 0) {
+        // a 256-entry boundary: the state the backward resumes from
+        const uint32_t batch = w >> 2;
+        if (lane == 0 && count > 0) atomicAdd(&a.bweight[base + tile + batch - 1], count);
+        count = 0;
+        if (inside) {
+          float* ck = a.ckpt + (size_t)(base + batch - 1) * 5 * 256 + tile_thread(dx, dy);
+          if (e == 0) ck[0] = T;
+#pragma unroll
+          for (int c = 0; c < kCh; ++c) ck[256 * (1 + kCh * e + c)] = C[c];
+        }
+      }
+      const uint32_t pos = w * 64u + (uint32_t)lane;
+      const bool hit = pos < n && splat_reaches(ea.x, ea.y, ea.z, ea.w, eb.x, eb.y, (float)(tx * kBX + bx),
+                                                (float)(ty * kBY + by), (float)kBW, (float)kBH);
+      const uint64_t hits = __ballot(hit);
+      if (hit) {
+        const uint32_t slot = have + (uint32_t)__popcll(hits & lanemask_lt());
+        s_geo[slot] = ea;
+        s_op[slot] = make_float2(eb.x, eb.y);
+        s_ch[slot] = make_float4(ec.x, ec.y, ec.z, eb.z);
+        s_pos[slot] = pos + 1u;
+      }
+      // a colour that is not finite must not meet a weight of zero
+      const bool odd = __ballot(hit && !(fabsf(ec.x) + fabsf(ec.y) + fabsf(ec.z) < __builtin_inff())) != 0;
+      have += (uint32_t)__popcll(hits);
+      count += (uint32_t)__popcll(hits);
+      const bool flush = (w & 3u) == 3u || w + 1 == nwin;
+      // the slots that fill up the last group weigh nothing
+      if (flush && lane < kGroup) {
+        s_op[have + lane] = make_float2(0.0f, 0.0f);
+        s_ch[have + lane] = make_float4(0.0f, 0.0f, 0.0f, 0.0f);
+      }
+      __builtin_amdgcn_wave_barrier();
+      uint32_t at = 0;
+      int hit_slot = -1;  // of the lane's last contributor in this window
+      for (; at + kGroup <= have || (flush && at < have); at += kGroup) {
+        const float* ch = &s_ch[at].x + kCh * e;
+        float pw[4], ex[4], al[4];
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const float4 ga = s_geo[at + s * E + e];
+          pw[s] = blend_power(ga.z, ga.w, s_op[at + s * E + e].x, ga.x - pfx, ga.y - pfy);
+        }
+        spec_expf4(pw, ex);
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          const float araw = fminf(0.99f, s_op[at + s * E + e].y * ex[s]);
+          // an entry that is skipped, or a pixel that is done, has alpha 0
+          al[s] = pw[s] > 0.0f || araw < a_min || done ? 0.0f : araw;
+        }
+        float wt[kGroup], Tn = T;
+        bool ok = true;
+#pragma unroll
+        for (int i = 0; i < kGroup; ++i) {
+          const float Ti = Tn * of_lane(1.0f - al[i / E], i % E);
+          ok = !(Ti < t_min);
+          wt[i] = ok ? of_lane(al[i / E], i % E) * Tn : 0.0f;
+          Tn = Ti;
+          T = ok ? Ti : T;
+        }
+        done = done || !ok;
+        if (!odd) {
+#pragma unroll
+          for (int i = 0; i < kGroup; ++i)
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) C[c] = fmaf(ch[4 * i + c], wt[i], C[c]);
+        } else {
+#pragma unroll
+          for (int i = 0; i < kGroup; ++i)
+#pragma unroll
+            for (int c = 0; c < kCh; ++c) C[c] = wt[i] != 0.0f ? fmaf(ch[4 * i + c], wt[i], C[c]) : C[c];
+        }
+#pragma unroll
+        for (int s = 0; s < 4; ++s) {
+          float mine = wt[s * E];
+          if constexpr (E == 4)
+            mine = e == 1 ? wt[s * E + 1] : (e == 2 ? wt[s * E + 2] : (e == 3 ? wt[s * E + 3] : mine));
+          hit_slot = mine != 0.0f ? (int)at + s * E + e : hit_slot;
+        }
+      }
+      if (hit_slot >= 0) last = s_pos[hit_slot];
+      if (__ballot(!done) == 0) break;
+      // the entries left over wait for the next window
+      have = at < have ? have - at : 0u;
+      if (at > 0 && (uint32_t)lane < have) {
+        const float4 g = s_geo[at + lane], c = s_ch[at + lane];
+        const float2 o = s_op[at + lane];
+        const uint32_t q = s_pos[at + lane];
+        s_geo[lane] = g;
+        s_op[lane] = o;
+        s_ch[lane] = c;
+        s_pos[lane] = q;
+      }
+      __builtin_amdgcn_wave_barrier();
     }
-    if (__syncthreads_count(done) == 256) break;
-    if (threadIdx.x == 0) {
-      if (batch > 0) a.bweight[a.ckpt_base[tile] + tile + batch - 1] = s_bw;
-      s_bw = 0;
-    }
-    const uint32_t k = base + threadIdx.x;
-    uint32_t m = 0u;
-    if (k < r1) {
-      const uint32_t g = a.list[k] & a.id_mask;
-      const float4 sa = a.splat[3 * g];
-      s_a[threadIdx.x] = sa;
-      float4 b = a.splat[3 * g + 1];
-      b.w = skip_threshold(b.y);  // (the clamp bits in .w are not needed here)
-      s_b[threadIdx.x] = b;
-      s_c[threadIdx.x] = a.splat[3 * g + 2];
-      m = splat_quads(sa.x, sa.y, sa.z, sa.w, b.x, b.w, (float)(tx * kBX), (float)(ty * kBY));
-    }
-    s_mask[threadIdx.x] = m;
-    __syncthreads();
-    // a splat that misses the wave's pixels is one every lane would skip
-    const int nw = compact_wave_list(s_mask, s_list[wv], wv, lane);
-    if (lane == 0) atomicMax(&s_bw, (uint32_t)nw);
-    const uint32_t first = base - r0 + 1;  // contributor index of staged position 0
-    // alpha of staged splat j at this pixel, 0 when it is skipped.  Branch
-    // free (the exponential is evaluated and then discarded for skipped
-    // pairs), so the loads and exponentials of the entries of one step
-    // overlap instead of each waiting behind its own branch.
-    auto alpha_at = [&](int j) -> float {
-      const float4 ga = s_a[j];
-      const float4 gb = s_b[j];
-      const float dx = ga.x - pfx, dy = ga.y - pfy;
-      const float power = blend_power(ga.z, ga.w, gb.x, dx, dy);
-      const float alpha = fminf(0.99f, gb.y * spec_expf(power));
-      // gb.w: alpha < 1/255 for sure below it
-      const bool skip = power > 0.0f || power < gb.w || alpha < a_min;
-      return skip ? 0.0f : alpha;
-    };
-    // in list order; selects instead of branches (the same arithmetic: a
-    // skipped or saturating pair leaves the state as it was)
-    auto apply = [&](int j, float alpha) {
-      const float test_T = T * (1.0f - alpha);
-      const bool live = alpha != 0.0f && !done;
-      const bool stop = live && test_T < 0.0001f;
-      const bool upd = live && !stop;
-      const float w = alpha * T;
-      const float4 gc = s_c[j];
-      const float dz = s_b[j].z;
-      const float n0 = fmaf(gc.x, w, C0), n1 = fmaf(gc.y, w, C1), n2 = fmaf(gc.z, w, C2), nd = fmaf(dz, w, D);
-      C0 = upd ? n0 : C0;
-      C1 = upd ? n1 : C1;
-      C2 = upd ? n2 : C2;
-      D = upd ? nd : D;
-      T = upd ? test_T : T;
-      last = upd ? first + (uint32_t)j : last;
-      done = done || stop;
-    };
-    // four list entries per step: their alphas do not depend on each other,
-    // so the four exponentials are in flight together (the heaviest tiles run
-    // nearly alone at the end of the launch, where this latency is the time);
-    // they are applied in order.  The indices come in one 4-byte LDS read;
-    // slots past nw hold stale indices of staged splats and are masked.
-    for (int i = 0; !done && i < nw; i += 4) {
-      const uint32_t jj = *reinterpret_cast<const uint32_t*>(&s_list[wv][i]);
-      const int j0 = jj & 0xffu, j1 = (jj >> 8) & 0xffu, j2 = (jj >> 16) & 0xffu, j3 = jj >> 24;
-      const int left = nw - i;
-      const float a0 = alpha_at(j0);
-      const float a1 = left > 1 ? alpha_at(j1) : 0.0f;
-      const float a2 = left > 2 ? alpha_at(j2) : 0.0f;
-      const float a3 = left > 3 ? alpha_at(j3) : 0.0f;
-      apply(j0, a0);
-      apply(j1, a1);
-      apply(j2, a2);
-      apply(j3, a3);
-    }
+    if (lane == 0 && count > 0) atomicAdd(&a.bweight[base + tile + min(w, nwin - 1) / 4], count);
+  }
+  // (the last contributor lies in the lane of its entry)
+  if constexpr (E == 4) {
+    last = max(last, (uint32_t)__shfl_xor((int)last, 1, 64));
+    last = max(last, (uint32_t)__shfl_xor((int)last, 2, 64));
   }
   if (inside) {
     const int pix = py * a.W + px;
     const int HW = a.H * a.W;
-    a.final_T[pix] = T;
-    a.n_contrib[pix] = last;
-    a.out_color[pix] = fmaf(T, a.bg[0], C0);
-    a.out_color[HW + pix] = fmaf(T, a.bg[1], C1);
-    a.out_color[2 * HW + pix] = fmaf(T, a.bg[2], C2);
-    a.out_depth[pix] = D;
-    if (a.out_alpha) a.out_alpha[pix] = 1.0f - T;
-    a.accum[pix] = C0;
-    a.accum[HW + pix] = C1;
-    a.accum[2 * HW + pix] = C2;
-    a.accum[3 * HW + pix] = D;
-    if (last) atomicMax(&s_maxc, last);
-  }
-  __syncthreads();
-  if (threadIdx.x == 0) {
-    a.tile_maxc[tile] = s_maxc;
-    if (batch > 0) a.bweight[a.ckpt_base[tile] + tile + batch - 1] = s_bw;  // the last batch run
-  }
-  __syncthreads();
-  // The backward's work items of this tile: its 256-entry chunks up to the
-  // last contributor, each with a cost class from the longest per-wave list
-  // the blend had in the same batch (class 0 = longest).
-  if (threadIdx.x < 64) {
-    const uint32_t nch = (s_maxc + 255u) / 256u;
-    const uint32_t wbase = a.ckpt_base[tile] + tile;
-    for (uint32_t c = lane; c < nch; c += 64) {
-      const uint32_t w = a.bweight[wbase + c];
-      const uint32_t cls = 63u - min(w >> 2, 63u);
-      const uint32_t slot = atomicAdd(&a.item_log[0], 1u);
-      a.item_log[1 + 2 * slot] = tile;
-      a.item_log[2 + 2 * slot] = (c << 6) | cls;
+#pragma unroll
+    for (int c = 0; c < kCh; ++c) {
+      const int ch = kCh * e + c;
+      a.accum[ch * HW + pix] = C[c];
+      if (ch < 3) a.out_color[ch * HW + pix] = fmaf(T, a.bg[ch], C[c]);
+      else a.out_depth[pix] = C[c];
     }
+    if (e == 0) {
+      a.final_T[pix] = T;
+      a.n_contrib[pix] = last;
+      if (a.out_alpha) a.out_alpha[pix] = 1.0f - T;
+    }
+  }
+  if (n == 0) return;
+  // The last of the tile's waves to get here logs the backward's work items:
+  // the list's 256-entry chunks up to the tile's last contributor, each with a
+  // cost class from the entries the waves kept of it (class 0 = most).  All of
+  // it goes through atomics, which are performed one after another wherever
+  // the waves ran; the waits keep a wave's own in order.
+  const uint32_t wlast = wave_max_u32(last);
+  uint32_t turn = 0;
+  if (lane == 0) {
+    atomicMax(&a.tile_maxc[tile], wlast);
+    asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    turn = atomicAdd(&a.tile_done[tile], 1u);
+  }
+  if (__builtin_amdgcn_readfirstlane((int)turn) != kBlocks - 1) return;
+  const uint32_t maxc = atomicMax(&a.tile_maxc[tile], 0u);
+  for (uint32_t c = lane; c * 256u < maxc; c += 64) {
+    const uint32_t kept = atomicAdd(&a.bweight[base + tile + c], 0u);
+    const uint32_t cls = 63u - min(kept / (4u * kBlocks), 63u);
+    const uint32_t slot = atomicAdd(&a.item_log[0], 1u);
+    a.item_log[1 + 2 * slot] = tile;
+    a.item_log[2 + 2 * slot] = (c << 6) | cls;
   }
 }
 
-__global__ __launch_bounds__(256) void k_blend(BlendArgs a) { blend_tile(a, a.tile_order[blockIdx.x]); }
+// Workgroup b's tile (rank in the blend's order) and block.  The blocks of a
+// tile read the same list and splats: they are 8 apart, so dispatch, which
+// deals workgroups round-robin over the 8 XCDs, puts them on one L2.
+template <int E>
+__device__ __forceinline__ uint32_t blend_rank(uint32_t b, int& part) {
+  part = (int)(b / 8u % (4u * E));
+  return b % 8u + 8u * (b / (32u * E));
+}
+// Launches of at most this many tiles blend on 4 x 4 blocks, larger ones on
+// 8 x 8: up to here four waves a tile leave the SIMDs half empty and the
+// longest wave sets the time, which the smaller block shortens; past it the
+// instructions count, of which the smaller blocks issue more.  8 x 8 / 4 x 4,
+// us: 46 / 26 at 256 tiles, 100 / 50 at 510, 87 / 50 at 858, 87 / 79 and
+// 100 / 77 at 1 170 - 1 450 (training scenes), but 73 / 82 at 920 and 71 / 109
+// at 2 040 for sparse views; 107 / 108 at 2 040, 270 / 564 at 8 160.
+constexpr int kCellTiles = 1024;
+inline unsigned blend_grid(unsigned tiles, int e) { return (tiles + 7u) / 8u * 32u * (unsigned)e; }
+
+template <int E>
+__global__ __launch_bounds__(64) void k_blend(BlendArgs a, uint32_t tiles) {
+  int part;
+  const uint32_t r = blend_rank<E>(blockIdx.x, part);
+  if (r < tiles) blend_block<E>(a, a.tile_order[r], part);
+}
 
 // Frame f of a set whose per-frame block counts have the exclusive prefix
 // `prefix` (n + 1 entries): the last f with prefix[f] <= b.
@@ -753,16 +891,21 @@ __device__ __forceinline__ int frame_of(const uint32_t* prefix, int n, uint32_t 
 
 // Blend of many frames in one launch: one workgroup per tile of every frame
 // (each frame's tiles in its longest-first order).
-__global__ __launch_bounds__(256) void k_blend_multi(const uint32_t* prefix, const BlendArgs* args, int n) {
-  const uint32_t b = blockIdx.x;
-  const int f = frame_of(prefix, n, b);
+template <int E>
+__global__ __launch_bounds__(64) void k_blend_multi(const uint32_t* prefix, const BlendArgs* args, int n) {
+  int part;
+  const uint32_t r = blend_rank<E>(blockIdx.x, part);
+  if (r >= prefix[n]) return;
+  const int f = frame_of(prefix, n, r);
   const BlendArgs a = args[f];
-  blend_tile(a, a.tile_order[b - prefix[f]]);
+  blend_block<E>(a, a.tile_order[r - prefix[f]], part);
 }
 
 // One workgroup: checkpoint base of every tile = exclusive prefix over tiles
 // of (batches in its list - 1); ckpt_base[n_tiles] = total checkpoints.
-// It also clears the blend's work-item log.
+// It also clears what the blend's waves count in: the work-item log, each
+// tile's words (tile_words: last contributors, then waves done) and the kept
+// entries per batch (item_log and bweight are null where no list can exist).
 // Also turns the ranges of empty tiles, left at [UINT_MAX, 0) by the
 // depth-first list sort, into [0, 0), and orders the tiles for the blend,
 // longest list first (a counting sort on the list length in 64-entry steps,
@@ -771,14 +914,15 @@ __global__ __launch_bounds__(256) void k_blend_multi(const uint32_t* prefix, con
 // tiles: the longest lists start first, and consecutive workgroups go to
 // different XCDs, so the long lists of one image region spread over the GPU.
 __device__ __forceinline__ void tile_ckpt_scan_block(uint32_t* ranges, int nt, uint32_t* ckpt_base,
-                                                     uint32_t* item_log, uint32_t* tile_order) {
+                                                     uint32_t* item_log, uint32_t* tile_order,
+                                                     uint32_t* tile_words, uint32_t* bweight) {
   __shared__ uint32_t s[1024];
   __shared__ uint32_t s_carry;
   __shared__ uint32_t s_cls[256];
   const int t = threadIdx.x;
   if (t == 0) {
     s_carry = 0;
-    item_log[0] = 0;
+    if (item_log) item_log[0] = 0;
   }
   __syncthreads();
   for (int b0 = 0; b0 < nt; b0 += 1024) {
@@ -804,6 +948,9 @@ __device__ __forceinline__ void tile_ckpt_scan_block(uint32_t* ranges, int nt, u
     __syncthreads();
   }
   if (t == 0) ckpt_base[nt] = s_carry;
+  for (int k = t; k < 2 * nt; k += 1024) tile_words[k] = 0;
+  if (bweight)
+    for (uint32_t k = t; k < s_carry + (uint32_t)nt; k += 1024) bweight[k] = 0;
   if (t < 256) s_cls[t] = 0;
   __syncthreads();
   auto cls_of = [&](int b) { return min((ranges[2 * b + 1] - ranges[2 * b] + 63u) / 64u, 255u); };
@@ -822,8 +969,9 @@ __device__ __forceinline__ void tile_ckpt_scan_block(uint32_t* ranges, int nt, u
 }
 
 __global__ __launch_bounds__(1024) void k_tile_ckpt_scan(uint32_t* ranges, int nt, uint32_t* ckpt_base,
-                                                         uint32_t* item_log, uint32_t* tile_order) {
-  tile_ckpt_scan_block(ranges, nt, ckpt_base, item_log, tile_order);
+                                                         uint32_t* item_log, uint32_t* tile_order,
+                                                         uint32_t* tile_words, uint32_t* bweight) {
+  tile_ckpt_scan_block(ranges, nt, ckpt_base, item_log, tile_order, tile_words, bweight);
 }
 
 struct CkptScan {
@@ -831,13 +979,15 @@ struct CkptScan {
   uint32_t* ckpt_base;
   uint32_t* item_log;
   uint32_t* tile_order;
+  uint32_t* tile_words;
+  uint32_t* bweight;
   int nt;
 };
 
 // Workgroup f: the checkpoint scan of frame f.
 __global__ __launch_bounds__(1024) void k_tile_ckpt_scan_multi(const CkptScan* cs) {
   const CkptScan c = cs[blockIdx.x];
-  tile_ckpt_scan_block(c.ranges, c.nt, c.ckpt_base, c.item_log, c.tile_order);
+  tile_ckpt_scan_block(c.ranges, c.nt, c.ckpt_base, c.item_log, c.tile_order, c.tile_words, c.bweight);
 }
 
 __global__ __launch_bounds__(256) void k_mark_visible(const float* means, int P, const float* view,
@@ -960,8 +1110,8 @@ extern "C" int gs_image_layout(int width, int height, gs_image_layout_t* out) {
   o = align_up(o + 16 * hw, 256);
   out->ckpt_base = o;
   o = align_up(o + 4 * ((size_t)nt + 1), 256);
-  out->tile_maxc = o;
-  o = align_up(o + 4 * (size_t)nt, 256);
+  out->tile_maxc = o;  // and behind them the count of the tile's waves that are through
+  o = align_up(o + 8 * (size_t)nt, 256);
   out->tile_order = o;
   o = align_up(o + 4 * (size_t)nt, 256);
   out->total = o;
@@ -1186,7 +1336,8 @@ static int render_binning(const gs_frame_t* f, int P, const void* geom, uint32_t
   }
   if (post || (df && do_ckpt))
     hipLaunchKernelGGL(k_tile_ckpt_scan, dim3(1), dim3(1024), 0, s, ranges, nt, (uint32_t*)(ib + LI.ckpt_base),
-                       (uint32_t*)(bb + LB.item_log), (uint32_t*)(ib + LI.tile_order));
+                       bb ? (uint32_t*)(bb + LB.item_log) : nullptr, (uint32_t*)(ib + LI.tile_order),
+                       (uint32_t*)(ib + LI.tile_maxc), bb ? (uint32_t*)(bb + LB.bweight) : nullptr);
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
 }
 
@@ -1222,6 +1373,7 @@ static BlendArgs make_blend_args(const gs_frame_t* f, int P, const void* geom, l
   b.ckpt_base = (const uint32_t*)(ib + LI.ckpt_base);
   b.ckpt = (float*)(bb + LB.ckpt);
   b.tile_maxc = (uint32_t*)(ib + LI.tile_maxc);
+  b.tile_done = b.tile_maxc + grid_tiles(f->width, f->height, gx, gy);
   b.tile_order = (const uint32_t*)(ib + LI.tile_order);
   b.bweight = (uint32_t*)(bb + LB.bweight);
   b.item_log = (uint32_t*)(bb + LB.item_log);
@@ -1247,7 +1399,8 @@ static int render_blend_from(int phase, const gs_frame_t* f, int P, const void* 
   const int nt = grid_tiles(f->width, f->height, gx, gy);
   {
     timing::Scope ts(timing::kBlend, s);
-    hipLaunchKernelGGL(k_blend, dim3(nt), dim3(256), 0, s, b);
+    if (nt <= kCellTiles) hipLaunchKernelGGL(k_blend<4>, dim3(blend_grid(nt, 4)), dim3(64), 0, s, b, (uint32_t)nt);
+    else hipLaunchKernelGGL(k_blend<1>, dim3(blend_grid(nt, 1)), dim3(64), 0, s, b, (uint32_t)nt);
   }
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
 }
@@ -1453,6 +1606,8 @@ extern "C" int gs_multi_binning_steps_build(int n, const gs_frame_t* frames, con
     ck[i].ranges = (uint32_t*)(ib + LI.ranges);
     ck[i].ckpt_base = (uint32_t*)(ib + LI.ckpt_base);
     ck[i].item_log = (uint32_t*)(bb + LB.item_log);
+    ck[i].tile_words = (uint32_t*)(ib + LI.tile_maxc);
+    ck[i].bweight = (uint32_t*)(bb + LB.bweight);
     ck[i].tile_order = (uint32_t*)(ib + LI.tile_order);
     ck[i].nt = nt;
   }
@@ -1642,7 +1797,10 @@ extern "C" int gs_multi_blend(int n, const void* dev_set, unsigned total_tiles, 
   const BlendArgs* args = (const BlendArgs*)((const char*)dev_set + multi_blend_args_offset(n));
   {
     timing::Scope ts(timing::kBlend, s);
-    hipLaunchKernelGGL(k_blend_multi, dim3(total_tiles), dim3(256), 0, s, prefix, args, n);
+    if (total_tiles <= (unsigned)kCellTiles)
+      hipLaunchKernelGGL(k_blend_multi<4>, dim3(blend_grid(total_tiles, 4)), dim3(64), 0, s, prefix, args, n);
+    else
+      hipLaunchKernelGGL(k_blend_multi<1>, dim3(blend_grid(total_tiles, 1)), dim3(64), 0, s, prefix, args, n);
   }
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
 }

@@ -132,8 +132,9 @@ typedef struct gs_binning_layout {
   size_t dscan, dblocks;       /* uint32[P] tiles prefix in depth order, per-256 block sums */
   size_t drect;                /* uint32[2P] tile rect per Gaussian: x0 | y0 << 16, x1 | y1 << 16 (DEPTH_FIRST) */
   size_t ckpt;                 /* float[capacity/256 + 1][5][256] blend state at list batch boundaries */
-  size_t bweight;              /* uint32[capacity/256 + 2 n_tiles + 2] per (tile, list batch): the blend's
-                                  longest per-wave list, the backward's estimate of that chunk's cost */
+  size_t bweight;              /* uint32[capacity/256 + 2 n_tiles + 2] per (tile, list batch): the entries
+                                  the blend's waves kept of the batch, the backward's estimate of
+                                  that chunk's cost */
   size_t items;                /* uint32[4 (1 + capacity/256 + n_tiles + 1)] backward work items: count,
                                   then from word 4 (tile, chunk, list start, last contributor),
                                   longest estimated first */
@@ -149,7 +150,8 @@ typedef struct gs_image_layout {
   size_t n_contrib; /* uint32[H*W] index (1-based) of the last contributor */
   size_t accum;     /* float[4][H*W] colour sums before the background term, depth */
   size_t ckpt_base; /* uint32[n_tiles+1] first checkpoint of each tile */
-  size_t tile_maxc; /* uint32[n_tiles] largest contributor index in the tile */
+  size_t tile_maxc; /* uint32[2 n_tiles] largest contributor index in the tile, then the blend's waves
+                       that are through with the tile */
   size_t tile_order; /* uint32[n_tiles] the blend's tile order, longest list first */
   size_t total;
 } gs_image_layout_t;

@@ -41,3 +41,27 @@ def test_list_lengths(n, small):
         np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
     _check(sc, 1, seed=n)
     _check(sc, 1, seed=n, deterministic=True)
+
+
+@pytest.mark.parametrize("tall", [False, True], ids=["4x4", "8x8"])
+@pytest.mark.parametrize("n", [1, 3, 4, 5, 64, 65, 127, 300])
+def test_blend_blocks(n, tall):
+    """Both of the blend's blocks (2 x 2 tiles, or 2 x 513 with the splats
+    spread over the first of them) where lists end inside a group, pixels
+    saturate and one colour is infinite: the pixels it misses stay finite."""
+    print("blend blocks", n, "tall" if tall else "small", flush=True)
+    sc = _stack(n, True)
+    if tall:
+        tall_sc = scenes.plain_scene(seed=50 + n, P=n, W=21, H=16 * 512 + 3)
+        for k in ("means", "scales", "bg"):
+            tall_sc[k] = sc[k]
+        sc = tall_sc
+    sc["opacities"] = torch.linspace(0.004, 1.0, n).reshape(n, 1)[torch.randperm(n, generator=torch.Generator().manual_seed(n))]
+    sc["shs"][n // 2, 0, 1] = float("inf")
+    g = run_gpu(sc, 1)
+    _, _, o = run_oracle(sc, 1)
+    np.testing.assert_array_equal(np_(g["views"]["n_contrib"]), o["n_contrib"])
+    np.testing.assert_array_equal(np_(g["views"]["final_T"]), o["final_T"])
+    for k in ("color", "depth", "alpha"):
+        np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
+    assert np.isfinite(o["color"][[0, 2]]).all()
