@@ -21,7 +21,7 @@ inline int bits_for(uint32_t n) {  // number of bits needed to hold values < n
   return b;
 }
 // LSD passes over bits [0, end_bit), kRadixBits at a time.
-inline int sort_passes(int end_bit) { return (end_bit + kRadixBits - 1) / kRadixBits; }
+constexpr int sort_passes(int end_bit) { return (end_bit + kRadixBits - 1) / kRadixBits; }
 
 namespace timing {
 enum Stage { kPreprocess = 0, kScan, kDuplicate, kSort, kRanges, kBlend, kRenderBwd, kPreprocessBwd, kKnn, kZero };
@@ -42,7 +42,18 @@ class Scope {
 bool enabled();
 }  // namespace timing
 
-size_t sort_tmp_bytes(long long capacity);
+// Keys per workgroup: short sorts use 1024 (4 per thread) so that they still
+// fill the 256 CUs (at 500k keys, 2048 per workgroup sorts slower); long
+// ones 2048 (8 per thread).  Measured at 5.7M keys, 8 per thread sorts faster
+// than 16 or 12: the scans are cheap enough that more, smaller workgroups pay.
+constexpr int sort_tile(long long capacity) { return capacity <= (1LL << 21) ? kSortThreads * 4 : kSortThreads * 8; }
+
+constexpr size_t sort_tmp_bytes(long long capacity) {
+  const long long tile = sort_tile(capacity);
+  const long long nb = (capacity + tile - 1) / tile;
+  return align_up((size_t)kRadix * 4 * (size_t)(nb > 0 ? nb : 1), 256) + kRadix * 4;
+}
+
 // Returns hipSuccess or the launch error.  *result_in_b tells where the
 // sorted data ends up.
 hipError_t sort_pairs_u64(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b,

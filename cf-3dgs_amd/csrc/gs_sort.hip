@@ -328,18 +328,6 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const K* __restri
                                 ranges, tshift, blockIdx.x);
 }
 
-// Keys per workgroup: short sorts use 1024 (4 per thread) so that they still
-// fill the 256 CUs (at 500k keys, 2048 per workgroup sorts slower); long
-// ones 2048 (8 per thread).  Measured at 5.7M keys, 8 per thread sorts faster
-// than 16 or 12: the scans are cheap enough that more, smaller workgroups pay.
-int sort_tile(long long capacity) { return capacity <= (1LL << 21) ? kSortThreads * 4 : kSortThreads * 8; }
-
-size_t sort_tmp_bytes(long long capacity) {
-  const long long tile = sort_tile(capacity);
-  const long long nb = (capacity + tile - 1) / tile;
-  return align_up((size_t)kRadix * 4 * (size_t)(nb > 0 ? nb : 1), 256) + kRadix * 4;
-}
-
 template <typename K, int ITEMS, int R>
 void sort_pass(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout, const uint32_t* n_dev, long long capacity,
                int shift, int bits, uint32_t* hist, uint32_t* totals, int nb_max, int tile, hipStream_t s,
