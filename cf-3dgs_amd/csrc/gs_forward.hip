@@ -245,40 +245,67 @@ __global__ __launch_bounds__(256) void k_preprocess_multi(const uint32_t* prefix
   preprocess_block(a, (int)(b - prefix[f]), (int)(prefix[f + 1] - prefix[f]), s_sh);
 }
 
+// In-place exclusive prefix of n values by one workgroup of NT threads; returns
+// their sum in every thread, `biggest` the largest of the thread's own values.
+// Eight values a thread and round, loaded together (data is 16-byte aligned).
+// One frame takes 1024 threads, a round for 2 million Gaussians; many frames
+// take 256 each: 1024 had to wait for a compute unit with 16 free wave slots
+// while another stream's blend ran (49 us a launch of 16 pose frames, now 6).
+template <int NT>
+__device__ __forceinline__ uint32_t scan_in_place(uint32_t* data, int n, uint32_t& biggest) {
+  constexpr int kRun = 8;
+  __shared__ uint32_t s_w[2][NT / 64];
+  const int t = threadIdx.x;
+  uint32_t carry = 0;
+  biggest = 0;
+  for (int b0 = 0, r = 0; b0 < n; b0 += NT * kRun, r ^= 1) {
+    const int first = b0 + t * kRun;
+    uint32_t v[kRun], sum = 0;
+    if (first + kRun <= n) {
+      const uint4 a = *reinterpret_cast<const uint4*>(data + first), b = *reinterpret_cast<const uint4*>(data + first + 4);
+      v[0] = a.x, v[1] = a.y, v[2] = a.z, v[3] = a.w;
+      v[4] = b.x, v[5] = b.y, v[6] = b.z, v[7] = b.w;
+    } else {
+#pragma unroll
+      for (int j = 0; j < kRun; ++j) v[j] = first + j < n ? data[first + j] : 0u;
+    }
+#pragma unroll
+    for (int j = 0; j < kRun; ++j) {
+      sum += v[j];
+      biggest = max(biggest, v[j]);
+    }
+    uint32_t tot;
+    uint32_t run = carry + block_scan_incl<NT>(sum, s_w[r], tot) - sum;
+#pragma unroll
+    for (int j = 0; j < kRun; ++j) {
+      if (first + j < n) data[first + j] = run;
+      run += v[j];
+    }
+    carry += tot;
+  }
+  return carry;
+}
+
 // Single workgroup: exclusive prefix of the per-workgroup tile sums (in place),
 // num_rendered and the OR of the status flags.
+template <int NT>
 __device__ __forceinline__ void scan_top_block(uint32_t* block_sum, int nblocks, uint32_t* counters) {
-  __shared__ uint32_t s[1024];
-  __shared__ uint32_t s_carry, s_flags;
-  const int t = threadIdx.x;
-  if (t == 0) {
-    s_carry = 0;
-    s_flags = 0;
-  }
+  __shared__ uint32_t s_flags;
+  if (threadIdx.x == 0) s_flags = 0;
+  uint32_t myflags = 0, biggest;
+  for (int b = threadIdx.x; b < nblocks; b += NT) myflags |= block_sum[nblocks + b];
   __syncthreads();
-  uint32_t myflags = 0;
-  for (int b0 = 0; b0 < nblocks; b0 += 1024) {
-    const int b = b0 + t;
-    const uint32_t v = b < nblocks ? block_sum[b] : 0u;
-    if (b < nblocks) myflags |= block_sum[nblocks + b];
-    uint32_t tot;
-    const uint32_t incl = block_scan_incl<1024>(v, s, tot);
-    const uint32_t carry = s_carry;
-    if (b < nblocks) block_sum[b] = carry + incl - v;
-    __syncthreads();
-    if (t == 0) s_carry = carry + tot;
-    __syncthreads();
-  }
   if (myflags) atomicOr(&s_flags, myflags);
+  const uint32_t total = scan_in_place<NT>(block_sum, nblocks, biggest);
   __syncthreads();
-  if (t == 0) {
-    counters[0] = s_carry;
+  if (threadIdx.x == 0) {
+    counters[0] = total;
     counters[1] = s_flags;
   }
 }
 
 __global__ __launch_bounds__(1024) void k_scan_top(uint32_t* block_sum, int nblocks, uint32_t* counters) {
-  scan_top_block(block_sum, nblocks, counters);
+  scan_top_block<1024>(block_sum, nblocks, counters);
 }
 
 struct ScanTop {
@@ -288,9 +315,9 @@ struct ScanTop {
 };
 
 // Workgroup f: the scan of frame f.
-__global__ __launch_bounds__(1024) void k_scan_top_multi(const ScanTop* st) {
+__global__ __launch_bounds__(256) void k_scan_top_multi(const ScanTop* st) {
   const ScanTop t = st[blockIdx.x];
-  scan_top_block(t.block_sum, t.nblocks, t.counters);
+  scan_top_block<256>(t.block_sum, t.nblocks, t.counters);
 }
 
 struct DupArgs {
@@ -430,27 +457,21 @@ __global__ __launch_bounds__(256) void k_df_scan(int P, const uint32_t* dvals, c
   df_scan_block(P, dvals, tiles, dscan, dblocks, blockIdx.x);
 }
 
-// One workgroup: in-place exclusive prefix of n values.
+// One workgroup: in-place exclusive prefix of the n block totals, and the
+// largest of them in data[n].
+template <int NT>
 __device__ __forceinline__ void excl_scan_block(uint32_t* data, int n) {
-  __shared__ uint32_t s[1024];
-  __shared__ uint32_t s_carry;
-  const int t = threadIdx.x;
-  if (t == 0) s_carry = 0;
+  __shared__ uint32_t s_max;
+  if (threadIdx.x == 0) s_max = 0;
+  uint32_t biggest;
+  scan_in_place<NT>(data, n, biggest);
   __syncthreads();
-  for (int b0 = 0; b0 < n; b0 += 1024) {
-    const int b = b0 + t;
-    const uint32_t v = b < n ? data[b] : 0u;
-    uint32_t tot;
-    const uint32_t incl = block_scan_incl<1024>(v, s, tot);
-    const uint32_t carry = s_carry;
-    if (b < n) data[b] = carry + incl - v;
-    __syncthreads();
-    if (t == 0) s_carry = carry + tot;
-    __syncthreads();
-  }
+  if (biggest) atomicMax(&s_max, biggest);
+  __syncthreads();
+  if (threadIdx.x == 0) data[n] = s_max;
 }
 
-__global__ __launch_bounds__(1024) void k_excl_scan_1wg(uint32_t* data, int n) { excl_scan_block(data, n); }
+__global__ __launch_bounds__(1024) void k_excl_scan_1wg(uint32_t* data, int n) { excl_scan_block<1024>(data, n); }
 
 struct DfDupArgs {
   int P, gx, gy;
@@ -466,74 +487,135 @@ struct DfDupArgs {
   int id_bits;
 };
 
-// Duplicate tile ids in depth order (sorted position k -> Gaussian dvals[k]).
-// Each Gaussian's entries form one run at its prefix offset.  The wave
-// expands its 64 runs cooperatively: output j of the wave's concatenated runs
-// goes to lane j mod 64, which finds its run by binary search over the
-// wave's exclusive prefix, so consecutive lanes write consecutive entries of
-// a run (a run leaves as one contiguous segment, not as one word from each of
-// 64 places per store).  Entry order and values are those of a per-Gaussian
-// loop over the rect, row by row.
-__device__ __forceinline__ void df_duplicate_block(const DfDupArgs& a, int bid) {
-  __shared__ uint32_t s_excl[4][64], s_off[4][64], s_g[4][64], s_xy[4][64], s_w[4][64];
-  const int k = bid * 256 + threadIdx.x;
-  const int w = threadIdx.x >> 6, lane = threadIdx.x & 63;
+// Tile ids in depth order (sorted position k -> Gaussian dvals[k]).  Each
+// Gaussian's entries form one run at its prefix offset, its rect row by row.
+//
+// Where no block of 256 Gaussians has more than 4096 entries, workgroup b
+// expands block b.  Else the work is split by output: a workgroup takes the same
+// number of consecutive entries as every other (at least 1024, and no more
+// workgroups than the GPU holds at once) and finds the run its first entry lies
+// in by a 64-wide search of the prefix.  Either way the runs are expanded 256 at a time,
+// four entries a thread and one 16-byte store.  With the split by Gaussian
+// alone the few splats that cover a whole image set the launch's length (1284
+// us for 71M entries of 1 200 000 Gaussians at 1920 x 1080, now 125; 49 and 7
+// for 100 000 at 480 x 270); where the blocks are even the search alone costs
+// (31 us with it for 16 pose frames, 22 without).
+__device__ __forceinline__ void df_duplicate_block(const DfDupArgs& a, uint32_t bid, uint32_t nblocks) {
+  __shared__ uint32_t s_start[256], s_g[256], s_xy[256], s_w[256], s_k0, s_end;
+  const uint32_t t = threadIdx.x;
   const uint32_t n = a.counters[0];
   if ((long long)n > a.capacity) {
-    if (k == 0) {
+    if (bid == 0 && t == 0) {
       atomicOr(&a.counters[1], GS_STATUS_CAPACITY);
       atomicOr(&a.counters[3], GS_STATUS_CAPACITY);  // sticky copy
     }
     return;
   }
-  uint32_t nt = 0, off = 0, g = 0, x0 = 0, y0 = 0, rw = 1;
-  if (k < a.P) {
-    g = a.dvals[k];
-    nt = a.tiles[g];
-    if (nt) {
-      off = a.dblocks[k >> 8] + a.dscan[k] - nt;
-      const uint2 r = a.rect[g];
-      x0 = r.x & 0xffffu;
-      y0 = r.x >> 16;
-      rw = (r.y & 0xffffu) - x0;
+  const uint32_t P = (uint32_t)a.P, chunk = (n / min(nblocks, 2048u) / 1024u + 1u) * 1024u;
+  const uint32_t nruns = (P + 255u) / 256u;
+  const bool even = a.dblocks[nruns] <= 4096u;
+  const uint32_t nchunks = even ? nruns : n / chunk + (n % chunk != 0 ? 1u : 0u);
+  for (uint32_t c = bid; c < nchunks; c += nblocks) {
+    uint32_t o0 = c * chunk, o1 = o0 + min(chunk, n - o0);
+    if (even) {
+      o0 = a.dblocks[c];
+      o1 = c + 1u < nruns ? a.dblocks[c + 1u] : n;
+      if (t == 0) s_k0 = 256u * c;
+    } else if (t < 64) {
+      // the last 256-run block that starts at or before o0, then its runs that
+      // end there
+      uint32_t lo = 0, len = nruns;
+      while (len > 1) {
+        const uint32_t step = (len + 63u) / 64u, k = t * step;
+        const uint32_t m = (uint32_t)__popcll(__ballot(k < len && a.dblocks[lo + min(k, len - 1u)] <= o0)) - 1u;
+        lo += m * step;
+        len = min(step, len - m * step);
+      }
+      const uint32_t b0 = a.dblocks[lo];
+      uint32_t k0 = lo * 256u;
+#pragma unroll
+      for (uint32_t q = 0; q < 4; ++q) {
+        const uint32_t k = lo * 256u + q * 64u + t;
+        k0 += (uint32_t)__popcll(__ballot(k < P && b0 + a.dscan[min(k, P - 1u)] <= o0));
+      }
+      if (t == 0) s_k0 = k0;
     }
-  }
-  // wave exclusive prefix of the run lengths
-  uint32_t incl = nt;
+    __syncthreads();
+    uint32_t pos = o0;
+    for (uint32_t k0 = s_k0; pos < o1; k0 += 256) {
+      const uint32_t k = k0 + t;
+      uint32_t start = n, end = n, g = 0, xy = 0, w = 1;
+      if (k < P) {
+        g = a.dvals[k];
+        end = a.dblocks[k >> 8] + a.dscan[k];
+        start = end - a.tiles[g];
+        if (start < end) {
+          const uint2 r = a.rect[g];
+          xy = r.x;
+          w = (r.y & 0xffffu) - (r.x & 0xffffu);
+        }
+      }
+      s_start[t] = start;
+      s_g[t] = g;
+      s_xy[t] = xy;
+      s_w[t] = w;
+      if (t == 255) s_end = end;
+      __syncthreads();
+      const uint32_t lim = min(o1, s_end);
+      for (uint32_t q = (pos >> 2) + t; 4u * q < lim; q += 256) {
+        const uint32_t first = max(4u * q, pos), stop = min(4u * q + 4u, lim);
+        // run j = last with start <= first
+        uint32_t j = 0;
 #pragma unroll
-  for (int d = 1; d < 64; d <<= 1) {
-    const uint32_t y = __shfl_up(incl, d, 64);
-    if (lane >= d) incl += y;
-  }
-  const uint32_t total = __shfl(incl, 63, 64);
-  s_excl[w][lane] = incl - nt;
-  s_off[w][lane] = off;
-  s_g[w][lane] = g;
-  s_xy[w][lane] = x0 | (y0 << 16);
-  s_w[w][lane] = rw;
-  __builtin_amdgcn_wave_barrier();
-  for (uint32_t o = (uint32_t)lane; o < total; o += 64) {
-    // run j = last lane with excl <= o (empty runs share their successor's
-    // excl and lose to it)
-    int j = 0;
+        for (uint32_t step = 128; step > 0; step >>= 1)
+          if (s_start[j + step] <= first) j += step;
+        uint32_t rw = s_w[j], id = s_g[j], p = s_xy[j];
+        const uint32_t r = first - s_start[j], ry = r / rw;
+        uint32_t rx = r - ry * rw, tile = ((p >> 16) + ry) * (uint32_t)a.gx + (p & 0xffffu) + rx;
+        uint32_t next = j < 255u ? s_start[j + 1] : lim;
+        uint32_t key[4], val[4];
 #pragma unroll
-    for (int step = 32; step > 0; step >>= 1)
-      if (s_excl[w][j + step] <= o) j += step;
-    const uint32_t r = o - s_excl[w][j];
-    const uint32_t wj = s_w[w][j], xy = s_xy[w][j];
-    const uint32_t ry = r / wj, rx = r - ry * wj;
-    const uint32_t dst = s_off[w][j] + r;
-    const uint32_t tile = ((xy >> 16) + ry) * (uint32_t)a.gx + (xy & 0xffffu) + rx;
-    if (a.id_bits) {
-      a.keys[dst] = (tile << a.id_bits) | s_g[w][j];
-    } else {
-      a.keys[dst] = tile;
-      a.vals[dst] = s_g[w][j];
+        for (uint32_t e = 0; e < 4; ++e) {
+          const uint32_t o = 4u * q + e;
+          key[e] = a.id_bits ? (tile << a.id_bits) | id : tile;
+          val[e] = id;
+          if (o < first) continue;
+          ++rx;
+          ++tile;
+          if (rx == rw) {
+            rx = 0;
+            tile += (uint32_t)a.gx - rw;
+          }
+          if (o + 1u == next && o + 1u < stop) {
+            ++j;
+            rw = s_w[j];
+            id = s_g[j];
+            p = s_xy[j];
+            rx = 0;
+            tile = (p >> 16) * (uint32_t)a.gx + (p & 0xffffu);
+            next = j < 255u ? s_start[j + 1] : lim;
+          }
+        }
+        if (stop - first == 4u) {
+          *reinterpret_cast<uint4*>(a.keys + 4u * q) = make_uint4(key[0], key[1], key[2], key[3]);
+          if (!a.id_bits) *reinterpret_cast<uint4*>(a.vals + 4u * q) = make_uint4(val[0], val[1], val[2], val[3]);
+        } else {
+#pragma unroll
+          for (uint32_t e = 0; e < 4; ++e) {
+            const uint32_t o = 4u * q + e;
+            if (o < first || o >= stop) continue;
+            a.keys[o] = key[e];
+            if (!a.id_bits) a.vals[o] = val[e];
+          }
+        }
+      }
+      pos = lim;
+      __syncthreads();
     }
   }
 }
 
-__global__ __launch_bounds__(256) void k_df_duplicate(DfDupArgs a) { df_duplicate_block(a, blockIdx.x); }
+__global__ __launch_bounds__(256) void k_df_duplicate(DfDupArgs a) { df_duplicate_block(a, blockIdx.x, gridDim.x); }
 
 // The depth-first binning's steps between its two sorts for one frame of a
 // multi-frame launch.
@@ -554,17 +636,18 @@ __global__ __launch_bounds__(256) void k_df_scan_multi(const uint32_t* prefix, c
 }
 
 // Workgroup f: the exclusive prefix of frame f's block totals.
-__global__ __launch_bounds__(1024) void k_excl_scan_multi(const DfMid* mid) {
+__global__ __launch_bounds__(256) void k_excl_scan_multi(const DfMid* mid) {
   const DfMid m = mid[blockIdx.x];
-  excl_scan_block(m.dblocks, m.nblocks);
+  excl_scan_block<256>(m.dblocks, m.nblocks);
 }
 
-// Many frames' duplicates, on the same workgroup ranges as k_df_scan_multi.
+// Many frames' duplicates, on the same workgroup ranges as k_df_scan_multi (a
+// frame's workgroups share its chunks out among them).
 __global__ __launch_bounds__(256) void k_df_duplicate_multi(const uint32_t* prefix, const DfMid* mid, int n) {
   const uint32_t b = blockIdx.x;
   const int f = frame_of_block(prefix, n, b);
   const DfDupArgs a = mid[f].dup;
-  df_duplicate_block(a, (int)(b - prefix[f]));
+  df_duplicate_block(a, b - prefix[f], prefix[f + 1] - prefix[f]);
 }
 
 struct BlendArgs {
@@ -1288,7 +1371,10 @@ static int render_binning(const gs_frame_t* f, int P, const void* geom, uint32_t
       d.keys = (uint32_t*)(bb + LB.keys_dup);
       d.vals = (uint32_t*)(bb + LB.vals_dup);
       d.id_bits = LB.id_bits;
-      hipLaunchKernelGGL(k_df_duplicate, dim3(nbp), dim3(256), 0, s, d);
+      // a workgroup per 1024 entries where there is room for as many, up to what
+      // the GPU holds at once
+      const long long nchunk = (capacity + 1023) / 1024;
+      hipLaunchKernelGGL(k_df_duplicate, dim3((unsigned)std::max<long long>(nbp, std::min(nchunk, 2048LL))), dim3(256), 0, s, d);
     }
     if (do_lsort) {
       timing::Scope ts(timing::kSort, s);
@@ -1527,7 +1613,7 @@ extern "C" int gs_multi_preprocess_keys(int n, const void* dev_set, const unsign
   }
   {
     timing::Scope ts(timing::kScan, s);
-    hipLaunchKernelGGL(k_scan_top_multi, dim3(n), dim3(1024), 0, s, (const ScanTop*)(d + mpk_top_offset(n)));
+    hipLaunchKernelGGL(k_scan_top_multi, dim3(n), dim3(256), 0, s, (const ScanTop*)(d + mpk_top_offset(n)));
   }
   if (launch[1] > 0) {
     timing::Scope ts(timing::kSort, s);
@@ -1623,7 +1709,7 @@ extern "C" int gs_multi_binning_duplicate(int n, const void* dev_set, unsigned t
   const DfMid* mid = (const DfMid*)((const char*)dev_set + mbm_mid_offset(n));
   timing::Scope ts(timing::kDuplicate, s);
   if (total_blocks > 0) hipLaunchKernelGGL(k_df_scan_multi, dim3(total_blocks), dim3(256), 0, s, prefix, mid, n);
-  hipLaunchKernelGGL(k_excl_scan_multi, dim3(n), dim3(1024), 0, s, mid);
+  hipLaunchKernelGGL(k_excl_scan_multi, dim3(n), dim3(256), 0, s, mid);
   if (total_blocks > 0)
     hipLaunchKernelGGL(k_df_duplicate_multi, dim3(total_blocks), dim3(256), 0, s, prefix, mid, n);
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;

@@ -65,3 +65,22 @@ def test_blend_blocks(n, tall):
     for k in ("color", "depth", "alpha"):
         np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
     assert np.isfinite(o["color"][[0, 2]]).all()
+
+
+@pytest.mark.parametrize("n", [8, 9, 255, 256, 257, 700])
+def test_runs_split_by_entry(n):
+    """Gaussians that cover all 510 tiles among ones that cover few: up to 4096
+    entries per 256 Gaussians the lists are expanded by Gaussian, past that by
+    entry.  The lists against the oracle's."""
+    print("runs", n, flush=True)
+    sc = scenes.plain_scene(seed=70 + n, P=n, W=479, H=270)
+    m = max(n // 3, min(n, 9))  # 9 x 510 entries are past 4096
+    sc["scales"][:m] = 3.0
+    sc["means"][:m] = torch.tensor([0.0, 0.0, 3.0])
+    sc["opacities"] = torch.full((n, 1), 0.02)
+    g = run_gpu(sc, 1)
+    _, _, o = run_oracle(sc, 1)
+    assert g["st"].num_rendered == o["num_rendered"]
+    for k in ("color", "depth", "alpha"):
+        np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
+    np.testing.assert_array_equal(np_(g["views"]["n_contrib"]), o["n_contrib"])
