@@ -1164,15 +1164,15 @@ extern "C" int gs_binning_layout(long long capacity, int P, int width, int heigh
   out->item_log = o;
   o = align_up(o + 4 * (1 + 2 * (c / 256 + (size_t)nt + 1)), 256);
   out->total = o;
-  const int end_bit = (df ? 0 : 32) + bits_for((uint32_t)nt);
-  out->sort_passes = sort_passes(end_bit > 0 ? end_bit : 1);
+  // one word per list entry when the Gaussian id and the tile id fit together
+  const int tb = bits_for((uint32_t)nt), idb = bits_for((uint32_t)(P > 1 ? P : 2));
+  out->id_bits = (df && idb + tb <= 32) ? idb : 0;
+  const int end_bit = (df ? 0 : 32) + tb;
+  out->sort_passes = out->id_bits && wide_digit(tb, capacity) ? 1 : sort_passes(end_bit > 0 ? end_bit : 1);
   out->key_bytes = (int)kb;
   const bool in_b = (out->sort_passes & 1) != 0;
   out->keys_sorted = in_b ? out->keys_alt : out->keys_dup;
   out->vals_sorted = in_b ? out->vals_alt : out->vals_dup;
-  // one word per list entry when the Gaussian id and the tile id fit together
-  const int idb = bits_for((uint32_t)(P > 1 ? P : 2));
-  out->id_bits = (df && idb + bits_for((uint32_t)nt) <= 32) ? idb : 0;
   if (out->id_bits) out->vals_sorted = out->keys_sorted;
   return GS_OK;
 }
@@ -1343,7 +1343,7 @@ static int render_binning(const gs_frame_t* f, int P, const void* geom, uint32_t
           hipLaunchKernelGGL(k_df_keys, dim3(std::max(nbp, nblocks256(2LL * nt))), dim3(256), 0, s, P, tiles,
                              splat, gx, gy, dka, dva, (uint2*)(bb + LB.drect), counters, ranges, 2 * nt);
         if (do_dsort)
-          e = sort_pairs_u32(dka, dva, (uint32_t*)(bb + LB.dkeys_b), (uint32_t*)(bb + LB.dvals_b), counters + 2, P,
+          e = sort_pairs_u32(dka, dva, (uint32_t*)(bb + LB.dkeys_b), (uint32_t*)(bb + LB.dvals_b), nullptr, P,
                              32, bb + LB.hist, s, &in_b);
       }
       if (e != hipSuccess) return GS_E_LAUNCH;
@@ -1757,7 +1757,7 @@ extern "C" int gs_multi_depth_sort_build(int n, const gs_frame_t* frames, const 
     if (binning_bytes[i] < LB.total) return GS_E_WORKSPACE;
     char* bb = (char*)binning[i];
     segs[i] = SortSeg{(uint32_t*)(bb + LB.dkeys_a), (uint32_t*)(bb + LB.dvals_a), (uint32_t*)(bb + LB.dkeys_b),
-                      (uint32_t*)(bb + LB.dvals_b), counters[i] + 2, (long long)P[i], bb + LB.hist, 0, 32,
+                      (uint32_t*)(bb + LB.dvals_b), nullptr, (long long)P[i], bb + LB.hist, 0, 32,
                       nullptr};
   }
   unsigned per[kSegMaxPasses];

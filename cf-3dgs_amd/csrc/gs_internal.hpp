@@ -9,8 +9,6 @@
 namespace gs {
 
 constexpr int kSortThreads = 256;
-constexpr int kSortItems = 16;
-constexpr int kSortTile = kSortThreads * kSortItems;  // keys per sort workgroup
 constexpr int kRadixBits = 8;  // digit width of the LSD passes: 256 buckets
 constexpr int kRadix = 1 << kRadixBits;
 
@@ -20,8 +18,17 @@ inline int bits_for(uint32_t n) {  // number of bits needed to hold values < n
   while (b < 32 && (1ull << b) < (uint64_t)n) ++b;
   return b;
 }
-// LSD passes over bits [0, end_bit), kRadixBits at a time.
+// LSD passes over end_bit bits, at most kRadixBits at a time.
 constexpr int sort_passes(int end_bit) { return (end_bit + kRadixBits - 1) / kRadixBits; }
+
+// Whether a keys-only sort of `bits` bits takes them as one digit of up to
+// kWideBits: the counters then fit LDS, and it saves the launches of a pass.
+// Past 2^21 keys two passes of narrow digits are as fast, and their workgroups'
+// counts take half the memory.
+constexpr int kWideBits = 10, kWideRadix = 1 << kWideBits, kWideItems = 16;
+constexpr bool wide_digit(int bits, long long capacity) {
+  return bits > kRadixBits && bits <= kWideBits && capacity <= (1LL << 21);
+}
 
 namespace timing {
 enum Stage { kPreprocess = 0, kScan, kDuplicate, kSort, kRanges, kBlend, kRenderBwd, kPreprocessBwd, kKnn, kZero };
@@ -43,19 +50,25 @@ bool enabled();
 }  // namespace timing
 
 // Keys per workgroup: short sorts use 1024 (4 per thread) so that they still
-// fill the 256 CUs (at 500k keys, 2048 per workgroup sorts slower); long
-// ones 2048 (8 per thread).  Measured at 5.7M keys, 8 per thread sorts faster
-// than 16 or 12: the scans are cheap enough that more, smaller workgroups pay.
-constexpr int sort_tile(long long capacity) { return capacity <= (1LL << 21) ? kSortThreads * 4 : kSortThreads * 8; }
+// fill the 256 CUs (at 500k keys, 2048 per workgroup sorts slower); longer
+// ones 2048.  Measured at 5.7M keys, 8 per thread sorts faster than 16 or 12:
+// the scans are cheap enough that more, smaller workgroups pay.  Past 2^24 the
+// traffic counts, and 4096 keys make longer runs: 339 us a scatter of 71M
+// pairs with 2048, 275 with 4096.
+constexpr int sort_tile(long long capacity) {
+  return kSortThreads * (capacity <= (1LL << 21) ? 4 : (capacity <= (1LL << 24) ? 8 : 16));
+}
 
+// (10-bit digits over 4096 keys need no more than 8-bit ones over 1024, but for
+// the last workgroup and the totals)
 constexpr size_t sort_tmp_bytes(long long capacity) {
   const long long tile = sort_tile(capacity);
   const long long nb = (capacity + tile - 1) / tile;
-  return align_up((size_t)kRadix * 4 * (size_t)(nb > 0 ? nb : 1), 256) + kRadix * 4;
+  return align_up((size_t)kRadix * 4 * (size_t)(nb > 0 ? nb : 1), 256) + 2 * kWideRadix * 4;
 }
 
 // Returns hipSuccess or the launch error.  *result_in_b tells where the
-// sorted data ends up.
+// sorted data ends up.  Without n_dev the count is the capacity.
 hipError_t sort_pairs_u64(uint64_t* keys_a, uint32_t* vals_a, uint64_t* keys_b, uint32_t* vals_b,
                           const uint32_t* n_dev, long long capacity, int end_bit, void* tmp, hipStream_t s,
                           int* result_in_b);
@@ -91,7 +104,8 @@ size_t seg_sort_desc_bytes(int n, int passes);
 // Host-side descriptor of the segments' passes (its pointers are the
 // segments' device buffers); the caller copies it to the device.  Returns
 // false on a segment it cannot take.  blocks[p] is pass p's upsweep /
-// scatter grid (0 past the longest segment's passes); *passes the pass count.
+// scatter grid and which kernels run it (0 past the longest segment's passes);
+// *passes the pass count.
 bool seg_sort_build(int n, const SortSeg* segs, void* host, size_t bytes, unsigned* blocks, int* passes);
 hipError_t seg_sort_launch(int n, const void* dev_desc, const unsigned* blocks, bool values, hipStream_t s);
 

@@ -35,7 +35,7 @@ constexpr int kKnnLeaf = 16, kKnnFan = 64;  // points of a leaf, children of a n
 constexpr int kKnnParts = 256;  // workgroups of the bounding box
 
 struct KnnLayout {
-  size_t partial, count, keys_a, keys_b, vals_a, vals_b, sorted, hist, leaves, nodes, tops, total;
+  size_t partial, keys_a, keys_b, vals_a, vals_b, sorted, hist, leaves, nodes, tops, total;
   long long n_leaf, n_node, n_top;
   int bits;  // of the curve, per axis
 };
@@ -52,8 +52,6 @@ constexpr KnnLayout knn_layout(int P) {
   size_t o = 0;
   L.partial = o;
   o = align_up(o + 24 * (size_t)kKnnParts, 256);
-  L.count = o;
-  o = align_up(o + 4, 256);
   // the gathered points take the place of three of the sort's four buffers
   // and of the fourth's size beyond; the sorted indices stay out of it
   const size_t n4 = align_up(4 * (size_t)padded, 256);
@@ -173,8 +171,7 @@ __device__ __forceinline__ float from_ordered(uint32_t u) {
 }
 
 __global__ __launch_bounds__(256) void k_knn_keys(const float* pts, int P, const float* partial, int parts, int bits,
-                                                  uint32_t* count, uint32_t* keys, uint32_t* vals, uint32_t* tops,
-                                                  int n_top) {
+                                                  uint32_t* keys, uint32_t* vals, uint32_t* tops, int n_top) {
   __shared__ float s[16][6];
   float lo[3] = {inf_f(), inf_f(), inf_f()}, hi[3] = {-inf_f(), -inf_f(), -inf_f()};
   if ((int)threadIdx.x < parts)
@@ -187,7 +184,6 @@ __global__ __launch_bounds__(256) void k_knn_keys(const float* pts, int P, const
   const float side = fmaxf(hi[0] - lo[0], fmaxf(hi[1] - lo[1], hi[2] - lo[2]));
   const float scale = side > 0.0f ? (float)(1 << bits) / side : 0.0f;
   const int i = blockIdx.x * 256 + threadIdx.x;
-  if (i == 0) *count = (uint32_t)P;
   for (int t = i; t < 6 * n_top; t += gridDim.x * 256) tops[t] = ordered(t % 6 < 3 ? inf_f() : -inf_f());
   if (i >= P) return;
   uint32_t c[3];
@@ -379,7 +375,6 @@ __global__ __launch_bounds__(256) void k_knn_query(int n_group, int n_leaf, int 
 // The launch sequence over a workspace laid out by knn_layout(P).
 static int knn_launch(const float* points, int P, float* out, char* b, const KnnLayout& L, hipStream_t s) {
   float* partial = (float*)(b + L.partial);
-  uint32_t* count = (uint32_t*)(b + L.count);
   uint32_t *ka = (uint32_t*)(b + L.keys_a), *kb = (uint32_t*)(b + L.keys_b);
   uint32_t *va = (uint32_t*)(b + L.vals_a), *vb = (uint32_t*)(b + L.vals_b);
   float4* sorted = (float4*)(b + L.sorted);
@@ -388,10 +383,10 @@ static int knn_launch(const float* points, int P, float* out, char* b, const Knn
   const int nb = (P + 255) / 256, parts = nb < kKnnParts ? nb : kKnnParts, n_group = (P + 63) / 64;
   timing::Scope ts(timing::kKnn, s);
   hipLaunchKernelGGL(k_knn_bbox, dim3(parts), dim3(256), 0, s, points, P, partial);
-  hipLaunchKernelGGL(k_knn_keys, dim3(nb), dim3(256), 0, s, points, P, partial, parts, L.bits, count, ka, va, tops,
+  hipLaunchKernelGGL(k_knn_keys, dim3(nb), dim3(256), 0, s, points, P, partial, parts, L.bits, ka, va, tops,
                      (int)L.n_top);
   int in_b;
-  if (sort_pairs_u32(ka, va, kb, vb, count, P, 3 * L.bits, b + L.hist, s, &in_b) != hipSuccess) return GS_E_LAUNCH;
+  if (sort_pairs_u32(ka, va, kb, vb, nullptr, P, 3 * L.bits, b + L.hist, s, &in_b) != hipSuccess) return GS_E_LAUNCH;
   hipLaunchKernelGGL(k_knn_gather, dim3((unsigned)L.n_node), dim3(1024), 0, s, points, P, in_b ? vb : va, sorted,
                      leaves, nodes, tops);
   hipLaunchKernelGGL(k_knn_query, dim3((n_group + 3) / 4), dim3(256), 0, s, n_group, (int)L.n_leaf, (int)L.n_node,

@@ -9,12 +9,15 @@
 // Keys-only sorts (32-bit keys that carry their payload in the low bits)
 // sort bits [start_bit, end_bit) and skip every value load and store.
 //
-// Per 8-bit digit pass:
-//   k_sort_upsweep  1024 or 2048 keys per workgroup (4 waves x 4 or 8 rounds
-//                   x 64 lanes), all loaded up front, counted with one LDS
-//                   atomic each -> per-workgroup digit counts (digit-major,
-//                   so one row scan per digit orders blocks)
-//   k_sort_scan     one workgroup per digit: exclusive scan of its row, total
+// A sort of B bits takes ceil(B / 8) passes of near equal digits; a keys-only
+// sort of 9 or 10 bits (the lists of up to 1024 tiles) takes one pass.  Per pass:
+//   k_sort_upsweep  1024 or 2048 keys per workgroup (4096 with 10-bit digits),
+//                   4 waves x 4, 8 or 16 rounds x 64 lanes, all loaded up
+//                   front, counted with one LDS atomic each -> per-workgroup
+//                   digit counts
+//   k_sort_scan     one workgroup per digit: exclusive scan of its row, total.
+//                   Sorts of up to kDirectBlocks workgroups have no such
+//                   launch: each scatter workgroup adds the counts up itself
 //   k_sort_scatter  recomputes the matches; rank = prior count of the digit in
 //                   this wave + lanes below with the same digit; waves are
 //                   ordered by an exclusive prefix over the 4 wave counts, so
@@ -23,6 +26,12 @@
 //                   order, then written out by consecutive threads: each
 //                   digit's run leaves as contiguous stores instead of one
 //                   scattered 4-byte store per lane.
+// Short sorts are bound by the chain of launches and of loads in each.  One pass
+// instead of two for 510 tiles: 28 us of kernels -> 22 (137 000 entries).  Long ones
+// are bound by memory: 71 million (key, value) pairs of 13 bits took 386 us a
+// scatter with digits of 8 and 5 bits over 2048 keys, where a digit's run in a
+// workgroup is 32 bytes and the counts as much again; with 7 and 6 bits over 4096
+// keys 275, 4.1 TB/s.
 // Upsweep and scatter map workgroups to key blocks XCD-aware (xcd_remap):
 // dispatch deals workgroups round-robin over the 8 XCDs, and each XCD gets a
 // contiguous run of blocks.  A cache line of a digit's counts covers 32
@@ -65,7 +74,9 @@ __device__ __forceinline__ uint32_t block_incl_scan256(uint32_t v, uint32_t* s_w
   return x + (w > 0 ? w0 : 0u) + (w > 1 ? w1 : 0u) + (w > 2 ? w2 : 0u);
 }
 
+// The element count: *n_dev, 0 past the capacity; the capacity without n_dev.
 __device__ __forceinline__ uint32_t n_eff(const uint32_t* n_dev, long long cap) {
+  if (!n_dev) return (uint32_t)cap;
   const uint32_t n = *n_dev;
   return ((long long)n > cap) ? 0u : n;
 }
@@ -75,7 +86,8 @@ __device__ __forceinline__ uint32_t n_eff(const uint32_t* n_dev, long long cap) 
 // segment).
 template <typename K, int ITEMS, int R>
 __device__ __forceinline__ void upsweep_block(const K* __restrict__ keys, const uint32_t* n_dev, long long cap,
-                                              int shift, int bits, uint32_t* hist, int nb_max, uint32_t bid) {
+                                              int shift, int bits, uint32_t* hist, int nb_max, bool direct,
+                                              uint32_t bid) {
   __shared__ uint32_t s_h[4][R];
   const uint32_t n = n_eff(n_dev, cap);
   constexpr uint32_t TILE = kSortThreads * ITEMS;
@@ -177,14 +189,14 @@ __device__ __forceinline__ void upsweep_block(const K* __restrict__ keys, const 
   }
   __syncthreads();
   for (int d = threadIdx.x; d < R; d += kSortThreads)
-    hist[(size_t)d * nb_max + blk] = s_h[0][d] + s_h[1][d] + s_h[2][d] + s_h[3][d];
+    hist[direct ? (size_t)blk * R + d : (size_t)d * nb_max + blk] = s_h[0][d] + s_h[1][d] + s_h[2][d] + s_h[3][d];
 }
 
 template <typename K, int ITEMS, int R>
 __global__ __launch_bounds__(kSortThreads) void k_sort_upsweep(const K* __restrict__ keys, const uint32_t* n_dev,
                                                                long long cap, int shift, int bits, uint32_t* hist,
-                                                               int nb_max) {
-  upsweep_block<K, ITEMS, R>(keys, n_dev, cap, shift, bits, hist, nb_max, blockIdx.x);
+                                                               int nb_max, bool direct) {
+  upsweep_block<K, ITEMS, R>(keys, n_dev, cap, shift, bits, hist, nb_max, direct, blockIdx.x);
 }
 
 // One workgroup per digit: exclusive scan over the active blocks' counts.
@@ -221,6 +233,43 @@ __device__ __forceinline__ void scan_row(uint32_t* hist, uint32_t* totals, const
   if (t == 0) totals[d] = carry;
 }
 
+// The same for 10-bit digits, whose rows are short (at most 512 workgroups): a
+// wave a row, four to a workgroup.
+__device__ __forceinline__ void scan_row_wide(uint32_t* hist, uint32_t* totals, const uint32_t* n_dev, long long cap,
+                                              int nb_max, int tile, int d) {
+  const uint32_t n = n_eff(n_dev, cap);
+  const int nb = (int)((n + tile - 1) / tile), lane = threadIdx.x & 63;
+  uint32_t* row = hist + (size_t)d * nb_max;
+  uint32_t carry = 0;
+  for (int b0 = 0; b0 < nb; b0 += 64 * kScanRun) {
+    const int first = b0 + lane * kScanRun;
+    uint32_t v[kScanRun], sum = 0;
+#pragma unroll
+    for (int j = 0; j < kScanRun; ++j) v[j] = first + j < nb ? row[first + j] : 0u;
+#pragma unroll
+    for (int j = 0; j < kScanRun; ++j) sum += v[j];
+    uint32_t x = sum;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const uint32_t y = __shfl_up(x, off, 64);
+      if (lane >= off) x += y;
+    }
+    uint32_t run = carry + x - sum;
+#pragma unroll
+    for (int j = 0; j < kScanRun; ++j) {
+      if (first + j < nb) row[first + j] = run;
+      run += v[j];
+    }
+    carry += __shfl(x, 63, 64);
+  }
+  if (lane == 0) totals[d] = carry;
+}
+
+__global__ __launch_bounds__(256) void k_sort_scan_wide(uint32_t* hist, uint32_t* totals, const uint32_t* n_dev,
+                                                        long long cap, int nb_max, int tile) {
+  scan_row_wide(hist, totals, n_dev, cap, nb_max, tile, (int)(blockIdx.x * 4 + (threadIdx.x >> 6)));
+}
+
 __global__ __launch_bounds__(256) void k_sort_scan(uint32_t* hist, uint32_t* totals, const uint32_t* n_dev,
                                                    long long cap, int nb_max, int tile) {
   scan_row(hist, totals, n_dev, cap, nb_max, tile, blockIdx.x);
@@ -231,9 +280,9 @@ __device__ __forceinline__ void scatter_block(const K* __restrict__ keys_in, con
                                               K* __restrict__ keys_out, uint32_t* __restrict__ vals_out,
                                               const uint32_t* n_dev, long long cap, int shift, int bits,
                                               const uint32_t* hist, const uint32_t* totals, int nb_max,
-                                              uint32_t* ranges, int tshift, uint32_t bid) {
-  static_assert(R == kSortThreads, "one digit per thread");
-  constexpr int TILE = kSortThreads * ITEMS;
+                                              uint32_t* ranges, int tshift, bool direct, uint32_t bid) {
+  static_assert(R % kSortThreads == 0, "thread t keeps digits [t DP, t DP + DP)");
+  constexpr int TILE = kSortThreads * ITEMS, DP = R / kSortThreads;
   __shared__ uint32_t s_cnt[4][R];
   __shared__ uint32_t s_scan[R];
   __shared__ uint32_t s_w[4];
@@ -245,26 +294,67 @@ __device__ __forceinline__ void scatter_block(const K* __restrict__ keys_in, con
   const uint32_t blk = xcd_remap(bid, nblk);  // the upsweep's mapping
   const uint32_t start = blk * (uint32_t)TILE;
   const int t = threadIdx.x;
-  // global base of each digit for this block = exclusive scan of totals + row offset
-  {
-    const uint32_t v = totals[t];
-    uint32_t tot;
-    s_scan[t] = block_incl_scan256(v, s_w, tot) - v + hist[(size_t)t * nb_max + blk];
-  }
-  for (int k = t; k < 4 * R; k += kSortThreads) (&s_cnt[0][0])[k] = 0;
-  __syncthreads();
   const int w = t >> 6, lane = t & 63;
   const uint32_t mask = (1u << bits) - 1u;
   const uint32_t wbase = start + (uint32_t)w * (ITEMS * 64);
+  // the keys are on their way while the counts are read
   K key[ITEMS];
   uint32_t val[ITEMS];
   uint32_t pos[ITEMS];
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
     const uint32_t idx = wbase + r * 64 + lane;
-    const bool valid = idx < n;
-    key[r] = valid ? keys_in[idx] : (K)0;
-    if constexpr (V) val[r] = valid ? vals_in[idx] : 0u;
+    key[r] = idx < n ? keys_in[idx] : (K)0;
+    if constexpr (V) val[r] = idx < n ? vals_in[idx] : 0u;
+  }
+  // global base of each digit for this block = exclusive scan of the digits'
+  // totals + the digit's count in the blocks before
+  {
+    uint32_t total[DP], before[DP], sum = 0;
+    bool added = false;
+    if constexpr (DP == 1) {
+      if (direct) {
+        added = true;
+        total[0] = before[0] = 0;
+        for (uint32_t b0 = 0; b0 < nblk; b0 += 16) {
+          uint32_t c[16];
+#pragma unroll
+          for (uint32_t j = 0; j < 16; ++j) c[j] = hist[(size_t)min(b0 + j, nblk - 1u) * R + t];
+#pragma unroll
+          for (uint32_t j = 0; j < 16; ++j) {
+            total[0] += b0 + j < nblk ? c[j] : 0u;
+            before[0] += b0 + j < blk ? c[j] : 0u;
+          }
+        }
+      }
+    }
+    if (!added) {
+#pragma unroll
+      for (int i = 0; i < DP; ++i) {
+        total[i] = totals[t * DP + i];
+        before[i] = hist[(size_t)(t * DP + i) * nb_max + blk];
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < DP; ++i) sum += total[i];
+    uint32_t tot;
+    uint32_t run = block_incl_scan256(sum, s_w, tot) - sum;
+#pragma unroll
+    for (int i = 0; i < DP; ++i) {
+      s_scan[t * DP + i] = run + before[i];
+      // in a sort of one pass the digit is the tile id
+      if (ranges && shift == tshift && blk == 0 && total[i] > 0) {
+        ranges[2 * (t * DP + i)] = run;
+        ranges[2 * (t * DP + i) + 1] = run + total[i];
+      }
+      run += total[i];
+    }
+  }
+  for (int k = t; k < 4 * R; k += kSortThreads) (&s_cnt[0][0])[k] = 0;
+  __syncthreads();
+#pragma unroll
+  for (int r = 0; r < ITEMS; ++r) {
+    const bool valid = wbase + r * 64 + lane < n;
     const uint32_t d = (uint32_t)(key[r] >> shift) & mask;
     const uint64_t peers = match_digit(d, valid, bits);
     const uint64_t below = peers & lanemask_lt();
@@ -273,17 +363,29 @@ __device__ __forceinline__ void scatter_block(const K* __restrict__ keys_in, con
     if (valid && below == 0) s_cnt[w][d] = prior + (uint32_t)__popcll(peers);
   }
   __syncthreads();
-  // digit t: its waves' local bases (exclusive scan over digits of the block
+  // each digit's waves' local bases (exclusive scan over digits of the block
   // counts, then over waves) and the offset from local to global position
-  const uint32_t c0 = s_cnt[0][t], c1 = s_cnt[1][t], c2 = s_cnt[2][t], c3 = s_cnt[3][t];
-  const uint32_t c = c0 + c1 + c2 + c3;
-  uint32_t tot;
-  const uint32_t lbase = block_incl_scan256(c, s_w, tot) - c;
-  s_cnt[0][t] = lbase;
-  s_cnt[1][t] = lbase + c0;
-  s_cnt[2][t] = lbase + c0 + c1;
-  s_cnt[3][t] = lbase + c0 + c1 + c2;
-  s_scan[t] = s_scan[t] - lbase;  // global = s_scan[d] + local position
+  {
+    uint32_t c[DP][4], sum = 0;
+#pragma unroll
+    for (int i = 0; i < DP; ++i)
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        c[i][k] = s_cnt[k][t * DP + i];
+        sum += c[i][k];
+      }
+    uint32_t tot;
+    uint32_t run = block_incl_scan256(sum, s_w, tot) - sum;
+#pragma unroll
+    for (int i = 0; i < DP; ++i) {
+      s_scan[t * DP + i] -= run;  // global = s_scan[d] + local position
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        s_cnt[k][t * DP + i] = run;
+        run += c[i][k];
+      }
+    }
+  }
   __syncthreads();
 #pragma unroll
   for (int r = 0; r < ITEMS; ++r) {
@@ -303,7 +405,7 @@ __device__ __forceinline__ void scatter_block(const K* __restrict__ keys_in, con
     const uint32_t dst = s_scan[d] + i;
     keys_out[dst] = k;
     if constexpr (V) vals_out[dst] = s_val[i];
-    if (ranges) {
+    if (ranges && shift != tshift) {
       // last pass of a tile-list sort: within a digit run the block's keys are
       // in final order, so a run of one tile id is contiguous here and in the
       // output; its ends give the tile's [start, end) across blocks by
@@ -323,24 +425,46 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const K* __restri
                                                                const uint32_t* n_dev, long long cap, int shift,
                                                                int bits, const uint32_t* hist,
                                                                const uint32_t* totals, int nb_max, uint32_t* ranges,
-                                                               int tshift) {
+                                                               int tshift, bool direct) {
   scatter_block<K, ITEMS, R, V>(keys_in, vals_in, keys_out, vals_out, n_dev, cap, shift, bits, hist, totals, nb_max,
-                                ranges, tshift, blockIdx.x);
+                                ranges, tshift, direct, blockIdx.x);
 }
+
+// Up to this many workgroups the scatter adds the counts up itself.  At 10 (10
+// 000 keys) a pass then takes 8.9 us of kernels instead of 12.9; at 98 to 127 the
+// scatter's reading of every count (6.9 -> 9.5 us) costs what the scan did.
+constexpr int kDirectBlocks = 32;
 
 template <typename K, int ITEMS, int R>
 void sort_pass(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout, const uint32_t* n_dev, long long capacity,
-               int shift, int bits, uint32_t* hist, uint32_t* totals, int nb_max, int tile, hipStream_t s,
-               uint32_t* ranges, int tshift) {
+               int shift, int bits, uint32_t* hist, uint32_t* totals, int nb_max, hipStream_t s, uint32_t* ranges,
+               int tshift) {
+  const bool direct = R == kRadix && nb_max <= kDirectBlocks;
   hipLaunchKernelGGL((k_sort_upsweep<K, ITEMS, R>), dim3(nb_max), dim3(kSortThreads), 0, s, kin, n_dev, capacity,
-                     shift, bits, hist, nb_max);
-  hipLaunchKernelGGL(k_sort_scan, dim3(R), dim3(256), 0, s, hist, totals, n_dev, capacity, nb_max, tile);
-  if (vin)
-    hipLaunchKernelGGL((k_sort_scatter<K, ITEMS, R, true>), dim3(nb_max), dim3(kSortThreads), 0, s, kin, vin, kout,
-                       vout, n_dev, capacity, shift, bits, hist, totals, nb_max, ranges, tshift);
-  else
-    hipLaunchKernelGGL((k_sort_scatter<K, ITEMS, R, false>), dim3(nb_max), dim3(kSortThreads), 0, s, kin, vin, kout,
-                       vout, n_dev, capacity, shift, bits, hist, totals, nb_max, ranges, tshift);
+                     shift, bits, hist, nb_max, direct);
+  if (R == kWideRadix)
+    hipLaunchKernelGGL(k_sort_scan_wide, dim3(R / 4), dim3(256), 0, s, hist, totals, n_dev, capacity, nb_max,
+                       kSortThreads * ITEMS);
+  else if (!direct)
+    hipLaunchKernelGGL(k_sort_scan, dim3(1u << bits), dim3(256), 0, s, hist, totals, n_dev, capacity, nb_max,
+                       kSortThreads * ITEMS);
+  if constexpr (R == kRadix) {
+    if (vin) {
+      hipLaunchKernelGGL((k_sort_scatter<K, ITEMS, R, true>), dim3(nb_max), dim3(kSortThreads), 0, s, kin, vin, kout,
+                         vout, n_dev, capacity, shift, bits, hist, totals, nb_max, ranges, tshift, direct);
+      return;
+    }
+  }
+  hipLaunchKernelGGL((k_sort_scatter<K, ITEMS, R, false>), dim3(nb_max), dim3(kSortThreads), 0, s, kin, vin, kout,
+                     vout, n_dev, capacity, shift, bits, hist, totals, nb_max, ranges, tshift, direct);
+}
+
+// Pass p of a sort of bits [start_bit, end_bit) in `passes` near equal digits:
+// its first bit and its width.
+inline void pass_digit(int start_bit, int end_bit, int passes, int p, int& shift, int& bits) {
+  const int total = end_bit - start_bit, base = total / passes, more = total % passes;
+  shift = start_bit + p * base + (p < more ? p : more);
+  bits = base + (p < more ? 1 : 0);
 }
 
 // Stable LSD sort on key bits [start_bit, end_bit); vals_a == nullptr sorts
@@ -351,29 +475,29 @@ template <typename K>
 hipError_t sort_pairs(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, const uint32_t* n_dev,
                       long long capacity, int start_bit, int end_bit, void* tmp, hipStream_t s, int* result_in_b,
                       uint32_t* ranges = nullptr) {
-  const int passes = sort_passes(end_bit - start_bit);
+  const bool wide = sizeof(K) == 4 && !vals_a && wide_digit(end_bit - start_bit, capacity);
+  const int passes = wide ? 1 : sort_passes(end_bit - start_bit);
   *result_in_b = passes & 1;
   if (capacity <= 0) return hipSuccess;
-  const int tile = sort_tile(capacity);
+  const int tile = wide ? kSortThreads * kWideItems : sort_tile(capacity);
   const int nb_max = (int)((capacity + tile - 1) / tile);
   uint32_t* hist = (uint32_t*)tmp;
-  uint32_t* totals = hist + align_up((size_t)kRadix * (size_t)nb_max, 64);
+  uint32_t* totals = hist + align_up((size_t)(wide ? kWideRadix : kRadix) * (size_t)nb_max, 64);
   K* kin = keys_a;
   uint32_t* vin = vals_a;
   K* kout = keys_b;
   uint32_t* vout = vals_b;
   for (int p = 0; p < passes; ++p) {
-    const int shift = start_bit + kRadixBits * p;
-    const int bits = end_bit - shift < kRadixBits ? end_bit - shift : kRadixBits;
+    int shift, bits;
+    pass_digit(start_bit, end_bit, passes, p, shift, bits);
     auto pass = tile == kSortThreads * 4 ? sort_pass<K, 4, kRadix> : sort_pass<K, 8, kRadix>;
-    pass(kin, vin, kout, vout, n_dev, capacity, shift, bits, hist, totals, nb_max, tile, s,
-         p + 1 == passes ? ranges : nullptr, start_bit);
-    K* tk = kin;
-    kin = kout;
-    kout = tk;
-    uint32_t* tv = vin;
-    vin = vout;
-    vout = tv;
+    if (tile == kSortThreads * 16) pass = sort_pass<K, 16, kRadix>;
+    if constexpr (sizeof(K) == 4)
+      if (wide) pass = sort_pass<K, kWideItems, kWideRadix>;
+    pass(kin, vin, kout, vout, n_dev, capacity, shift, bits, hist, totals, nb_max, s, p + 1 == passes ? ranges : nullptr,
+         start_bit);
+    std::swap(kin, kout);
+    std::swap(vin, vout);
   }
   return hipGetLastError();
 }
@@ -383,8 +507,9 @@ hipError_t sort_pairs(K* keys_a, uint32_t* vals_a, K* keys_b, uint32_t* vals_b, 
 // scatter workgroups in that pass, rounded up to a multiple of 8 so that a
 // segment's first block starts a round of the XCD round-robin, as a launch
 // of its own does; 0 once the segment has no pass left), then one SegPass
-// per segment.  Every segment sorts with 1024-key workgroups (sort_tile of a
-// capacity up to kSegMaxKeys).
+// per segment.  The segments of a sort share their workgroups' size and digit
+// array: 4096 keys and 10-bit digits if any segment takes such a digit, else
+// 1024 keys (sort_tile of a capacity up to kSegMaxKeys) and 8-bit ones.
 struct SegPass {
   const uint32_t* kin;
   const uint32_t* vin;
@@ -401,6 +526,8 @@ struct SegPass {
   int tshift;
 };
 constexpr int kSegItems = 4;
+// beside a pass's workgroup count in blocks[p]: what the launch has to know
+constexpr unsigned kSegWide = 1u << 31, kSegDirect = 1u << 30, kSegBlocks = kSegDirect - 1u;
 
 static size_t seg_pass_bytes(int n) {
   return align_up(sizeof(uint32_t) * (size_t)(n + 1), 256) + align_up(sizeof(SegPass) * (size_t)n, 256);
@@ -417,28 +544,39 @@ __device__ __forceinline__ int seg_of(const uint32_t* prefix, int n, uint32_t b)
   return lo;
 }
 
-__global__ __launch_bounds__(kSortThreads) void k_seg_upsweep(const uint32_t* prefix, const SegPass* ps, int n) {
+template <int ITEMS, int R>
+__global__ __launch_bounds__(kSortThreads) void k_seg_upsweep(const uint32_t* prefix, const SegPass* ps, int n,
+                                                              bool direct) {
   const uint32_t b = blockIdx.x;
   const int f = seg_of(prefix, n, b);
   const SegPass p = ps[f];
-  upsweep_block<uint32_t, kSegItems, kRadix>(p.kin, p.n_dev, p.cap, p.shift, p.bits, p.hist, p.nb_max,
-                                             b - prefix[f]);
+  upsweep_block<uint32_t, ITEMS, R>(p.kin, p.n_dev, p.cap, p.shift, p.bits, p.hist, p.nb_max, direct, b - prefix[f]);
 }
 
 // 256 workgroups per segment, one per digit.
 __global__ __launch_bounds__(256) void k_seg_scan(const SegPass* ps) {
   const SegPass p = ps[blockIdx.x >> kRadixBits];
-  if (p.nb_max == 0) return;
-  scan_row(p.hist, p.totals, p.n_dev, p.cap, p.nb_max, kSortThreads * kSegItems, (int)(blockIdx.x & (kRadix - 1)));
+  const int d = (int)(blockIdx.x & (kRadix - 1));
+  if (p.nb_max == 0 || d >> p.bits) return;
+  scan_row(p.hist, p.totals, p.n_dev, p.cap, p.nb_max, kSortThreads * kSegItems, d);
 }
 
-template <bool V>
-__global__ __launch_bounds__(kSortThreads) void k_seg_scatter(const uint32_t* prefix, const SegPass* ps, int n) {
+// 256 workgroups per segment, four digits each.
+__global__ __launch_bounds__(256) void k_seg_scan_wide(const SegPass* ps) {
+  const SegPass p = ps[blockIdx.x / (kWideRadix / 4)];
+  const int d = (int)(blockIdx.x % (kWideRadix / 4) * 4 + (threadIdx.x >> 6));
+  if (p.nb_max == 0 || d >> p.bits) return;
+  scan_row_wide(p.hist, p.totals, p.n_dev, p.cap, p.nb_max, kSortThreads * kWideItems, d);
+}
+
+template <int ITEMS, int R, bool V>
+__global__ __launch_bounds__(kSortThreads) void k_seg_scatter(const uint32_t* prefix, const SegPass* ps, int n,
+                                                              bool direct) {
   const uint32_t b = blockIdx.x;
   const int f = seg_of(prefix, n, b);
   const SegPass p = ps[f];
-  scatter_block<uint32_t, kSegItems, kRadix, V>(p.kin, p.vin, p.kout, p.vout, p.n_dev, p.cap, p.shift, p.bits,
-                                                p.hist, p.totals, p.nb_max, p.ranges, p.tshift, b - prefix[f]);
+  scatter_block<uint32_t, ITEMS, R, V>(p.kin, p.vin, p.kout, p.vout, p.n_dev, p.cap, p.shift, p.bits, p.hist,
+                                       p.totals, p.nb_max, p.ranges, p.tshift, direct, b - prefix[f]);
 }
 
 size_t seg_sort_desc_bytes(int n, int passes) {
@@ -450,16 +588,22 @@ bool seg_sort_build(int n, const SortSeg* segs, void* host, size_t bytes, unsign
   if (n <= 0 || !segs || !host || !blocks || !passes) return false;
   int np = 0;
   const bool values = segs[0].vals_a != nullptr;
+  bool wide = false;
+  long long most = 0;
   for (int f = 0; f < n; ++f) {
     const SortSeg& g = segs[f];
-    if (g.capacity <= 0 || g.capacity > kSegMaxKeys || !g.keys_a || !g.keys_b || !g.n_dev || !g.tmp) return false;
+    if (g.capacity <= 0 || g.capacity > kSegMaxKeys || !g.keys_a || !g.keys_b || !g.tmp) return false;
     if ((g.vals_a != nullptr) != values || (values && !g.vals_b)) return false;
     if (g.start_bit < 0 || g.end_bit <= g.start_bit || g.end_bit > 32) return false;
     if (((uintptr_t)g.keys_a | (uintptr_t)g.keys_b) & 15) return false;  // 16-byte key loads
-    if (sort_tile(g.capacity) != kSortThreads * kSegItems) return false;
-    np = std::max(np, sort_passes(g.end_bit - g.start_bit));
+    const bool gw = !values && wide_digit(g.end_bit - g.start_bit, g.capacity);
+    wide |= gw;
+    most = std::max(most, g.capacity);
+    np = std::max(np, gw ? 1 : sort_passes(g.end_bit - g.start_bit));
   }
   if (np > kSegMaxPasses || bytes < seg_sort_desc_bytes(n, np)) return false;
+  const int tile = kSortThreads * (wide ? kWideItems : kSegItems);
+  const bool direct = !wide && (most + tile - 1) / tile <= kDirectBlocks;
   for (int p = 0; p < kSegMaxPasses; ++p) blocks[p] = 0;
   for (int p = 0; p < np; ++p) {
     char* base = (char*)host + seg_pass_bytes(n) * (size_t)p;
@@ -468,9 +612,9 @@ bool seg_sort_build(int n, const SortSeg* segs, void* host, size_t bytes, unsign
     unsigned long long total = 0;
     for (int f = 0; f < n; ++f) {
       const SortSeg& g = segs[f];
-      const int tile = kSortThreads * kSegItems;
       const int nb_max = (int)((g.capacity + tile - 1) / tile);
-      const int gp = sort_passes(g.end_bit - g.start_bit);
+      const int width = g.end_bit - g.start_bit;
+      const int gp = !values && wide_digit(width, g.capacity) ? 1 : sort_passes(width);
       uint32_t* hist = (uint32_t*)g.tmp;
       SegPass& q = ps[f];
       const bool odd = p & 1;
@@ -480,22 +624,33 @@ bool seg_sort_build(int n, const SortSeg* segs, void* host, size_t bytes, unsign
       q.vout = odd ? g.vals_a : g.vals_b;
       q.n_dev = g.n_dev;
       q.hist = hist;
-      q.totals = hist + align_up((size_t)kRadix * (size_t)nb_max, 64);  // sort_pairs' layout of tmp
+      q.totals = hist + align_up((size_t)(wide ? kWideRadix : kRadix) * (size_t)nb_max, 64);  // sort_pairs' layout of tmp
       q.ranges = p + 1 == gp ? g.ranges : nullptr;
       q.cap = g.capacity;
       q.nb_max = p < gp ? nb_max : 0;
-      q.shift = g.start_bit + kRadixBits * p;
-      q.bits = g.end_bit - q.shift < kRadixBits ? g.end_bit - q.shift : kRadixBits;
+      q.shift = q.bits = 0;
+      if (p < gp) pass_digit(g.start_bit, g.end_bit, gp, p, q.shift, q.bits);
       q.tshift = g.start_bit;
       prefix[f] = (uint32_t)total;
       total += p < gp ? align_up((size_t)nb_max, 8) : 0;
-      if (total > 0x7fffffffULL) return false;
+      if (total > kSegBlocks) return false;
     }
     prefix[n] = (uint32_t)total;
-    blocks[p] = (unsigned)total;
+    blocks[p] = (unsigned)total | (wide ? kSegWide : 0u) | (direct ? kSegDirect : 0u);
   }
   *passes = np;
   return true;
+}
+
+template <int ITEMS, int R, bool V>
+static void seg_pass_launch(int n, const uint32_t* prefix, const SegPass* q, unsigned blocks, bool direct,
+                            hipStream_t s) {
+  hipLaunchKernelGGL((k_seg_upsweep<ITEMS, R>), dim3(blocks), dim3(kSortThreads), 0, s, prefix, q, n, direct);
+  if (R == kWideRadix)
+    hipLaunchKernelGGL(k_seg_scan_wide, dim3((unsigned)n * (kWideRadix / 4)), dim3(256), 0, s, q);
+  else if (!direct)
+    hipLaunchKernelGGL(k_seg_scan, dim3((unsigned)n * kRadix), dim3(256), 0, s, q);
+  hipLaunchKernelGGL((k_seg_scatter<ITEMS, R, V>), dim3(blocks), dim3(kSortThreads), 0, s, prefix, q, n, direct);
 }
 
 hipError_t seg_sort_launch(int n, const void* dev_desc, const unsigned* blocks, bool values, hipStream_t s) {
@@ -503,12 +658,11 @@ hipError_t seg_sort_launch(int n, const void* dev_desc, const unsigned* blocks, 
     const char* base = (const char*)dev_desc + seg_pass_bytes(n) * (size_t)p;
     const uint32_t* prefix = (const uint32_t*)base;
     const SegPass* q = (const SegPass*)(base + align_up(sizeof(uint32_t) * (size_t)(n + 1), 256));
-    hipLaunchKernelGGL(k_seg_upsweep, dim3(blocks[p]), dim3(kSortThreads), 0, s, prefix, q, n);
-    hipLaunchKernelGGL(k_seg_scan, dim3((unsigned)n * kRadix), dim3(256), 0, s, q);
-    if (values)
-      hipLaunchKernelGGL(k_seg_scatter<true>, dim3(blocks[p]), dim3(kSortThreads), 0, s, prefix, q, n);
-    else
-      hipLaunchKernelGGL(k_seg_scatter<false>, dim3(blocks[p]), dim3(kSortThreads), 0, s, prefix, q, n);
+    const unsigned nb = blocks[p] & kSegBlocks;
+    const bool direct = blocks[p] & kSegDirect;
+    if (values) seg_pass_launch<kSegItems, kRadix, true>(n, prefix, q, nb, direct, s);
+    else if (blocks[p] & kSegWide) seg_pass_launch<kWideItems, kWideRadix, false>(n, prefix, q, nb, direct, s);
+    else seg_pass_launch<kSegItems, kRadix, false>(n, prefix, q, nb, direct, s);
   }
   return hipGetLastError();
 }

@@ -123,7 +123,7 @@ typedef struct gs_binning_layout {
   size_t keys_alt, vals_alt;   /* ping-pong buffers of the radix sort */
   size_t keys_sorted, vals_sorted; /* whichever of the above holds the sorted result */
   size_t hist;                 /* sort digit histograms */
-  int sort_passes;             /* 8-bit LSD passes of the list sort */
+  int sort_passes;             /* LSD passes of the list sort */
   int key_bytes;               /* 8 (SORT64) or 4 (DEPTH_FIRST) */
   int id_bits;                 /* DEPTH_FIRST with bits(P) + bits(n_tiles) <= 32: the list entries are
                                   single words tile << id_bits | Gaussian id, sorted in place of the keys
