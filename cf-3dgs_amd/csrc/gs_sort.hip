@@ -432,8 +432,10 @@ __global__ __launch_bounds__(kSortThreads) void k_sort_scatter(const K* __restri
 
 // Up to this many workgroups the scatter adds the counts up itself.  At 10 (10
 // 000 keys) a pass then takes 8.9 us of kernels instead of 12.9; at 98 to 127 the
-// scatter's reading of every count (6.9 -> 9.5 us) costs what the scan did.
-constexpr int kDirectBlocks = 32;
+// scatter's reading of every count (6.9 -> 9.5 us) costs what the scan did, but
+// the host is spared 3 us for its launch.  A segmented sort, which runs in
+// graphs, takes the lower limit.
+constexpr int kDirectBlocks = 128, kSegDirectBlocks = 32;
 
 template <typename K, int ITEMS, int R>
 void sort_pass(const K* kin, const uint32_t* vin, K* kout, uint32_t* vout, const uint32_t* n_dev, long long capacity,
@@ -603,7 +605,7 @@ bool seg_sort_build(int n, const SortSeg* segs, void* host, size_t bytes, unsign
   }
   if (np > kSegMaxPasses || bytes < seg_sort_desc_bytes(n, np)) return false;
   const int tile = kSortThreads * (wide ? kWideItems : kSegItems);
-  const bool direct = !wide && (most + tile - 1) / tile <= kDirectBlocks;
+  const bool direct = !wide && (most + tile - 1) / tile <= kSegDirectBlocks;
   for (int p = 0; p < kSegMaxPasses; ++p) blocks[p] = 0;
   for (int p = 0; p < np; ++p) {
     char* base = (char*)host + seg_pass_bytes(n) * (size_t)p;

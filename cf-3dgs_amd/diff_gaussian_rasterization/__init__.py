@@ -79,7 +79,8 @@ class _RasterizeGaussians(torch.autograd.Function):
         cv_ = _none_if_empty(cov3Ds_precomp)
         po_ = _none_if_empty(pose)
         color, radii, depth, alpha, st = _raster.forward(
-            raster_settings, means3D, sh_, col_, opacities, sc_, ro_, cv_, pose=po_, want_alpha=True)
+            raster_settings, means3D, sh_, col_, opacities, sc_, ro_, cv_, pose=po_,
+            want_alpha=return_alpha)
         if raster_settings.debug:
             torch.cuda.synchronize(means3D.device)
         ctx.raster_settings = raster_settings
@@ -118,7 +119,7 @@ class _RasterizeGaussians(torch.autograd.Function):
 
         def shaped(name, like):
             t = g[name]
-            return t.view_as(like) if t is not None else None
+            return t if t is None or t.shape == like.shape else t.view_as(like)
 
         grad_means3D = shaped("means3D", means3D)
         grad_means2D = g["means2D"]
@@ -135,17 +136,8 @@ class _RasterizeGaussians(torch.autograd.Function):
 
 def rasterize_gaussians(means3D, means2D, sh, colors_precomp, opacities, scales, rotations, cov3Ds_precomp,
                         raster_settings, pose=None, return_alpha=False, adam_in_backward=None):
-    empty = torch.empty(0, device=means3D.device)
-    return _RasterizeGaussians.apply(
-        means3D, means2D,
-        sh if sh is not None else empty,
-        colors_precomp if colors_precomp is not None else empty,
-        opacities,
-        scales if scales is not None else empty,
-        rotations if rotations is not None else empty,
-        cov3Ds_precomp if cov3Ds_precomp is not None else empty,
-        pose if pose is not None else empty,
-        raster_settings, bool(return_alpha), adam_in_backward)
+    return _RasterizeGaussians.apply(means3D, means2D, sh, colors_precomp, opacities, scales, rotations,
+                                     cov3Ds_precomp, pose, raster_settings, bool(return_alpha), adam_in_backward)
 
 
 class GaussianRasterizer(nn.Module):

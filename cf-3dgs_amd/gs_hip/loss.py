@@ -13,6 +13,9 @@ import math
 import torch
 import torch.nn.functional as F
 
+from . import _lib
+from .raster import _stream
+
 _WINDOWS = {}
 
 
@@ -71,8 +74,6 @@ _TAPS = None
 class _FusedPhotometric(torch.autograd.Function):
     @staticmethod
     def forward(ctx, pred, gt, lambda_dssim, clamp01):
-        import ctypes
-        from . import _lib
         global _TAPS
         if _TAPS is None:
             _TAPS = _window_taps()
@@ -86,11 +87,11 @@ class _FusedPhotometric(torch.autograd.Function):
         C, H, W = x.shape
         ws = torch.empty(lib.gs_loss_workspace_bytes(C, H, W), dtype=torch.uint8, device=x.device)
         out = torch.empty(3, dtype=torch.float32, device=x.device)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-        _lib.check(lib.gs_ssim_l1_forward(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), C, H, W,
+        stream = _stream(x.device)
+        _lib.check(lib.gs_ssim_l1_forward(x.data_ptr(), y.data_ptr(), C, H, W,
                                           _TAPS, float(lambda_dssim), int(bool(clamp01)),
-                                          ctypes.c_void_p(out.data_ptr()),
-                                          ctypes.c_void_p(ws.data_ptr()), ws.numel(), stream), "gs_ssim_l1_forward")
+                                          out.data_ptr(),
+                                          ws.data_ptr(), ws.numel(), stream), "gs_ssim_l1_forward")
         ctx.save_for_backward(x, y, ws)
         ctx.shape = pred.shape
         ctx.lam = float(lambda_dssim)
@@ -101,21 +102,19 @@ class _FusedPhotometric(torch.autograd.Function):
 
     @staticmethod
     def backward(ctx, g_loss, g_out):
-        import ctypes
-        from . import _lib
         lib = _lib.load()
         if g_loss is None:
             return None, None, None, None
         x, y, ws = ctx.saved_tensors
         C, H, W = x.shape
-        go = g_loss.reshape(1).contiguous().float()
+        go = g_loss.float()
         dx = torch.empty_like(x)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-        _lib.check(lib.gs_ssim_l1_backward(ctypes.c_void_p(x.data_ptr()), ctypes.c_void_p(y.data_ptr()), C, H, W,
-                                           _TAPS, ctx.lam, ctx.clamp01, ctypes.c_void_p(go.data_ptr()),
-                                           ctypes.c_void_p(ws.data_ptr()), ws.numel(), ctypes.c_void_p(dx.data_ptr()),
+        stream = _stream(x.device)
+        _lib.check(lib.gs_ssim_l1_backward(x.data_ptr(), y.data_ptr(), C, H, W,
+                                           _TAPS, ctx.lam, ctx.clamp01, go.data_ptr(),
+                                           ws.data_ptr(), ws.numel(), dx.data_ptr(),
                                            stream), "gs_ssim_l1_backward")
-        return dx.view(ctx.shape), None, None, None
+        return (dx if dx.shape == ctx.shape else dx.view(ctx.shape)), None, None, None
 
 
 def fused_photometric_loss(pred: torch.Tensor, gt: torch.Tensor, lambda_dssim: float = 0.2, clamp01: bool = False):
@@ -128,8 +127,6 @@ def fused_photometric_value_and_grad(pred: torch.Tensor, gt: torch.Tensor, lambd
                                      clamp01: bool = False):
     """Forward and backward of the fused loss in one call, outside autograd:
     returns (stats [loss, SSIM, L1] on the device, d loss / d pred)."""
-    import ctypes
-    from . import _lib
     global _TAPS
     if _TAPS is None:
         _TAPS = _window_taps()
@@ -143,8 +140,8 @@ def fused_photometric_value_and_grad(pred: torch.Tensor, gt: torch.Tensor, lambd
     out = torch.empty(3, dtype=torch.float32, device=x.device)
     one = torch.ones(1, dtype=torch.float32, device=x.device)
     dx = torch.empty_like(x)
-    stream = ctypes.c_void_p(torch.cuda.current_stream(x.device).cuda_stream)
-    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    stream = _stream(x.device)
+    p = lambda t: t.data_ptr()  # noqa: E731
     _lib.check(lib.gs_ssim_l1_forward(p(x), p(y), C, H, W, _TAPS, float(lambda_dssim), int(bool(clamp01)), p(out),
                                       p(ws), ws.numel(), stream), "gs_ssim_l1_forward")
     _lib.check(lib.gs_ssim_l1_backward(p(x), p(y), C, H, W, _TAPS, float(lambda_dssim), int(bool(clamp01)), p(one),

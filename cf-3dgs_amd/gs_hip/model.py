@@ -25,6 +25,7 @@ Two layout choices differ from the reference's module, not its arithmetic:
 from __future__ import annotations
 
 import ctypes
+from typing import Optional
 
 import torch
 import torch.nn as nn
@@ -34,10 +35,11 @@ from diff_gaussian_rasterization import GaussianRasterizer
 
 from . import _lib
 from .camera import Camera, raster_settings
+from .raster import _stream
 
 
-def _p(t: torch.Tensor):
-    return ctypes.c_void_p(t.data_ptr()) if t is not None else None
+def _p(t: Optional[torch.Tensor]) -> Optional[int]:
+    return t.data_ptr() if t is not None else None
 
 
 def _aligned(t: torch.Tensor) -> torch.Tensor:
@@ -63,7 +65,7 @@ class _Activate(torch.autograd.Function):
         scales = torch.empty_like(rs)
         rots = torch.empty_like(rr)
         opac = torch.empty_like(ro)
-        stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+        stream = _stream(dev)
         _lib.check(_lib.load().gs_activate_forward(P, _p(rs), _p(rr), _p(ro), _p(scales), _p(rots), _p(opac),
                                                    stream), "gs_activate_forward")
         ctx.set_materialize_grads(False)
@@ -78,7 +80,7 @@ class _Activate(torch.autograd.Function):
         P = rr.shape[0]
         # an output that took no part in the loss passes no gradient on (as in torch)
         need = ctx.needs_input_grad
-        stream = ctypes.c_void_p(torch.cuda.current_stream(rr.device).cuda_stream)
+        stream = _stream(rr.device)
         if ctx.adam is not None and all(need[:3]) and g_s is not None and g_r is not None and g_o is not None:
             # one Adam step of the raw parameters here; they get no gradient
             ad = ctx.adam.take()

@@ -19,6 +19,7 @@ import ctypes
 import torch
 
 from . import _lib
+from .raster import _stream
 
 
 class FusedAdam(torch.optim.Optimizer):
@@ -105,7 +106,7 @@ class FusedAdam(torch.optim.Optimizer):
                 LLR = (ctypes.c_float * n)(*[c[5] for c in chunk])
                 LEAD = (ctypes.c_int * n)(*[c[6] for c in chunk])
                 ROW = (ctypes.c_int * n)(*[c[7] for c in chunk])
-                stream = ctypes.c_void_p(torch.cuda.current_stream(dev).cuda_stream)
+                stream = _stream(dev)
                 _lib.check(lib.gs_adam_step_rows(n, P, G, M, V, N, LR, LLR, LEAD, ROW, b1, b2, eps, step, stream),
                            "gs_adam_step_rows")
         return loss

@@ -42,6 +42,8 @@ def _dev_f32(t: Optional[torch.Tensor], device: torch.device, name: str) -> Opti
         t = torch.as_tensor(t, dtype=torch.float32)
     if t.numel() == 0:
         return None
+    if t.dtype is torch.float32 and t.device == device and t.is_contiguous() and t.data_ptr() % 16 == 0:
+        return t  # nothing to convert
     if t.device.type == "cpu" and device.type == "cuda":
         t = t.to(device)
     if t.device != device:
@@ -54,12 +56,15 @@ def _dev_f32(t: Optional[torch.Tensor], device: torch.device, name: str) -> Opti
     return t
 
 
-def _ptr(t: Optional[torch.Tensor]):
-    return None if t is None else ctypes.c_void_p(t.data_ptr())
+def _ptr(t: Optional[torch.Tensor]) -> Optional[int]:
+    return None if t is None else t.data_ptr()
 
 
-def _stream(device: torch.device) -> ctypes.c_void_p:
-    return ctypes.c_void_p(torch.cuda.current_stream(device).cuda_stream)
+def _stream(device: torch.device) -> int:
+    """The handle of the calling thread's current stream (torch.cuda.current_stream
+    builds a Stream object around it, 4 us of host time a call)."""
+    i = device.index
+    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device() if i is None else i)
 
 
 def require_device(t: torch.Tensor, name: str = "means3D") -> torch.device:
@@ -254,7 +259,8 @@ def forward(settings, means3D, shs, colors_precomp, opacities, scales, rotations
     # does not need the count runs under the last capacity used for this size.
     host, ev = _readback(device)
     host.copy_(counters, non_blocking=True)
-    ev.record(torch.cuda.current_stream(device))
+    sid, idx, kind = torch._C._cuda_getCurrentStream(device.index)
+    ev.record(torch.cuda.Stream(stream_id=sid, device_index=idx, device_type=kind))
     key = (P, W, H, fa.frame.binning)
     guess = _LAST_CAPACITY.get(key, 0)
     binning = None
@@ -265,8 +271,8 @@ def forward(settings, means3D, shs, colors_precomp, opacities, scales, rotations
                                          _ptr(binning), binning.numel(), _ptr(image), image.numel(), stream),
                    "gs_render_prepare")
     ev.synchronize()
-    num_rendered = int(host[0]) & 0xFFFFFFFF
-    status = int(host[1])
+    num_rendered, status = host.tolist()[:2]
+    num_rendered &= 0xFFFFFFFF
     if status & _lib.GS_STATUS_PREFILTERED:
         raise RuntimeError("a point was culled by the near plane although prefiltered=True")
     # capacity rounded up so the caching allocator can reuse the binning block
