@@ -480,12 +480,17 @@ struct DfDupArgs {
   const uint32_t* tiles;
   const uint32_t* dvals;
   const uint32_t* dscan;
-  const uint32_t* dblocks;
+  const uint32_t* dblocks;  // block totals (up to kOwnPrefix blocks), else their prefix and the largest total
   uint32_t* counters;
   uint32_t* keys;  // tile ids, or tile << id_bits | id when id_bits > 0
   uint32_t* vals;  // ids (unused when id_bits > 0)
   int id_bits;
 };
+
+// Up to this many blocks of 256 Gaussians every workgroup of the duplicate forms
+// the prefix of their totals itself (1024 words from L2, four a thread), which
+// is as quick as the wait for a launch that does, and spares that launch.
+constexpr uint32_t kOwnPrefix = 1024;
 
 // Tile ids in depth order (sorted position k -> Gaussian dvals[k]).  Each
 // Gaussian's entries form one run at its prefix offset, its rect row by row.
@@ -502,6 +507,7 @@ struct DfDupArgs {
 // (31 us with it for 16 pose frames, 22 without).
 __device__ __forceinline__ void df_duplicate_block(const DfDupArgs& a, uint32_t bid, uint32_t nblocks) {
   __shared__ uint32_t s_start[256], s_g[256], s_xy[256], s_w[256], s_k0, s_end;
+  __shared__ uint32_t s_pref[kOwnPrefix], s_w4[4], s_most[4];
   const uint32_t t = threadIdx.x;
   const uint32_t n = a.counters[0];
   if ((long long)n > a.capacity) {
@@ -513,13 +519,38 @@ __device__ __forceinline__ void df_duplicate_block(const DfDupArgs& a, uint32_t 
   }
   const uint32_t P = (uint32_t)a.P, chunk = (n / min(nblocks, 2048u) / 1024u + 1u) * 1024u;
   const uint32_t nruns = (P + 255u) / 256u;
-  const bool even = a.dblocks[nruns] <= 4096u;
+  const bool own = nruns <= kOwnPrefix;
+  uint32_t biggest;
+  if (own) {
+    uint32_t v[4], sum = 0, most = 0;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+      v[q] = 4u * t + q < nruns ? a.dblocks[4u * t + q] : 0u;
+      sum += v[q];
+      most = max(most, v[q]);
+    }
+    most = wave_max_u32(most);
+    if ((t & 63u) == 0) s_most[t >> 6] = most;
+    uint32_t total;
+    uint32_t run = block_incl_scan_256(sum, s_w4, total) - sum;
+#pragma unroll
+    for (uint32_t q = 0; q < 4; ++q) {
+      s_pref[4u * t + q] = run;
+      run += v[q];
+    }
+    __syncthreads();
+    biggest = max(max(s_most[0], s_most[1]), max(s_most[2], s_most[3]));
+  } else {
+    biggest = a.dblocks[nruns];
+  }
+  auto before = [&](uint32_t b) { return own ? s_pref[b] : a.dblocks[b]; };  // entries of the blocks before b
+  const bool even = biggest <= 4096u;
   const uint32_t nchunks = even ? nruns : n / chunk + (n % chunk != 0 ? 1u : 0u);
   for (uint32_t c = bid; c < nchunks; c += nblocks) {
     uint32_t o0 = c * chunk, o1 = o0 + min(chunk, n - o0);
     if (even) {
-      o0 = a.dblocks[c];
-      o1 = c + 1u < nruns ? a.dblocks[c + 1u] : n;
+      o0 = before(c);
+      o1 = c + 1u < nruns ? before(c + 1u) : n;
       if (t == 0) s_k0 = 256u * c;
     } else if (t < 64) {
       // the last 256-run block that starts at or before o0, then its runs that
@@ -527,11 +558,11 @@ __device__ __forceinline__ void df_duplicate_block(const DfDupArgs& a, uint32_t 
       uint32_t lo = 0, len = nruns;
       while (len > 1) {
         const uint32_t step = (len + 63u) / 64u, k = t * step;
-        const uint32_t m = (uint32_t)__popcll(__ballot(k < len && a.dblocks[lo + min(k, len - 1u)] <= o0)) - 1u;
+        const uint32_t m = (uint32_t)__popcll(__ballot(k < len && before(lo + min(k, len - 1u)) <= o0)) - 1u;
         lo += m * step;
         len = min(step, len - m * step);
       }
-      const uint32_t b0 = a.dblocks[lo];
+      const uint32_t b0 = before(lo);
       uint32_t k0 = lo * 256u;
 #pragma unroll
       for (uint32_t q = 0; q < 4; ++q) {
@@ -547,7 +578,7 @@ __device__ __forceinline__ void df_duplicate_block(const DfDupArgs& a, uint32_t 
       uint32_t start = n, end = n, g = 0, xy = 0, w = 1;
       if (k < P) {
         g = a.dvals[k];
-        end = a.dblocks[k >> 8] + a.dscan[k];
+        end = before(k >> 8) + a.dscan[k];
         start = end - a.tiles[g];
         if (start < end) {
           const uint2 r = a.rect[g];
@@ -638,7 +669,7 @@ __global__ __launch_bounds__(256) void k_df_scan_multi(const uint32_t* prefix, c
 // Workgroup f: the exclusive prefix of frame f's block totals.
 __global__ __launch_bounds__(256) void k_excl_scan_multi(const DfMid* mid) {
   const DfMid m = mid[blockIdx.x];
-  excl_scan_block<256>(m.dblocks, m.nblocks);
+  if (m.nblocks > (int)kOwnPrefix) excl_scan_block<256>(m.dblocks, m.nblocks);
 }
 
 // Many frames' duplicates, on the same workgroup ranges as k_df_scan_multi (a
@@ -1354,7 +1385,8 @@ static int render_binning(const gs_frame_t* f, int P, const void* geom, uint32_t
       timing::Scope ts(timing::kDuplicate, s);
       hipLaunchKernelGGL(k_df_scan, dim3(nbp), dim3(256), 0, s, P, dvals, tiles, (uint32_t*)(bb + LB.dscan),
                          (uint32_t*)(bb + LB.dblocks));
-      hipLaunchKernelGGL(k_excl_scan_1wg, dim3(1), dim3(1024), 0, s, (uint32_t*)(bb + LB.dblocks), nbp);
+      if (nbp > (int)kOwnPrefix)
+        hipLaunchKernelGGL(k_excl_scan_1wg, dim3(1), dim3(1024), 0, s, (uint32_t*)(bb + LB.dblocks), nbp);
     }
     if (do_dup) {
       timing::Scope ts(timing::kDuplicate, s);
@@ -1627,6 +1659,9 @@ extern "C" int gs_multi_preprocess_keys(int n, const void* dev_set, const unsign
 // ---- many frames' binning steps around the list sort ----------------------
 // Set layout: uint32 prefix[n + 1] of per-Gaussian workgroup bounds per frame,
 // then DfMid[n] and CkptScan[n], each array at a 256-byte boundary.
+// beside the workgroup count the build returns: some frame needs the launch
+// that forms the block prefixes
+constexpr unsigned kMidPrefixes = 1u << 31;
 static size_t mbm_mid_offset(int n) { return align_up(sizeof(uint32_t) * (size_t)(n + 1), 256); }
 static size_t mbm_ckpt_offset(int n) { return mbm_mid_offset(n) + align_up(sizeof(DfMid) * (size_t)n, 256); }
 
@@ -1647,6 +1682,7 @@ extern "C" int gs_multi_binning_steps_build(int n, const gs_frame_t* frames, con
   DfMid* mid = (DfMid*)((char*)host_set + mbm_mid_offset(n));
   CkptScan* ck = (CkptScan*)((char*)host_set + mbm_ckpt_offset(n));
   unsigned long long total = 0;
+  bool prefixes = false;
   for (int i = 0; i < n; ++i) {
     const gs_frame_t* f = &frames[i];
     // the depth-first schedule's split phases, as gs_render_binning_duplicate
@@ -1665,6 +1701,7 @@ extern "C" int gs_multi_binning_steps_build(int n, const gs_frame_t* frames, con
     const int nt = grid_tiles(f->width, f->height, gx, gy);
     if (gx > 0xffff || gy > 0xffff) return GS_E_ARG;  // tile rects are packed in 16-bit fields
     const int nbp = nblocks256(P[i]);
+    prefixes |= nbp > (int)kOwnPrefix;
     prefix[i] = (uint32_t)total;
     total += (unsigned long long)nbp;
     if (total > 0x7fffffffULL) return GS_E_ARG;
@@ -1699,18 +1736,20 @@ extern "C" int gs_multi_binning_steps_build(int n, const gs_frame_t* frames, con
     ck[i].nt = nt;
   }
   prefix[n] = (uint32_t)total;
-  *total_blocks = (unsigned)total;
+  *total_blocks = (unsigned)total | (prefixes ? kMidPrefixes : 0u);
   return GS_OK;
 }
 
 extern "C" int gs_multi_binning_duplicate(int n, const void* dev_set, unsigned total_blocks, void* stream) {
   if (n <= 0 || !dev_set) return GS_E_ARG;
+  const bool prefixes = total_blocks & kMidPrefixes;
+  total_blocks &= ~kMidPrefixes;
   hipStream_t s = (hipStream_t)stream;
   const uint32_t* prefix = (const uint32_t*)dev_set;
   const DfMid* mid = (const DfMid*)((const char*)dev_set + mbm_mid_offset(n));
   timing::Scope ts(timing::kDuplicate, s);
   if (total_blocks > 0) hipLaunchKernelGGL(k_df_scan_multi, dim3(total_blocks), dim3(256), 0, s, prefix, mid, n);
-  hipLaunchKernelGGL(k_excl_scan_multi, dim3(n), dim3(256), 0, s, mid);
+  if (prefixes) hipLaunchKernelGGL(k_excl_scan_multi, dim3(n), dim3(256), 0, s, mid);
   if (total_blocks > 0)
     hipLaunchKernelGGL(k_df_duplicate_multi, dim3(total_blocks), dim3(256), 0, s, prefix, mid, n);
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;

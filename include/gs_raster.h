@@ -326,7 +326,7 @@ int gs_render_after_depth_sort(const gs_frame_t* frame, int P, const void* geom,
  * gs_render_binning does; frames with one-word list entries only, capacity
  * up to 2^21), then per frame gs_render_binning_after_list_sort (checkpoint
  * scan) or gs_render_after_list_sort (the same and the blend).  blocks[4]
- * holds the grid of each pass (0 past the last). */
+ * is what the build returned (each pass's grid and variant, 0 past the last). */
 int gs_render_binning_duplicate(const gs_frame_t* frame, int P, const void* geom, uint32_t* counters,
                                 long long capacity, void* binning, size_t binning_bytes, void* image,
                                 size_t image_bytes, void* stream);
@@ -337,13 +337,13 @@ int gs_multi_list_sort_build(int n, const gs_frame_t* frames, const int* P, cons
 int gs_multi_list_sort(int n, const void* dev_set, const unsigned* blocks, void* stream);
 /* The depth-first binning's steps on either side of the list sort for many
  * frames: gs_multi_binning_duplicate is gs_render_binning_duplicate of every
- * frame (three launches: the workgroup-local scans of the tile counts in
- * depth order, one workgroup per frame for the block prefix, the
- * duplicates); gs_multi_binning_after_list_sort is
+ * frame (two launches: the workgroup-local scans of the tile counts in depth
+ * order and the duplicates; between them, if a frame has more than 262144
+ * Gaussians, one workgroup per frame for the block prefix); gs_multi_binning_after_list_sort is
  * gs_render_binning_after_list_sort of every frame (one launch, a workgroup
  * per frame).  The results are those of the per-frame calls, bit for bit.
  * The build takes those calls' per-frame arguments as arrays and checks them
- * as they do; total_blocks is returned by the build.  Replaces, for many
+ * as they do; total_blocks is what the build returned.  Replaces, for many
  * frames at once, the duplicate and the tile-range step of forward phase 2
  * above. */
 size_t gs_multi_binning_steps_bytes(int n);

@@ -84,3 +84,23 @@ def test_runs_split_by_entry(n):
     for k in ("color", "depth", "alpha"):
         np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
     np.testing.assert_array_equal(np_(g["views"]["n_contrib"]), o["n_contrib"])
+
+
+@pytest.mark.parametrize("big", [0, 40], ids=["even", "uneven"])
+@pytest.mark.parametrize("n", [1024 * 256, 1024 * 256 + 1])
+def test_block_prefix(n, big):
+    """1024 blocks of 256 Gaussians, whose prefix the duplicate forms itself, and
+    1025, which have a launch for it; by Gaussian, and by entry (40 Gaussians
+    that cover all 130 tiles)."""
+    print("block prefix", n, big, flush=True)
+    sc = scenes.plain_scene(seed=9, P=n, W=200, H=150)
+    sc["scales"] *= 0.05
+    sc["scales"][:big] = 3.0
+    sc["means"][:big] = torch.tensor([0.0, 0.0, 3.0])
+    sc["opacities"] *= 0.05
+    g = run_gpu(sc, 1)
+    _, _, o = run_oracle(sc, 1)
+    assert g["st"].num_rendered == o["num_rendered"]
+    for k in ("color", "depth", "alpha"):
+        np.testing.assert_array_equal(np_(g[k]), o[k], err_msg=k)
+    np.testing.assert_array_equal(np_(g["views"]["n_contrib"]), o["n_contrib"])
