@@ -165,13 +165,31 @@ __device__ __forceinline__ void upsweep_block(const K* __restrict__ keys, const 
       }
       if ((uint32_t)lane <= mask) s_h[w][lane] = cnt;
     } else {
+      // digits of 7, 6 or 5 bits leave room for 2, 4 or 8 counters of each: lanes
+      // side by side add to different ones, in different banks (their adds to
+      // one word follow each other: 11.4 us an upsweep of the 500 000-Gaussian
+      // training scene's lists, 7.4 this way; 85 and 75 for 71M entries)
+      const int room = R == 256 ? 8 - bits : 0;
+      const uint32_t copy = (uint32_t)lane & ((1u << room) - 1u), at = copy << bits, skew = copy * (mask + 1u) >> room;
 #pragma unroll
       for (int r = 0; r < V; ++r) {
         const uint32_t idx = wbase + 4u * (uint32_t)(r * 64 + lane);
         const uint32_t e[4] = {kv[r].x, kv[r].y, kv[r].z, kv[r].w};
 #pragma unroll
         for (int c = 0; c < 4; ++c)
-          if (idx + (uint32_t)c < n) atomicAdd(&s_h[w][(e[c] >> shift) & mask], 1u);
+          if (idx + (uint32_t)c < n) atomicAdd(&s_h[w][at | (((e[c] >> shift) & mask) ^ skew)], 1u);
+      }
+      if (room > 0) {
+        __syncthreads();
+        uint32_t sum = 0;
+        const int d = threadIdx.x;
+        if (d <= (int)mask)
+          for (uint32_t q = 0; q < 1u << room; ++q) {
+            const uint32_t k = q << bits | ((uint32_t)d ^ (q * (mask + 1u) >> room));
+            sum += s_h[0][k] + s_h[1][k] + s_h[2][k] + s_h[3][k];
+          }
+        if (d <= (int)mask || direct) hist[direct ? (size_t)blk * R + d : (size_t)d * nb_max + blk] = sum;
+        return;
       }
     }
   } else {
