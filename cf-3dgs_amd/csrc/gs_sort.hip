@@ -349,8 +349,9 @@ __device__ __forceinline__ void scatter_block(const K* __restrict__ keys_in, con
     if (!added) {
 #pragma unroll
       for (int i = 0; i < DP; ++i) {
-        total[i] = totals[t * DP + i];
-        before[i] = hist[(size_t)(t * DP + i) * nb_max + blk];
+        const uint32_t d = (uint32_t)(t * DP + i);
+        total[i] = d <= mask ? totals[d] : 0u;
+        before[i] = d <= mask ? hist[(size_t)d * nb_max + blk] : 0u;  // (a cache line of its own each)
       }
     }
 #pragma unroll
