@@ -5,8 +5,7 @@
 //                    largest contributor count, longest first, from the
 //                    forward's item log); the others clear the per-Gaussian
 //                    render-gradient accumulators (a kernel, not a memset, so
-//                    the sequence can be captured in a graph), or, in
-//                    deterministic mode, write each tile's last entry
+//                    the sequence can be captured in a graph)
 //   k_render_bwd     one chunk per workgroup (16x16 pixels), back to front.
 //                    A chunk that is not the tile's last starts from the
 //                    forward's checkpoint at its end: T_b, and the sum of what
@@ -31,7 +30,6 @@
 //   k_pose_finalize  sums the wave partials in a fixed tree order, then
 //                    d/dR, d/dt -> d/d(q, t) through the quaternion
 //                    normalisation.
-#include <algorithm>
 #include <cmath>
 
 #include "gs_common.hpp"
@@ -69,7 +67,6 @@ struct RBArgs {
   const uint32_t* local_incl;  // [P] tiles prefix within each 256-Gaussian block
   const uint32_t* block_excl;  // [ceil(P/256)] exclusive block prefix
   float* part;                 // [capacity][10] partial per (Gaussian, tile) pair
-  unsigned long long* tile_last;  // [nt] depth bits << 32 | id of the last entry visited (k_bwd_prepare)
 };
 
 // One workgroup orders the backward's work items.  A tile's items are its
@@ -114,15 +111,11 @@ __device__ __forceinline__ void bwd_items(const uint32_t* item_log, const uint32
 
 // The backward's set-up in one launch: workgroup 0 builds the work-item table
 // (bwd_items; none when items is null), the others clear the zn accumulator
-// floats at zp or, with tile_last (deterministic mode), write the entry each
-// of the nt tiles' render backward ends at.
-//
-// Pairs past a tile's last contributor get no partial.  The gathers know them
-// by tile_last: lists are in (depth bits, id) order, so a Gaussian's pair with a
-// tile was visited if its (depth, id) is not past the tile's.  Clearing every
-// pair's partial instead took 115 us a launch of 16 pose frames beside the other
-// stream (now 13; a solve of them 20.4 -> 20.2 ms: the backward next to it gets
-// the bandwidth).
+// floats at zp.
+// The set-up of one frame: zn floats at zp to clear, or, when terms > 0
+// (the deterministic mode's pair partials), only the first num_rendered *
+// terms of them (counters[0] = num_rendered; no pair slot at or past it is
+// written or read).
 struct BwdPrep {
   float* zp;
   long long zn;
@@ -130,11 +123,8 @@ struct BwdPrep {
   const uint32_t* ranges;
   const uint32_t* tile_maxc;
   uint32_t* items;
-  const uint32_t* list;
-  uint32_t id_mask;
-  const float4* splat;
-  unsigned long long* tile_last;
-  int nt;
+  const uint32_t* counters;
+  int terms;
 };
 
 // Workgroup bid of a set-up over nblocks workgroups.
@@ -144,38 +134,10 @@ __device__ __forceinline__ void bwd_prepare_block(const BwdPrep& p, int bid, int
     bwd_items(p.item_log, p.ranges, p.tile_maxc, p.items);
     return;
   }
+  long long zn = p.zn;
+  if (p.terms > 0) zn = min(zn, (long long)p.counters[0] * p.terms);
   const long long nb = (long long)nblocks - first;
-  const long long k0 = ((long long)bid - first) * 1024 + threadIdx.x;
-  for (long long k = k0; k < p.zn; k += nb * 1024) p.zp[k] = 0.0f;
-  if (!p.tile_last) return;
-  for (long long k = k0; k < p.nt; k += nb * 1024) {
-    const uint32_t maxc = p.tile_maxc[k];
-    unsigned long long last = 0;  // (no depth is zero)
-    if (maxc > 0) {
-      const uint32_t id = p.list[p.ranges[2 * k] + maxc - 1u] & p.id_mask;
-      last = (unsigned long long)__float_as_uint(p.splat[3 * (size_t)id + 1].z) << 32 | id;
-    }
-    p.tile_last[k] = last;
-  }
-}
-
-// The sums of Gaussian i's NT-term partials, in the order of its tiles (rows of
-// its rect), over the pairs that were visited; off: its first pair's slot.
-template <int NT>
-__device__ __forceinline__ void gather_pairs(uint32_t i, uint32_t off, const float4* splat, int gx, int gy,
-                                             const unsigned long long* tile_last, const float* part,
-                                             float (&acc)[NT]) {
-  const float4 s0 = splat[3 * (size_t)i], s1 = splat[3 * (size_t)i + 1], s2 = splat[3 * (size_t)i + 2];
-  const unsigned long long mine = (unsigned long long)__float_as_uint(s1.z) << 32 | i;
-  int x0, y0, x1, y1;
-  tile_rect(s0.x, s0.y, __float_as_int(s2.w), gx, gy, x0, y0, x1, y1);
-  const float* src = part + (size_t)off * NT;
-  for (int y = y0; y < y1; ++y)
-    for (int x = x0; x < x1; ++x, src += NT) {
-      if (mine > tile_last[y * gx + x]) continue;
-#pragma unroll
-      for (int k = 0; k < NT; ++k) acc[k] += src[k];
-    }
+  for (long long k = ((long long)bid - first) * 1024 + threadIdx.x; k < zn; k += nb * 1024) p.zp[k] = 0.0f;
 }
 
 __global__ __launch_bounds__(1024) void k_bwd_prepare(BwdPrep p) { bwd_prepare_block(p, blockIdx.x, gridDim.x); }
@@ -600,21 +562,27 @@ __global__ __launch_bounds__(256) void k_render_bwd_multi(const uint32_t* prefix
 }
 
 // Deterministic mode: per Gaussian, the partials of its (Gaussian, tile)
-// pairs summed in rect order into its render-gradient record.  Nothing is
-// read when the frame overflowed the binning capacity (no pairs were made).
+// pairs (NT terms each) summed in rect order into its render-gradient
+// record.  Nothing is read when the frame
+// overflowed the binning capacity (no pairs were made).
+template <int NT>
 __global__ __launch_bounds__(256) void k_det_gather(int P, const uint32_t* tiles, const uint32_t* local_incl,
                                                     const uint32_t* block_excl, const uint32_t* counters,
-                                                    long long capacity, const float4* splat, int gx, int gy,
-                                                    const unsigned long long* tile_last, const float* part,
-                                                    float* g_render) {
+                                                    long long capacity, const float* part, float* g_render) {
   const int g = blockIdx.x * 256 + threadIdx.x;
   if (g >= P) return;
   float acc[10];
 #pragma unroll
   for (int k = 0; k < 10; ++k) acc[k] = 0.f;
   const uint32_t nt = tiles[g];
-  if ((long long)counters[0] <= capacity && nt > 0)
-    gather_pairs<10>((uint32_t)g, block_excl[g >> 8] + local_incl[g] - nt, splat, gx, gy, tile_last, part, acc);
+  if ((long long)counters[0] <= capacity && nt > 0) {
+    const uint32_t off = block_excl[g >> 8] + local_incl[g] - nt;
+    for (uint32_t e = off; e < off + nt; ++e) {
+      const float* src = part + (size_t)e * NT;
+#pragma unroll
+      for (int k = 0; k < NT; ++k) acc[k] += src[k];
+    }
+  }
   float4* dst = reinterpret_cast<float4*>(g_render + (size_t)g * kRG);
   dst[0] = make_float4(acc[0], acc[1], acc[2], acc[3]);
   dst[1] = make_float4(acc[4], acc[5], acc[6], acc[7]);
@@ -655,8 +623,6 @@ struct PBArgs {
   const uint32_t* block_excl;
   const uint32_t* counters;
   long long capacity;
-  const unsigned long long* tile_last;
-  int gx, gy;
   // gs_backward_adam: one Adam step of the means and SH coefficients instead
   // of writing their gradients (adam_on == 0 otherwise)
   int adam_on;
@@ -804,12 +770,17 @@ __device__ __forceinline__ void preprocess_bwd_block(const PBArgs& a, int bid, f
     const bool vis = a.radii[i] > 0;
     float4 rA, rB, rC;  // the render-gradient record, then m2x m2y ca cb | cc opac r g | b depth - -
     if (a.part5) {
-      // the sums k_det_gather forms, in its order (terms 5..9 are zero)
+      // the sums k_det_gather<5> forms, in its order (terms 5..9 are zero)
       float acc[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
       const uint32_t nt = a.g_tiles[i];
-      if ((long long)a.counters[0] <= a.capacity && nt > 0)
-        gather_pairs<5>((uint32_t)i, a.block_excl[i >> 8] + a.local_incl[i] - nt, a.splat, a.gx, a.gy, a.tile_last,
-                        a.part5, acc);
+      if ((long long)a.counters[0] <= a.capacity && nt > 0) {
+        const uint32_t off = a.block_excl[i >> 8] + a.local_incl[i] - nt;
+        for (uint32_t e = off; e < off + nt; ++e) {
+          const float* src = a.part5 + (size_t)e * 5;
+#pragma unroll
+          for (int k = 0; k < 5; ++k) acc[k] += src[k];
+        }
+      }
       rA = make_float4(acc[0], acc[1], acc[2], acc[3]);
       rB = make_float4(acc[4], 0.f, 0.f, 0.f);
       rC = make_float4(0.f, 0.f, 0.f, 0.f);
@@ -1267,7 +1238,6 @@ static RBArgs make_rb_args(const gs_frame_t* f, int P, const void* geom, long lo
   r.local_incl = (const uint32_t*)(gb + LG.offsets);
   r.block_excl = (const uint32_t*)(gb + LG.scan_tmp);
   r.part = part;
-  r.tile_last = capacity > 0 ? (unsigned long long*)(bb + LB.items + items_bytes(capacity, r.nt)) : nullptr;
   return r;
 }
 
@@ -1314,30 +1284,30 @@ static int bwd_check(const gs_frame_t* f, const gs_gaussians_t* g, const int* ra
 
 // Phase 1: clear the accumulators and build the work-item table.
 // One frame's set-up and the workgroups it takes (0: nothing to do).
-static BwdPrep bwd_prep_of(const gs_frame_t* f, int P, long long capacity, const RBArgs& r, unsigned* grid) {
+static BwdPrep bwd_prep_of(const gs_frame_t* f, int P, long long capacity, const uint32_t* counters,
+                           const RBArgs& r, bool po, unsigned* grid) {
   BwdPrep p;
-  // (deterministic mode writes every record in k_det_gather)
-  p.zp = r.g_render;
-  p.zn = f->deterministic ? 0 : (long long)P * kRG;
+  // deterministic mode writes every record in k_det_gather; pairs past a
+  // tile's last contributor are never visited, so their partials start at 0
+  p.zp = f->deterministic ? r.part : r.g_render;
+  p.zn = f->deterministic ? capacity * (po ? 5 : 10) : (long long)P * kRG;
+  p.counters = counters;
+  p.terms = f->deterministic ? (po ? 5 : 10) : 0;
   // the work-item table, from the forward's item log (both live in the
   // binning workspace)
   p.item_log = r.item_log;
   p.items = capacity > 0 && P > 0 ? (uint32_t*)r.items : nullptr;
   p.ranges = r.ranges;
   p.tile_maxc = r.tile_maxc;
-  p.list = r.list;
-  p.id_mask = r.id_mask;
-  p.splat = r.splat;
-  p.tile_last = f->deterministic && p.items ? r.tile_last : nullptr;
-  p.nt = r.nt;
-  const long long nzb = (std::max(p.zn, p.tile_last ? (long long)p.nt : 0LL) + 1023) / 1024;
+  const long long nzb = (p.zn + 1023) / 1024;
   *grid = (unsigned)((nzb < 2048 ? nzb : 2048) + (p.items ? 1 : 0));
   return p;
 }
 
-static void bwd_prepare(const gs_frame_t* f, int P, long long capacity, const RBArgs& r, hipStream_t s) {
+static void bwd_prepare(const gs_frame_t* f, int P, long long capacity, const uint32_t* counters, const RBArgs& r,
+                        hipStream_t s, bool po) {
   unsigned grid = 0;
-  const BwdPrep p = bwd_prep_of(f, P, capacity, r, &grid);
+  const BwdPrep p = bwd_prep_of(f, P, capacity, counters, r, po, &grid);
   if (grid > 0) hipLaunchKernelGGL(k_bwd_prepare, dim3(grid), dim3(1024), 0, s, p);
 }
 
@@ -1416,9 +1386,6 @@ static PBArgs make_pb_args(const gs_frame_t* f, const gs_gaussians_t* g, const i
   b.block_excl = (const uint32_t*)(gb + LG.scan_tmp);
   b.counters = counters;
   b.capacity = capacity;
-  b.tile_last = r.tile_last;
-  b.gx = r.gx;
-  b.gy = r.gy;
   b.adam_on = ad ? 1 : 0;
   b.means_p = ad ? ad->means_p : nullptr;
   b.means_m = ad ? ad->in->means_m : nullptr;
@@ -1447,9 +1414,9 @@ static void bwd_finish(const gs_frame_t* f, const gs_gaussians_t* g, const int* 
   float* pose_part = (float*)((char*)r.g_render + align_up((size_t)P * kRG * sizeof(float), 256));
   // (the pose-only backward gathers its 5-term partials inside k_preprocess_bwd)
   if (f->deterministic && P > 0 && !po)
-    hipLaunchKernelGGL(k_det_gather, dim3((P + 255) / 256), dim3(256), 0, s, P,
+    hipLaunchKernelGGL(k_det_gather<10>, dim3((P + 255) / 256), dim3(256), 0, s, P,
                        (const uint32_t*)(gb + LG.tiles), (const uint32_t*)(gb + LG.offsets),
-                       (const uint32_t*)(gb + LG.scan_tmp), counters, capacity, r.splat, r.gx, r.gy, r.tile_last, (const float*)r.part, r.g_render);
+                       (const uint32_t*)(gb + LG.scan_tmp), counters, capacity, (const float*)r.part, r.g_render);
   if (P > 0) {
     const PBArgs b = make_pb_args(f, g, radii, geom, capacity, counters, out, r, po, ad);
     timing::Scope ts(timing::kPreprocessBwd, s);
@@ -1479,7 +1446,7 @@ extern "C" int gs_backward(GS_BWD_ARGS) {
   hipStream_t s = (hipStream_t)stream;
   const RBArgs r = make_rb_args(f, g->P, geom, capacity, binning, image, dL_dcolor, dL_ddepth, dL_dalpha, scratch);
   const bool po = pose_only(f, g, out, dL_ddepth || dL_dalpha);
-  bwd_prepare(f, g->P, capacity, r, s);
+  bwd_prepare(f, g->P, capacity, counters, r, s, po);
   bwd_render(f, g->P, capacity, r, s, po);
   bwd_finish(f, g, radii, geom, capacity, counters, out, r, s, po);
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
@@ -1516,7 +1483,7 @@ extern "C" int gs_backward_adam(const gs_frame_t* f, const gs_gaussians_t* g, co
   ad.inv_sqrt_bc2 = (float)(1.0 / std::sqrt(bc2));
   hipStream_t s = (hipStream_t)stream;
   const RBArgs r = make_rb_args(f, P, geom, capacity, binning, image, dL_dcolor, dL_ddepth, dL_dalpha, scratch);
-  bwd_prepare(f, P, capacity, r, s);
+  bwd_prepare(f, P, capacity, counters, r, s, false);
   bwd_render(f, P, capacity, r, s, false);
   bwd_finish(f, g, radii, geom, capacity, counters, out, r, s, false, &ad);
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
@@ -1527,7 +1494,7 @@ extern "C" int gs_backward_prepare(GS_BWD_ARGS) {
                            scratch_bytes);
   if (rc != GS_OK) return rc;
   const RBArgs r = make_rb_args(f, g->P, geom, capacity, binning, image, dL_dcolor, dL_ddepth, dL_dalpha, scratch);
-  bwd_prepare(f, g->P, capacity, r, (hipStream_t)stream);
+  bwd_prepare(f, g->P, capacity, counters, r, (hipStream_t)stream, pose_only(f, g, out, dL_ddepth || dL_dalpha));
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
 }
 
@@ -1644,7 +1611,7 @@ extern "C" int gs_multi_pose_bwd_build(int n, const gs_frame_t* frames, const gs
     const RBArgs r = make_rb_args(f, P, geom[i], capacity[i], binning[i], image[i], dL_dcolor[i], nullptr, nullptr,
                                   scratch[i]);
     unsigned pgrid = 0;
-    prep[i] = bwd_prep_of(f, P, capacity[i], r, &pgrid);
+    prep[i] = bwd_prep_of(f, P, capacity[i], counters[i], r, true, &pgrid);
     pprefix[i] = (uint32_t)ptotal;
     ptotal += pgrid;
     prefix[i] = (uint32_t)total;

@@ -1191,8 +1191,7 @@ extern "C" int gs_binning_layout(long long capacity, int P, int width, int heigh
   out->bweight = o;
   o = align_up(o + 4 * (c / 256 + 2 * (size_t)nt + 2), 256);
   out->items = o;
-  // (and, behind them, the deterministic backward's last entry of every tile)
-  o = align_up(o + items_bytes(capacity, nt) + 8 * (size_t)nt, 256);
+  o = align_up(o + 16 * (1 + (c / 256 + (size_t)nt + 1)), 256);
   out->item_log = o;
   o = align_up(o + 4 * (1 + 2 * (c / 256 + (size_t)nt + 1)), 256);
   out->total = o;

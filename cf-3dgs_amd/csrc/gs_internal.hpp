@@ -30,11 +30,6 @@ constexpr bool wide_digit(int bits, long long capacity) {
   return bits > kRadixBits && bits <= kWideBits && capacity <= (1LL << 21);
 }
 
-// The backward's work-item table of a binning workspace: 16-byte records.
-constexpr size_t items_bytes(long long capacity, int n_tiles) {
-  return 16 * (1 + ((size_t)(capacity > 1 ? capacity : 1) / 256 + (size_t)n_tiles + 1));
-}
-
 namespace timing {
 enum Stage { kPreprocess = 0, kScan, kDuplicate, kSort, kRanges, kBlend, kRenderBwd, kPreprocessBwd, kKnn, kZero };
 // RAII pair of events around the launches issued inside the scope (no-op

@@ -137,8 +137,7 @@ typedef struct gs_binning_layout {
                                   that chunk's cost */
   size_t items;                /* uint32[4 (1 + capacity/256 + n_tiles + 1)] backward work items: count,
                                   then from word 4 (tile, chunk, list start, last contributor),
-                                  longest estimated first; behind them uint64[n_tiles] (deterministic
-                                  backward) depth bits << 32 | id of each tile's last entry */
+                                  longest estimated first */
   size_t item_log;             /* uint32[1 + 2 (capacity/256 + n_tiles + 1)] the blend's record of the
                                   work items, in completion order: count, then
                                   (tile, chunk << 6 | cost class) */
