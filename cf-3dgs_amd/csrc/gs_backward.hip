@@ -8,18 +8,24 @@
 //                    the sequence can be captured in a graph)
 //   k_render_bwd     one chunk per workgroup (16x16 pixels), back to front.
 //                    A chunk that is not the tile's last starts from the
-//                    forward's checkpoint at its end: T_b, and the sum of what
-//                    lies behind it, C_final - C_b, so heavy tiles spread over
-//                    many workgroups instead of serialising in one.  Within
-//                    the chunk 16 entries x 4 pixels go through a wave at a
-//                    time, T and the sum behind each entry by scans over the
-//                    entries (render_bwd_item).  The sums of the Gaussian's 10
-//                    terms over the pixels go to LDS, one set per wave, and
-//                    leave as one global atomic per term.
-//                    Deterministic mode: the chunk writes one 10-float partial
-//                    per (Gaussian, tile) pair into a slot of its own (the
-//                    Gaussian's offset in the Gaussian-order tile prefix + the
-//                    tile's rank in its rect) -- no atomics;
+//                    forward's checkpoint at its end: T_b, and the suffix sums
+//                    (C_final - C_b) / T_b that the back-to-front recurrence
+//                    would have accumulated, so heavy tiles spread over many
+//                    workgroups instead of serialising in one.  T is then
+//                    recovered by division as in the forward's algebra.  The
+//                    10 per-(pixel, Gaussian) terms are summed over the
+//                    wave with permlane swaps + DPP (wave_sum12), the wave
+//                    sums go to LDS accumulators, and each Gaussian of the
+//                    chunk receives one global atomic per term.
+//                    k_render_bwd_cells does the same for the fixed-order
+//                    colour backward of a frame with a pose, 16 entries x 4
+//                    pixels of a 4x4-pixel cell at a time, T and the sum
+//                    behind each entry by scans over the entries.
+//                    Deterministic mode: each wave keeps its own LDS
+//                    partials (summed in wave order), and the chunk writes one
+//                    10-float partial per (Gaussian, tile) pair into a slot
+//                    of its own (the Gaussian's offset in the Gaussian-order
+//                    tile prefix + the tile's rank in its rect) -- no atomics;
 //   k_det_gather     deterministic mode: per Gaussian, its partials summed in
 //                    rect order (the pose-only backward sums its 5-term
 //                    partials the same way inside k_preprocess_bwd);
@@ -37,28 +43,35 @@
 
 namespace gs {
 
-// render-gradient record, sums over the pixels a Gaussian blends into, with
-// g = G dL/dalpha, (dx, dy) = centre - pixel and t = dy + s dx (conic_shear):
-//   g dx, g t, g dx^2, g dx t, g t^2, g, w dL/dr, w dL/dg, w dL/db,
-//   w dL/ddepth, -, -
-// (k_preprocess_bwd applies the opacity and the conic to the sums)
+// render-gradient record: m2x m2y xx xt tt opac r g b depth - -, where xx, xt
+// and tt are the sums of o g dx^2, -o g dx t and o g t^2 (g = G dL/dalpha, t = dy
+// + s dx, s = record_shear).  With s = 0 they are the conic's gradients, xx and
+// tt times -2: their factor -0.5 is applied to the Gaussian's sum instead of to
+// every pixel's term (a power of two, so the sums and their rounding are
+// exactly the same)
 constexpr int kRG = 12;
 
 // The shear s = b / c that makes the conic diagonal: a dx^2 + 2 b dx dy +
-// c dy^2 = (a - b s) dx^2 + c (dy + s dx)^2.  What a thin, tilted splat's
-// gradient depends on is the small difference of its second moments in dx and
-// dy; in dx and t it is no difference, and the rounding of the sums stays what
-// it is instead of growing with the splat's length over its width.  (Any s
-// gives the same sums exactly, so the approximate reciprocal loses nothing:
-// both kernels take this one.)  0 where c has no finite reciprocal.
-// Error of the rotation gradients against float64, moments in dy -> in t,
-// medians: 100k splats at 613 x 347 3.7e-6 -> 2.4e-6 (50 scenes), 10k at
-// 256 x 256 2.3e-6 -> 0.9e-6 (40 scenes); a single scene's was up to nine
-// times that of sums that apply the conic pixel by pixel, and is now at most
-// theirs.  It costs an fma a pair: the 500k training step takes 648 us with
-// either.
+// c dy^2 = (a - b s) dx^2 + c (dy + s dx)^2.  In dx and t = dy + s dx the second
+// moments of a thin, tilted splat do not cancel.  (Any s gives the same sums
+// exactly, so the approximate reciprocal loses nothing.)  0 where c has no
+// finite reciprocal.
 __device__ __forceinline__ float conic_shear(float b, float c) {
   return c > 1e-30f ? b * __builtin_amdgcn_rcpf(c) : 0.0f;
+}
+
+// The shear of a splat's record.  0, the moments in dx and dy, unless the
+// conic's determinant is less than a 128th of a c: what the covariance's
+// gradient then makes of the sums is the reference's arithmetic, operation by
+// operation, and so is its rounding.  That of dx and dy grows with a c / det:
+// over 500 scenes of 2 000 to 30 000 splats the largest a c / det of a splat
+// that decided a gradient's rounding was 111, and the rotations' gradients were
+// off by up to 4e-4 of their norm there; past 128 a single splat's can have no
+// digit left in the direction of its thin axis.
+__device__ __forceinline__ float record_shear(float a, float b, float c) {
+  const float bb = b * b;
+  const float det = fmaf(a, c, -bb) - fmaf(b, b, -bb);
+  return a * c > 128.0f * det && det > 0.0f ? conic_shear(b, c) : 0.0f;
 }
 
 struct RBArgs {
@@ -211,6 +224,262 @@ __device__ __forceinline__ void wave_sum12(const float v[12], float w[3]) {
   }
 }
 
+// wave_sum12 of v[0..9] with v[10] = v[11] = 0 (the render backward's 10
+// terms): the last stage-1 sum is the literal 0, not a swap of two zeros.
+__device__ __forceinline__ void wave_sum10(const float v[10], float w[3]) {
+  float u[6];
+#pragma unroll
+  for (int i = 0; i < 5; ++i) swap_add32(v[2 * i], v[2 * i + 1], u[i]);
+  u[5] = 0.0f;
+#pragma unroll
+  for (int m = 0; m < 3; ++m) {
+    swap_add16(u[2 * m], u[2 * m + 1], w[m]);
+    w[m] = row_sum16(w[m]);
+  }
+  // keep the last row step with the reduction: the sums are consumed only
+  // by the storing lanes, and an add sunk into that branch would leave its
+  // DPP permutation as a separate move
+  asm volatile("" : : "v"(w[0]), "v"(w[1]), "v"(w[2]));
+}
+
+template <bool B>
+struct BoolTag {
+  static constexpr bool value = B;
+};
+
+// Fixed-order mode: the slot of a (Gaussian, tile) pair's sums -- the Gaussian's
+// first slot in the Gaussian-order prefix of tiles touched + the tile's
+// row-major rank in its rect (every pair of a list has exactly one chunk).
+__device__ __forceinline__ uint32_t pair_slot(const RBArgs& a, uint32_t g, const float4& sa, int radius, int tx, int ty) {
+  int x0, y0, x1, y1;
+  tile_rect(sa.x, sa.y, radius, a.gx, a.gy, x0, y0, x1, y1);
+  const uint32_t w = (uint32_t)(x1 - x0);
+  const uint32_t ntg = w * (uint32_t)(y1 - y0);
+  return a.block_excl[g >> 8] + a.local_incl[g] - ntg + (uint32_t)(ty - y0) * w + (uint32_t)(tx - x0);
+}
+
+// One 256-entry chunk of one tile's list, back to front, by 256 threads: thread
+// t is pixel t of the tile, and a wave takes its 8 x 8 quadrant through the
+// entries that reach it, one at a time.
+// VALU issue bounds it: ~100 instructions a (64-pixel, entry) step, 30 of them
+// the wave reduction, and half of the lanes blend nothing.  Sums by 4 x 4-pixel
+// cells (render_bwd_cells_item) need fewer, but round differently, and what a
+// thin, tilted splat's gradient keeps of its second moments is their rounding:
+// of 500 drop-in scenes of 2 000 to 30 000 splats, 13 had gradients of scales or
+// rotations moved by more than 2e-5 of their norm, up to 4e-4.  So the terms and
+// their order are those of the reference's formula here.  us, by pixels / by
+// cells: 163 / 108 for the training step (500 000 splats, 960 x 540), 73 / 34 at
+// 60 000 and 479 x 270, 60 / 28 at 10 000 and 256 x 256, 79 / 47 at 100 003 and 613
+// x 347 with a depth cotangent.  (202 for the step with the sums leaving one
+// entry a thread.)
+template <bool DET, bool DEP>
+__device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) {
+  constexpr int kTerms = 10;
+  constexpr int kParts = DET ? 4 : 1;  // LDS partial sets: one per wave when deterministic
+  // The item's 256-entry chunk is staged 128 entries at a time (back half
+  // first): half the LDS per workgroup, so twice as many workgroups fit on a
+  // CU (deterministic mode: 5 instead of 2).  The pixel state carries over.
+  constexpr int kSub = 128;
+  __shared__ uint32_t s_to[kSub];      // where a staged splat's sums go
+  __shared__ float4 s_a[kSub];
+  __shared__ float4 s_b[kSub];
+  __shared__ float4 s_c[kSub];
+  __shared__ uint32_t s_mask[kSub];    // quadrants each staged splat can reach (splat_quads)
+  __shared__ uint8_t s_list[4][kSub];  // per wave: the staged splats that reach its pixels
+  __shared__ __align__(16) float s_acc[kParts][kSub * kTerms];  // [..][entry][term]
+  if (item >= a.items[0]) return;
+  const uint4 rec = reinterpret_cast<const uint4*>(a.items)[1 + item];
+  const int tile = __builtin_amdgcn_readfirstlane((int)rec.x);
+  const uint32_t chunk = __builtin_amdgcn_readfirstlane((int)rec.y), r0 = __builtin_amdgcn_readfirstlane((int)rec.z);
+  const uint32_t maxc = __builtin_amdgcn_readfirstlane((int)rec.w);
+  const uint32_t cstart = chunk * 256;
+  const uint32_t cend = min(cstart + 256, maxc);
+  const int tx = tile % a.gx, ty = tile / a.gx;
+  int pdx, pdy;
+  tile_pixel(threadIdx.x, pdx, pdy);
+  const int px = tx * kBX + pdx, py = ty * kBY + pdy;
+  const bool inside = px < a.W && py < a.H;
+  const int pix = py * a.W + px;
+  const int HW = a.W * a.H;
+  const float pfx = (float)px, pfy = (float)py;
+  const float T_fin = inside ? a.final_T[pix] : 0.0f;
+  const uint32_t last = inside ? a.n_contrib[pix] : 0u;
+  float dpix0 = 0.f, dpix1 = 0.f, dpix2 = 0.f, dD = 0.f, dA = 0.f;
+  // per-pixel state at position cend (the end of this chunk)
+  float T = T_fin;
+  float acc0 = 0.f, acc1 = 0.f, acc2 = 0.f, acc_d = 0.f, acc_a = 0.f;
+  if (inside && last > cstart) {
+    dpix0 = a.dL_dcolor[pix];
+    dpix1 = a.dL_dcolor[HW + pix];
+    dpix2 = a.dL_dcolor[2 * HW + pix];
+    if constexpr (DEP) {
+      if (a.dL_ddepth) dD = a.dL_ddepth[pix];
+      if (a.dL_dalpha) dA = a.dL_dalpha[pix];
+    }
+    if (last > cend) {
+      // suffix sums from the forward's state at the boundary: sum_{k >= b} c_k a_k T_k = C_final - C_b
+      const float* ck = a.ckpt + (size_t)(a.ckpt_base[tile] + chunk) * 5 * 256 + threadIdx.x;
+      const float Tb = ck[0];
+      const float inv = 1.0f / Tb;
+      T = Tb;
+      acc0 = (a.accum[pix] - ck[256]) * inv;
+      acc1 = (a.accum[HW + pix] - ck[512]) * inv;
+      acc2 = (a.accum[2 * HW + pix] - ck[768]) * inv;
+      if constexpr (DEP) {
+        acc_d = (a.accum[3 * HW + pix] - ck[1024]) * inv;
+        acc_a = 1.0f - T_fin * inv;
+      }
+    }
+  }
+  const float bg_dot = (a.bg[0] * dpix0 + a.bg[1] * dpix1) + a.bg[2] * dpix2;
+  const bool bg_black = a.bg[0] == 0.0f && a.bg[1] == 0.0f && a.bg[2] == 0.0f;
+  const float ddelx = 0.5f * (float)a.W, ddely = 0.5f * (float)a.H;
+  const float a_min = 1.0f / 255.0f;
+  const int lane = threadIdx.x & 63;
+  const int wv = threadIdx.x >> 6;
+  // entries at or past the last contributor of every pixel of the wave are
+  // inactive on every lane
+  const uint32_t wlast = wave_max_u32(last);
+#pragma unroll 1
+  for (int sb = 1; sb >= 0; --sb) {
+    const uint32_t sbase = cstart + (uint32_t)(sb * kSub);
+    if (sbase >= cend) continue;  // (uniform) a chunk of at most 128 entries
+    const uint32_t send = min(sbase + (uint32_t)kSub, cend);
+    __syncthreads();  // the previous half's staged data has been flushed
+    if (threadIdx.x < kSub) {
+      const uint32_t q = sbase + threadIdx.x;
+      uint32_t m = 0u;
+      if (q < send) {
+        const uint32_t g = a.list[r0 + q] & a.id_mask;
+        const float4 sa = a.splat[3 * g], sb = a.splat[3 * g + 1], sc = a.splat[3 * g + 2];
+        s_a[threadIdx.x] = sa;
+        s_b[threadIdx.x] = make_float4(sb.x, sb.y, sb.z, record_shear(sa.z, sa.w, sb.x));
+        s_c[threadIdx.x] = sc;
+        m = splat_quads(sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, (float)(tx * kBX), (float)(ty * kBY));
+        s_to[threadIdx.x] = DET ? pair_slot(a, g, sa, __float_as_int(sc.w), tx, ty) : g;
+      }
+      s_mask[threadIdx.x] = m;
+    }
+    for (int k = threadIdx.x; k < kParts * kSub * kTerms / 4; k += 256)
+      reinterpret_cast<float4*>(&s_acc[0][0])[k] = make_float4(0.f, 0.f, 0.f, 0.f);
+    __syncthreads();
+    // the wave's own list: splats that miss its 8 x 8 pixels are ones no lane would use
+    const int lim = wlast > sbase ? (int)min(wlast - sbase, (uint32_t)kSub) : 0;
+    // (a sum of ballot counts, so wave-uniform; read from the first lane so
+    // that the pair loop below counts in a scalar register)
+    const int nw = __builtin_amdgcn_readfirstlane(compact_wave_list<kSub / 64>(s_mask, s_list[wv], wv, lane, lim));
+    // Branch-free per pair: masked lanes cost a SIMD as much as active ones,
+    // so every lane evaluates the pair; the only branches are wave-uniform
+    // skips when no lane is active.  An inactive lane runs with alpha = G = 0,
+    // which leaves its state unchanged (T / (1 - 0) = T, 0 c + 1 acc = acc) and
+    // makes each of its gradient terms 0, so no per-lane selects are needed.
+    // The running sums acc = sum_{k > current} c_k alpha_k T_k / T_{current+1}
+    // are advanced right after each splat (the reference advances them
+    // lazily at the next one, from last_alpha / last_color; same expression,
+    // same rounding).
+    // The pair loop in two forms: a black background (the reference's
+    // default) adds nothing to dL/dalpha -- its term is a signed zero -- so
+    // that form leaves the term out (the choice is wave-uniform).
+    auto pair_loop = [&](auto bg_on) {
+      for (int i = nw - 1; i >= 0; --i) {
+        // Gradient arithmetic may fuse multiply-adds (the library is built
+        // without contraction for the forward's bit-exactness).  What decides
+        // which pairs contribute -- blend_power, spec_expf and the single
+        // product alpha = o G -- is outside this scope or has no add, so it
+        // stays exactly the forward's.
+  #pragma clang fp contract(fast)
+        const int j = s_list[wv][i];
+        const uint32_t q = sbase + j;  // 0-based list position; contributor index q + 1
+        const float4 ga = s_a[j];
+        const float4 gb = s_b[j];
+        const float dx = ga.x - pfx, dy = ga.y - pfy;
+        const float power = blend_power(ga.z, ga.w, gb.x, dx, dy);
+        // (q < last implies inside: last is 0 outside the image.)  The
+        // wave-uniform skip tests the product of one ballot per compare, which
+        // is the ballot of the conjunction: a ballot of a single compare is
+        // that compare's lane mask.
+        const float Graw = spec_expf(power);
+        const float alpha_raw = fminf(0.99f, gb.y * Graw);
+        const bool in_list = q < last, p_le0 = !(power > 0.0f), a_ok = !(alpha_raw < a_min);
+        const uint64_t live = __builtin_amdgcn_ballot_w64(in_list) & __builtin_amdgcn_ballot_w64(p_le0) &
+                              __builtin_amdgcn_ballot_w64(a_ok);
+        if (live == 0ull) continue;
+        const bool active = in_list && p_le0 && a_ok;
+        const float G = active ? Graw : 0.0f;
+        const float alpha = active ? alpha_raw : 0.0f;
+        const float4 gc = s_c[j];
+        // T before this splat; the gradient tolerates the 1-ulp reciprocal
+        const float inv_1ma = __builtin_amdgcn_rcpf(1.0f - alpha);
+        const float Tn = T * inv_1ma;
+        const float w = alpha * Tn;
+        float dL_da = (gc.x - acc0) * dpix0;
+        dL_da += (gc.y - acc1) * dpix1;
+        dL_da += (gc.z - acc2) * dpix2;
+        if constexpr (DEP) {
+          dL_da += (gb.z - acc_d) * dD;
+          dL_da += (1.0f - acc_a) * dA;
+        }
+        dL_da *= Tn;
+        if constexpr (decltype(bg_on)::value) dL_da += (-T_fin * inv_1ma) * bg_dot;
+        const float dL_dG = gb.y * dL_da;
+        const float gdx = G * dx, gdy = G * dy;
+        const float dG_dx = -gdx * ga.z - gdy * ga.w;
+        const float dG_dy = -gdy * gb.x - gdx * ga.w;
+        float v[10];
+        v[0] = dL_dG * dG_dx * ddelx;
+        v[1] = dL_dG * dG_dy * ddely;
+        const float t = fmaf(gb.w, dx, dy);  // dy for all but the thinnest splats (record_shear)
+        v[2] = gdx * dx * dL_dG;
+        v[3] = -gdx * t * dL_dG;
+        v[4] = G * t * t * dL_dG;
+        v[5] = G * dL_da;
+        v[6] = w * dpix0;
+        v[7] = w * dpix1;
+        v[8] = w * dpix2;
+        v[9] = DEP ? w * dD : 0.0f;
+        T = Tn;
+        const float oma = 1.0f - alpha;
+        acc0 = alpha * gc.x + oma * acc0;
+        acc1 = alpha * gc.y + oma * acc1;
+        acc2 = alpha * gc.z + oma * acc2;
+        if constexpr (DEP) {
+          acc_d = alpha * gb.z + oma * acc_d;
+          acc_a = alpha + oma * acc_a;
+        }
+        float sums[3];
+        wave_sum10(v, sums);
+        if ((lane & 15) == 0) {
+          const int r = lane >> 4;
+          const int o = r == 1 ? 2 : (r == 2 ? 1 : r);  // value of row r: 4m + {0, 2, 1, 3}[r]
+#pragma unroll
+          for (int m = 0; m < 3; ++m) {
+            const int k = 4 * m + o;
+            if (k < (DEP ? 10 : 9)) {
+              if constexpr (DET) s_acc[wv][j * kTerms + k] = sums[m];
+              else atomicAdd(&s_acc[0][j * kTerms + k], sums[m]);  // (a zero adds nothing; testing for it costs more)
+            }
+          }
+        }
+      }
+    };
+    if (bg_black) pair_loop(BoolTag<false>{});
+    else pair_loop(BoolTag<true>{});
+    __syncthreads();
+    // The sums leave with consecutive threads on consecutive words of an
+    // entry's record, so an instruction touches a record's cache line once: one
+    // thread per entry sends every word of a wave's 64 records on its own.
+    for (uint32_t i = threadIdx.x; i < (send - sbase) * kTerms; i += 256) {
+      const uint32_t en = i / kTerms, t = i - en * kTerms;
+      if constexpr (DET) {
+        a.part[(size_t)s_to[en] * kTerms + t] = ((s_acc[0][i] + s_acc[1][i]) + s_acc[2][i]) + s_acc[3][i];
+      } else {
+        const float s = s_acc[0][i];
+        if (s != 0.0f) unsafeAtomicAdd(a.g_render + (size_t)s_to[en] * kRG + t, s);
+      }
+    }
+  }
+}
+
 // ---- scans over the 16 lanes of each DPP row, four independent chains -------
 // Lane e of a row holds entry e of a group, and the four chains are the four
 // pixels the lane works on.  A DPP operand needs two wait states after the
@@ -278,7 +547,12 @@ __device__ __forceinline__ void rows_reduce(const float (&v)[N], float (&w)[(N +
   for (int m = 0; m < M; ++m) swap_add16(u[2 * m], u[2 * m + 1], w[m]);
 }
 
-// One 256-entry chunk of one tile's list, back to front, by 256 threads.
+// The same chunk by 4 x 4-pixel cells, for the fixed-order colour backward of a
+// frame with a pose.  What such a caller wants is the pose's gradient, a sum over
+// all Gaussians in which the rounding of a single thin one does not show (the
+// poses of 24 batches of solves differ by 1.4e-6 of their norm in the median,
+// 9e-6 at most, with either kernel's sums), and it is 44 us by cells and 110 by
+// pixels for a frame of 129 600 splats at 480 x 270.
 //
 // What bounds it is VALU issue: the exact exponential and the gradient of
 // every (pixel, splat) pair.  Three choices keep the instructions per pair low.
@@ -293,39 +567,36 @@ __device__ __forceinline__ void rows_reduce(const float (&v)[N], float (&w)[(N +
 //    its own lanes over the cell's 16 pixels and are summed over the 4 rows of
 //    lanes once per group (rows_reduce), where one entry at a time on 64
 //    pixels needs a 30-instruction wave reduction for every entry.
-//  * Only sums over pixels are formed here: with g = G dL/dalpha the moments
+//  * Only sums over pixels are formed per pair: with g = G dL/dalpha the moments
 //    of g in (dx, t) up to the second order (conic_shear), and w dL/dcolour.  What is
-//    constant per splat (its opacity, its conic) is applied to the sums in
-//    k_preprocess_bwd.
+//    constant per splat (its opacity, its conic) is applied to the chunk's sums.
 // The colour recurrence is carried as one number per pixel: with d = colour .
-// dL/dcolour (+ depth and alpha terms), dL/dalpha_k = T_k d_k - R_k / (1 -
+// dL/dcolour, dL/dalpha_k = T_k d_k - R_k / (1 -
 // alpha_k), R_k = the sum of w d over the later entries plus T_final times
 // background . dL/dcolour.
-template <bool DET, bool DEP, bool PO>
-__device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) {
-  // PO (pose-only, fixed-order, colour cotangent only): the caller wants only
-  // the pose gradient, which at active SH degree 0 depends on a splat's
+template <bool PO>
+__device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t item) {
+  // PO (pose-only): the caller wants only the pose gradient, which at active SH degree 0 depends on a splat's
   // screen position and conic alone, so only those five sums are formed and
   // stored per (Gaussian, tile) pair.  Their arithmetic is the full path's,
   // term for term, so the pose gradient has the same bits either way.
-  static_assert(!PO || (DET && !DEP), "the pose-only backward is fixed-order and colour-only");
   constexpr int kTerms = PO ? 5 : 10;
-  constexpr int kVals = PO ? 5 : (DEP ? 10 : 9);  // (without a depth cotangent its sum is 0)
+  constexpr int kVals = PO ? 5 : 9;  // (without a depth cotangent its sum is 0)
   constexpr int kSub = 256;                       // entries of a chunk
   // LDS sizes decide how many workgroups share a CU: 53 KB for the colour
   // gradient, so three; 37 KB for the pose-only form, four.
   __shared__ float4 s_a[kSub];  // x, y, conic a, conic b
   __shared__ float4 s_b[kSub];  // conic c, opacity, r, g
-  __shared__ float s_c[DEP ? 2 : 1][kSub];  // b, depth
+  __shared__ float s_c[kSub];   // b
   __shared__ uint16_t s_mask[kSub];    // cells each staged splat can reach (splat_cells)
   __shared__ __align__(4) uint8_t s_list[4][kSub];  // per wave: the staged splats that reach the cell at hand
   // per pixel, cell by cell: T and R at the chunk's end, last contributor, the cotangents
   __shared__ float2 s_tr[256];
   __shared__ uint32_t s_last[256];
-  __shared__ float s_d[DEP ? 5 : 3][256];
+  __shared__ float s_d[3][256];
   // every wave sums into rows of its own with plain reads and writes: float
   // adds to LDS from 64 lanes took ~100 cycles each and held the kernel
-  __shared__ float s_acc[4][kSub * kVals];  // [wave][entry][sum]
+  __shared__ __align__(16) float s_acc[4][kSub * kVals];  // [wave][entry][sum]
   if (item >= a.items[0]) return;
   const uint4 rec = reinterpret_cast<const uint4*>(a.items)[1 + item];
   const int tile = __builtin_amdgcn_readfirstlane((int)rec.x);
@@ -343,15 +614,11 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
     const int pix = py * a.W + px;
     const int HW = a.W * a.H;
     const uint32_t last = inside ? a.n_contrib[pix] : 0u;
-    float T = 0.f, R = 0.f, d0 = 0.f, d1 = 0.f, d2 = 0.f, dD = 0.f, dA = 0.f;
+    float T = 0.f, R = 0.f, d0 = 0.f, d1 = 0.f, d2 = 0.f;
     if (last > cstart) {
       d0 = a.dL_dcolor[pix];
       d1 = a.dL_dcolor[HW + pix];
       d2 = a.dL_dcolor[2 * HW + pix];
-      if constexpr (DEP) {
-        if (a.dL_ddepth) dD = a.dL_ddepth[pix];
-        if (a.dL_dalpha) dA = a.dL_dalpha[pix];
-      }
       const float T_fin = a.final_T[pix];
       T = T_fin;
       R = T_fin * ((a.bg[0] * d0 + a.bg[1] * d1) + a.bg[2] * d2);
@@ -362,10 +629,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
         R += (a.accum[pix] - ck[256]) * d0;
         R += (a.accum[HW + pix] - ck[512]) * d1;
         R += (a.accum[2 * HW + pix] - ck[768]) * d2;
-        if constexpr (DEP) {
-          R += (a.accum[3 * HW + pix] - ck[1024]) * dD;
-          R += (T - T_fin) * dA;
-        }
       }
     }
     const int slot = ((pdy >> 2) * 4 + (pdx >> 2)) * 16 + (pdy & 3) * 4 + (pdx & 3);
@@ -374,10 +637,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
     s_d[0][slot] = d0;
     s_d[1][slot] = d1;
     s_d[2][slot] = d2;
-    if constexpr (DEP) {
-      s_d[3][slot] = dD;
-      s_d[4][slot] = dA;
-    }
   }
   const float a_min = 1.0f / 255.0f;
   const int e = lane & 15, k = lane >> 4;
@@ -392,8 +651,7 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
       radius = __float_as_int(sc.w);
       s_a[threadIdx.x] = sa;
       s_b[threadIdx.x] = make_float4(sb.x, sb.y, sc.x, sc.y);
-      s_c[0][threadIdx.x] = sc.z;
-      if constexpr (DEP) s_c[1][threadIdx.x] = sb.z;
+      s_c[threadIdx.x] = sc.z;
       m = splat_cells(sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, (float)(tx * kBX), (float)(ty * kBY));
     }
     s_mask[threadIdx.x] = (uint16_t)m;
@@ -409,7 +667,7 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
 #pragma unroll 1
   for (int cy = 0; cy < 4; ++cy) {
     const int cx = (wv + cy) & 3, cell = 4 * cy + cx;
-    float T[4], R[4], dc0[4], dc1[4], dc2[4], dD[4], dA[4];
+    float T[4], R[4], dc0[4], dc1[4], dc2[4];
     uint32_t last[4];
     uint32_t cl = 0;  // the cell's last contributor
 #pragma unroll
@@ -422,10 +680,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
       dc0[q] = s_d[0][at];
       dc1[q] = s_d[1][at];
       dc2[q] = s_d[2][at];
-      if constexpr (DEP) {
-        dD[q] = s_d[3][at];
-        dA[q] = s_d[4][at];
-      }
       cl = max(cl, last[q]);
     }
     cl = max(cl, (uint32_t)__shfl_xor((int)cl, 16, 64));
@@ -451,7 +705,7 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
       const int j = s_list[wv][have ? i0 + e : n - 1];  // (lanes past the list repeat its last entry, inactive)
       const uint32_t pos = have ? cstart + (uint32_t)j : 0xffffffffu;  // 0-based list position
       const float4 ga = s_a[j], gb = s_b[j];
-      const float cb = s_c[0][j];
+      const float cb = s_c[j];
       const float dx = ga.x - pfx;
       const float ax = ga.z * dx, bx = ga.w * dx, sh = conic_shear(ga.w, gb.x);
       float dy[4], alpha[4], G[4], d[4], inv[4];
@@ -466,7 +720,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
         G[q] = active ? Graw : 0.0f;
         inv[q] = __builtin_amdgcn_rcpf(1.0f - alpha[q]);
         d[q] = fmaf(cb, dc2[q], fmaf(gb.w, dc1[q], gb.z * dc0[q]));
-        if constexpr (DEP) d[q] = fmaf(s_c[1][j], dD[q], d[q]) + dA[q];
       }
       // T before each entry from T after the group, and the sum behind it
       float Q[4], Tb[4], w[4], X[4], S[4];
@@ -479,7 +732,7 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
         X[q] = w[q] * d[q];
       }
       row_suffix_sum4(X, R, S);
-      float m0 = 0.f, m1 = 0.f, m2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f, c3 = 0.f;
+      float m0 = 0.f, m1 = 0.f, m2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
         const float g = G[q] * fmaf(Tb[q], d[q], -(S[q] * inv[q]));
@@ -491,7 +744,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
           c0 = fmaf(w[q], dc0[q], c0);
           c1 = fmaf(w[q], dc1[q], c1);
           c2 = fmaf(w[q], dc2[q], c2);
-          if constexpr (DEP) c3 = fmaf(w[q], dD[q], c3);
         }
       }
       const float mx = dx * m0;
@@ -506,7 +758,6 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
         v[6] = c0;
         v[7] = c1;
         v[8] = c2;
-        if constexpr (DEP) v[9] = c3;
       }
       rows_reduce<kVals>(v, o);
       const int val = k == 1 ? 2 : (k == 2 ? 1 : k);
@@ -523,59 +774,77 @@ __device__ __forceinline__ void render_bwd_item(const RBArgs& a, uint32_t item) 
   // thread per entry sends every word of a wave's 64 records on its own, and
   // the atomics of the 500k-Gaussian training scene then held the kernel).
   const uint32_t ne = cend - cstart;
-  uint32_t* s_to = reinterpret_cast<uint32_t*>(&s_list[0][0]);  // per entry: where its sums go
+  uint32_t* s_to = reinterpret_cast<uint32_t*>(&s_list[0][0]);  // per entry: the slot of its sums
   if (threadIdx.x < ne) {
-    uint32_t to = g;
-    if constexpr (DET) {
-      // slot of this (Gaussian, tile) pair: the Gaussian's first slot in the
-      // Gaussian-order prefix of tiles touched + the tile's row-major rank in
-      // its rect (every pair of the list has exactly one chunk)
-      int x0, y0, x1, y1;
-      const float4 sa = s_a[threadIdx.x];
-      tile_rect(sa.x, sa.y, radius, a.gx, a.gy, x0, y0, x1, y1);
-      const uint32_t w = (uint32_t)(x1 - x0);
-      const uint32_t ntg = w * (uint32_t)(y1 - y0);
-      to = a.block_excl[g >> 8] + a.local_incl[g] - ntg + (uint32_t)(ty - y0) * w + (uint32_t)(tx - x0);
+    // the entry's sums over the four waves, turned into the record's terms:
+    // dL/dG = o g, dG/ddx = -G (a dx + b dy) = -G ((a - b s) dx + b t), dG/ddy = -G
+    // (c t + (b - c s) dx), a pixel's displacement in NDC units; dy = t - s dx
+    float v[kVals];
+    float* row = &s_acc[0][threadIdx.x * kVals];
+#pragma unroll
+    for (int i = 0; i < kVals; ++i)
+      v[i] = ((row[i] + row[kSub * kVals + i]) + row[2 * kSub * kVals + i]) + row[3 * kSub * kVals + i];
+    const float4 sa = s_a[threadIdx.x];
+    const float cc = s_b[threadIdx.x].x, op = s_b[threadIdx.x].y, sh = conic_shear(sa.w, cc);
+    const float gx = op * v[0], gt = op * v[1];
+    row[0] = -(fmaf(-sa.w, sh, sa.z) * gx + sa.w * gt) * (0.5f * (float)a.W);
+    row[1] = -(cc * gt + fmaf(-cc, sh, sa.w) * gx) * (0.5f * (float)a.H);
+    if (record_shear(sa.z, sa.w, cc) == 0.0f) {
+      const float xy = fmaf(-sh, v[2], v[3]);
+      v[4] = fmaf(-sh, v[3] + xy, v[4]);
+      v[3] = xy;
     }
-    s_to[threadIdx.x] = to;
+    row[2] = op * v[2];
+    row[3] = -op * v[3];
+    row[4] = op * v[4];
+#pragma unroll
+    for (int i = 5; i < kVals; ++i) row[i] = v[i];
+    s_to[threadIdx.x] = pair_slot(a, g, sa, radius, tx, ty);
   }
   __syncthreads();
   for (uint32_t i = threadIdx.x; i < ne * kTerms; i += 256) {
     const uint32_t en = i / kTerms, t = i - en * kTerms;
-    float sum = 0.0f;
-    if (t < kVals) {
-      const uint32_t at = en * kVals + t;
-      sum = ((s_acc[0][at] + s_acc[1][at]) + s_acc[2][at]) + s_acc[3][at];
-    }
-    if constexpr (DET) {
-      a.part[(size_t)s_to[en] * kTerms + t] = sum;
-    } else {
-      if (sum != 0.0f) unsafeAtomicAdd(a.g_render + (size_t)s_to[en] * kRG + t, sum);
-    }
+    a.part[(size_t)s_to[en] * kTerms + t] = t < kVals ? s_acc[0][en * kVals + t] : 0.0f;
   }
 }
 
 // The grid is an upper bound on the item count, so items are taken in
 // dispatch order: live items then go round-robin over all 8 XCDs (a
 // contiguous-per-XCD remap would put them all on the first few).
-template <bool DET, bool DEP, bool PO>
+template <bool DET, bool DEP>
 __global__ __launch_bounds__(256) void k_render_bwd(RBArgs a) {
-  render_bwd_item<DET, DEP, PO>(a, blockIdx.x);
+  render_bwd_item<DET, DEP>(a, blockIdx.x);
+}
+
+template <bool PO>
+__global__ __launch_bounds__(256) void k_render_bwd_cells(RBArgs a) {
+  render_bwd_cells_item<PO>(a, blockIdx.x);
 }
 
 // Many frames in one launch: frame f owns blocks [prefix[f], prefix[f + 1]),
 // an upper bound on its work items.
-template <bool DET, bool DEP, bool PO>
-__global__ __launch_bounds__(256) void k_render_bwd_multi(const uint32_t* prefix, const RBArgs* args, int n) {
-  const uint32_t b = blockIdx.x;
+__device__ __forceinline__ int frame_of_item(const uint32_t* prefix, int n, uint32_t b) {
   int lo = 0, hi = n - 1;
   while (lo < hi) {
     const int mid = (lo + hi + 1) >> 1;
     if (prefix[mid] <= b) lo = mid;
     else hi = mid - 1;
   }
-  const RBArgs a = args[lo];
-  render_bwd_item<DET, DEP, PO>(a, b - prefix[lo]);
+  return lo;
+}
+
+template <bool DET, bool DEP>
+__global__ __launch_bounds__(256) void k_render_bwd_multi(const uint32_t* prefix, const RBArgs* args, int n) {
+  const int f = frame_of_item(prefix, n, blockIdx.x);
+  const RBArgs a = args[f];
+  render_bwd_item<DET, DEP>(a, blockIdx.x - prefix[f]);
+}
+
+template <bool PO>
+__global__ __launch_bounds__(256) void k_render_bwd_cells_multi(const uint32_t* prefix, const RBArgs* args, int n) {
+  const int f = frame_of_item(prefix, n, blockIdx.x);
+  const RBArgs a = args[f];
+  render_bwd_cells_item<PO>(a, blockIdx.x - prefix[f]);
 }
 
 // Deterministic mode: per Gaussian, the partials of its (Gaussian, tile)
@@ -785,9 +1054,7 @@ __device__ __forceinline__ void preprocess_bwd_block(const PBArgs& a, int bid, f
   if (a.pose) make_pose(a.pose, ps);
   if (i < a.P) {
     const bool vis = a.radii[i] > 0;
-    // the render-gradient record, then m2x m2y and o times the second moments dx^2 dx t | t^2 opac r g | b depth - -
-    float4 rA, rB, rC;
-    float shear = 0.0f;
+    float4 rA, rB, rC;  // m2x m2y xx xt | tt opac r g | b depth - -
     if (a.part5) {
       // the sums k_det_gather<5> forms, in its order (terms 5..9 are zero)
       float acc[5] = {0.f, 0.f, 0.f, 0.f, 0.f};
@@ -808,18 +1075,6 @@ __device__ __forceinline__ void preprocess_bwd_block(const PBArgs& a, int bid, f
       rA = reinterpret_cast<const float4*>(rg)[0];
       rB = reinterpret_cast<const float4*>(rg)[1];
       rC = reinterpret_cast<const float4*>(rg)[2];
-    }
-    if (vis) {
-      // the record's moments times the splat's constants: dL/dG = o g, dG/ddx =
-      // -G (a dx + b dy) = -G ((a - b s) dx + b t) and dG/ddy = -G (c dy + b dx)
-      // = -G (c t + (b - c s) dx), with a pixel's displacement in NDC units
-      const float4 s0 = a.splat[3 * i], s1 = a.splat[3 * i + 1];
-      shear = conic_shear(s0.w, s1.x);
-      const float gx = s1.y * rA.x, gt = s1.y * rA.y;
-      const float mx = -(fmaf(-s0.w, shear, s0.z) * gx + s0.w * gt) * (0.5f * (float)a.W);
-      const float my = -(s1.x * gt + fmaf(-s1.x, shear, s0.w) * gx) * (0.5f * (float)a.H);
-      rA = make_float4(mx, my, s1.y * rA.z, s1.y * rA.w);
-      rB.x = s1.y * rB.x;
     }
     // (every per-Gaussian output is optional: a pose-only solve asks for none)
     if (a.dL_dmeans2D) {
@@ -867,20 +1122,35 @@ __device__ __forceinline__ void preprocess_bwd_block(const PBArgs& a, int bid, f
       const float ca = T0[0] * ST0[0] + T0[1] * ST0[1] + T0[2] * ST0[2] + 0.3f;
       const float cb = T0[0] * ST1[0] + T0[1] * ST1[1] + T0[2] * ST1[2];
       const float cc = T1[0] * ST1[0] + T1[1] * ST1[1] + T1[2] * ST1[2] + 0.3f;
-      // With p = cc dx - cb dy and r = ca dy - cb dx (the conic's rows times the
-      // determinant): dL/dca = o g p^2 / (2 den^2), dL/dcb = o g p r / den^2,
-      // dL/dcc = o g r^2 / (2 den^2), and p = k1 dx - cb t, r = ca t - k2 dx.
-      // The differences k1, k2 and den are rounded once.
-      const float cb2 = cb * cb;
-      const float den = fmaf(ca, cc, -cb2) + fmaf(-cb, cb, cb2);
-      const float k1 = fmaf(cb, shear, cc), k2 = fmaf(ca, shear, cb);
-      const float mxx = rA.z, mxt = rA.w, mtt = rB.x;
-      const float d2i = 1.0f / (den * den + 0.0000001f);
-      float dLa = 0.f, dLb = 0.f, dLc = 0.f;
+      const float4 s0 = a.splat[3 * i], s1 = a.splat[3 * i + 1];
+      const float shear = record_shear(s0.z, s0.w, s1.x);
+      float dLa = 0.f, dLb = 0.f, dLc = 0.f, d2i;
+      if (shear == 0.0f) {
+        const float den = ca * cc - cb * cb;
+        const float gA = -0.5f * rA.z, gB = rA.w, gC = -0.5f * rB.x;
+        d2i = 1.0f / (den * den + 0.0000001f);
+        if (d2i != 0.0f) {
+          dLa = d2i * (-cc * cc * gA + cb * cc * gB + (den - ca * cc) * gC);
+          dLc = d2i * (-ca * ca * gC + ca * cb * gB + (den - ca * cc) * gA);
+          dLb = d2i * (2.0f * cb * cc * gA - (den + 2.0f * cb * cb) * gB + 2.0f * ca * cb * gC);
+        }
+      } else {
+        // With p = cc dx - cb dy and r = ca dy - cb dx (the conic's rows times the
+        // determinant): dL/dca = o g p^2 / (2 den^2), dL/dcb = o g p r / den^2,
+        // dL/dcc = o g r^2 / (2 den^2), and p = k1 dx - cb t, r = ca t - k2 dx.
+        // The differences k1, k2 and den are rounded once.
+        const float cb2 = cb * cb;
+        const float den = fmaf(ca, cc, -cb2) + fmaf(-cb, cb, cb2);
+        const float k1 = fmaf(cb, shear, cc), k2 = fmaf(ca, shear, cb);
+        const float mxx = rA.z, mxt = -rA.w, mtt = rB.x;
+        d2i = 1.0f / (den * den + 0.0000001f);
+        if (d2i != 0.0f) {
+          dLa = 0.5f * d2i * (k1 * k1 * mxx - 2.0f * k1 * cb * mxt + cb2 * mtt);
+          dLc = 0.5f * d2i * (ca * ca * mtt - 2.0f * ca * k2 * mxt + k2 * k2 * mxx);
+          dLb = d2i * ((k1 * ca + cb * k2) * mxt - k1 * k2 * mxx - ca * cb * mtt);
+        }
+      }
       if (d2i != 0.0f) {
-        dLa = 0.5f * d2i * (k1 * k1 * mxx - 2.0f * k1 * cb * mxt + cb2 * mtt);
-        dLc = 0.5f * d2i * (ca * ca * mtt - 2.0f * ca * k2 * mxt + k2 * k2 * mxx);
-        dLb = d2i * ((k1 * ca + cb * k2) * mxt - k1 * k2 * mxx - ca * cb * mtt);
         gS[0] = T0[0] * T0[0] * dLa + T0[0] * T1[0] * dLb + T1[0] * T1[0] * dLc;
         gS[3] = T0[1] * T0[1] * dLa + T0[1] * T1[1] * dLb + T1[1] * T1[1] * dLc;
         gS[5] = T0[2] * T0[2] * dLa + T0[2] * T1[2] * dLb + T1[2] * T1[2] * dLc;
@@ -1343,14 +1613,15 @@ static void bwd_render(const gs_frame_t* f, int P, long long capacity, const RBA
   timing::Scope ts(timing::kRenderBwd, s);
   const dim3 grid((unsigned)max_items);
   const bool dep = r.dL_ddepth || r.dL_dalpha;
-  if (po) {
-    hipLaunchKernelGGL((k_render_bwd<true, false, true>), grid, dim3(256), 0, s, r);
+  if (f->deterministic && f->pose && !dep) {
+    if (po) hipLaunchKernelGGL(k_render_bwd_cells<true>, grid, dim3(256), 0, s, r);
+    else hipLaunchKernelGGL(k_render_bwd_cells<false>, grid, dim3(256), 0, s, r);
   } else if (f->deterministic) {
-    if (dep) hipLaunchKernelGGL((k_render_bwd<true, true, false>), grid, dim3(256), 0, s, r);
-    else hipLaunchKernelGGL((k_render_bwd<true, false, false>), grid, dim3(256), 0, s, r);
+    if (dep) hipLaunchKernelGGL((k_render_bwd<true, true>), grid, dim3(256), 0, s, r);
+    else hipLaunchKernelGGL((k_render_bwd<true, false>), grid, dim3(256), 0, s, r);
   } else {
-    if (dep) hipLaunchKernelGGL((k_render_bwd<false, true, false>), grid, dim3(256), 0, s, r);
-    else hipLaunchKernelGGL((k_render_bwd<false, false, false>), grid, dim3(256), 0, s, r);
+    if (dep) hipLaunchKernelGGL((k_render_bwd<false, true>), grid, dim3(256), 0, s, r);
+    else hipLaunchKernelGGL((k_render_bwd<false, false>), grid, dim3(256), 0, s, r);
   }
 }
 
@@ -1536,6 +1807,8 @@ extern "C" int gs_backward_finish(GS_BWD_ARGS) {
 // ---- many frames in one render-backward launch -----------------------------
 // Set layout: uint32 prefix[n + 1] of work-item bounds per frame, then
 // RBArgs[n] at a 256-byte boundary.
+// beside the workgroup count the build returns: every frame has a pose
+constexpr unsigned kSetPosed = 1u << 31;
 static size_t multi_rb_args_offset(int n) { return align_up(sizeof(uint32_t) * (size_t)(n + 1), 256); }
 
 extern "C" size_t gs_multi_render_bwd_bytes(int n) {
@@ -1555,6 +1828,7 @@ extern "C" int gs_multi_render_bwd_build(int n, const gs_frame_t* frames, const 
   RBArgs* args = (RBArgs*)((char*)host_set + multi_rb_args_offset(n));
   unsigned long long total = 0;
   const int det = frames[0].deterministic != 0;
+  bool posed = true;
   for (int i = 0; i < n; ++i) {
     const gs_frame_t* f = &frames[i];
     if (f->width <= 0 || f->height <= 0 || !f->bg || P[i] < 0 || !image[i] || !dL_dcolor[i] || !scratch[i])
@@ -1565,11 +1839,12 @@ extern "C" int gs_multi_render_bwd_build(int n, const gs_frame_t* frames, const 
     prefix[i] = (uint32_t)total;
     if (capacity[i] > 0 && P[i] > 0) total += (unsigned long long)rb_max_items(f, capacity[i]);
     if (total > 0x7fffffffULL) return GS_E_ARG;
+    posed &= f->pose != nullptr;
     args[i] = make_rb_args(f, P[i], geom[i], capacity[i], binning[i], image[i], dL_dcolor[i],
                            dL_ddepth ? dL_ddepth[i] : nullptr, dL_dalpha ? dL_dalpha[i] : nullptr, scratch[i]);
   }
   prefix[n] = (uint32_t)total;
-  *total_blocks = (unsigned)total;
+  *total_blocks = (unsigned)total | (posed ? kSetPosed : 0u);
   return GS_OK;
 }
 
@@ -1577,6 +1852,8 @@ extern "C" int gs_multi_render_bwd(int n, const void* dev_set, unsigned total_bl
   if (n <= 0 || !dev_set || (flags & ~7)) return GS_E_ARG;
   const bool det = flags & 1, dep = !(flags & GS_RB_COLOR_ONLY), po = flags & GS_RB_POSE_ONLY;
   if (po && (!det || dep)) return GS_E_ARG;
+  const bool posed = total_blocks & kSetPosed;
+  total_blocks &= ~kSetPosed;
   if (total_blocks == 0) return GS_OK;
   hipStream_t s = (hipStream_t)stream;
   const uint32_t* prefix = (const uint32_t*)dev_set;
@@ -1584,13 +1861,15 @@ extern "C" int gs_multi_render_bwd(int n, const void* dev_set, unsigned total_bl
   timing::Scope ts(timing::kRenderBwd, s);
   const dim3 grid(total_blocks);
   if (po) {
-    hipLaunchKernelGGL((k_render_bwd_multi<true, false, true>), grid, dim3(256), 0, s, prefix, args, n);
+    hipLaunchKernelGGL(k_render_bwd_cells_multi<true>, grid, dim3(256), 0, s, prefix, args, n);
+  } else if (det && !dep && posed) {
+    hipLaunchKernelGGL(k_render_bwd_cells_multi<false>, grid, dim3(256), 0, s, prefix, args, n);
   } else if (det) {
-    if (dep) hipLaunchKernelGGL((k_render_bwd_multi<true, true, false>), grid, dim3(256), 0, s, prefix, args, n);
-    else hipLaunchKernelGGL((k_render_bwd_multi<true, false, false>), grid, dim3(256), 0, s, prefix, args, n);
+    if (dep) hipLaunchKernelGGL((k_render_bwd_multi<true, true>), grid, dim3(256), 0, s, prefix, args, n);
+    else hipLaunchKernelGGL((k_render_bwd_multi<true, false>), grid, dim3(256), 0, s, prefix, args, n);
   } else {
-    if (dep) hipLaunchKernelGGL((k_render_bwd_multi<false, true, false>), grid, dim3(256), 0, s, prefix, args, n);
-    else hipLaunchKernelGGL((k_render_bwd_multi<false, false, false>), grid, dim3(256), 0, s, prefix, args, n);
+    if (dep) hipLaunchKernelGGL((k_render_bwd_multi<false, true>), grid, dim3(256), 0, s, prefix, args, n);
+    else hipLaunchKernelGGL((k_render_bwd_multi<false, false>), grid, dim3(256), 0, s, prefix, args, n);
   }
   return hipGetLastError() == hipSuccess ? GS_OK : GS_E_LAUNCH;
 }

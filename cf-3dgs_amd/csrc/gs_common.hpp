@@ -477,6 +477,40 @@ __device__ __forceinline__ uint32_t splat_cells(float x, float y, float a, float
   return e.none ? 0u : (e.all ? 0xffffu : m);
 }
 
+// The 8 x 8-pixel quadrants of the tile at (x0, y0) that the splat can reach:
+// bit 2 qy + qx.  One band per row of quadrants.
+__device__ __forceinline__ uint32_t splat_quads(float x, float y, float a, float b, float c, float o, float x0,
+                                                float y0) {
+  const SplatReach e(a, b, c, o);
+  const float u = x0 - x, v = y0 - y;
+  uint32_t m = 0u;
+#pragma unroll
+  for (int r = 0; r < 2; ++r) {
+    float left, right;
+    const bool hit = e.band(v + (float)(8 * r), v + (float)(8 * r + 7), left, right);
+    const uint32_t row = (left <= u + 7.0f && right >= u ? 1u : 0u) | (left <= u + 15.0f && right >= u + 8.0f ? 2u : 0u);
+    m |= hit ? row << (2 * r) : 0u;
+  }
+  return e.none ? 0u : (e.all ? 0xfu : m);
+}
+
+// A wave's own list of the staged splats that meet its pixels: positions j
+// < limit (ascending) with bit `wv` set in s_mask[j]; returns the count
+// (wave-uniform).  Needs all 64 lanes active.  NC * 64 staged entries.
+template <int NC>
+__device__ __forceinline__ int compact_wave_list(const uint32_t* s_mask, uint8_t* s_list, int wv, int lane, int limit) {
+  int n = 0;
+#pragma unroll
+  for (int c = 0; c < NC; ++c) {
+    const int idx = c * 64 + lane;
+    const bool hit = idx < limit && ((s_mask[idx] >> wv) & 1u);
+    const uint64_t bal = __ballot(hit);
+    if (hit) s_list[n + __popcll(bal & lanemask_lt())] = (uint8_t)idx;
+    n += __popcll(bal);
+  }
+  return n;
+}
+
 // Block id -> logical id so that each of the 8 XCDs (dispatch is round-robin
 // over XCDs) receives a contiguous run of logical work items: neighbouring
 // tiles share Gaussians, so this keeps their gathers in one L2.
