@@ -597,6 +597,7 @@ __device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t 
   // every wave sums into rows of its own with plain reads and writes: float
   // adds to LDS from 64 lanes took ~100 cycles each and held the kernel
   __shared__ __align__(16) float s_acc[4][kSub * kVals];  // [wave][entry][sum]
+  __shared__ int s_odd[4];
   if (item >= a.items[0]) return;
   const uint4 rec = reinterpret_cast<const uint4*>(a.items)[1 + item];
   const int tile = __builtin_amdgcn_readfirstlane((int)rec.x);
@@ -606,6 +607,7 @@ __device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t 
   const uint32_t cend = min(cstart + 256, maxc);
   const int tx = tile % a.gx, ty = tile / a.gx;
   const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+  bool odd = false;  // something here is not finite: it must not meet the weight 0 of a pair that does not blend
   {
     int pdx, pdy;
     tile_pixel(threadIdx.x, pdx, pdy);
@@ -631,6 +633,7 @@ __device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t 
         R += (a.accum[2 * HW + pix] - ck[768]) * d2;
       }
     }
+    odd = !(fabsf(R) + fabsf(d0) + fabsf(d1) + fabsf(d2) < __builtin_inff());
     const int slot = ((pdy >> 2) * 4 + (pdx >> 2)) * 16 + (pdy & 3) * 4 + (pdx & 3);
     s_tr[slot] = make_float2(T, R);
     s_last[slot] = last;
@@ -652,13 +655,16 @@ __device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t 
       s_a[threadIdx.x] = sa;
       s_b[threadIdx.x] = make_float4(sb.x, sb.y, sc.x, sc.y);
       s_c[threadIdx.x] = sc.z;
+      odd |= !(fabsf(sc.x) + fabsf(sc.y) + fabsf(sc.z) < __builtin_inff());
       m = splat_cells(sa.x, sa.y, sa.z, sa.w, sb.x, sb.y, (float)(tx * kBX), (float)(ty * kBY));
     }
     s_mask[threadIdx.x] = (uint16_t)m;
   }
   for (int i = threadIdx.x; i < 4 * kVals * kSub / 4; i += 256)
     reinterpret_cast<float4*>(&s_acc[0][0])[i] = make_float4(0.f, 0.f, 0.f, 0.f);
+  if (const uint64_t bal = __ballot(odd); lane == 0) s_odd[wv] = bal != 0;
   __syncthreads();
+  const bool any_odd = __builtin_amdgcn_readfirstlane(s_odd[0] | s_odd[1] | s_odd[2] | s_odd[3]);
   uint32_t hits[kSub / 64];
 #pragma unroll
   for (int c = 0; c < kSub / 64; ++c) hits[c] = s_mask[c * 64 + lane];
@@ -721,6 +727,9 @@ __device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t 
         inv[q] = __builtin_amdgcn_rcpf(1.0f - alpha[q]);
         d[q] = fmaf(cb, dc2[q], fmaf(gb.w, dc1[q], gb.z * dc0[q]));
       }
+      if (any_odd)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) d[q] = alpha[q] != 0.0f ? d[q] : 0.0f;
       // T before each entry from T after the group, and the sum behind it
       float Q[4], Tb[4], w[4], X[4], S[4];
 #pragma unroll
@@ -735,7 +744,8 @@ __device__ __forceinline__ void render_bwd_cells_item(const RBArgs& a, uint32_t 
       float m0 = 0.f, m1 = 0.f, m2 = 0.f, c0 = 0.f, c1 = 0.f, c2 = 0.f;
 #pragma unroll
       for (int q = 0; q < 4; ++q) {
-        const float g = G[q] * fmaf(Tb[q], d[q], -(S[q] * inv[q]));
+        float g = G[q] * fmaf(Tb[q], d[q], -(S[q] * inv[q]));
+        if (any_odd) g = alpha[q] != 0.0f ? g : 0.0f;
         const float t = fmaf(sh, dx, dy[q]), gt = g * t;
         m0 += g;
         m1 += gt;

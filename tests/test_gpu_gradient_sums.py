@@ -1,17 +1,20 @@
-"""The render backward's sums, where another grouping shows.
+"""The render backward's sums, where another grouping or a value that is not
+finite shows.
 
 * Scenes whose rotation gradients are decided by the rounding of one thin,
   tilted splat's second moments: in the fixed-order mode that splat's gradients
   are the recorded ones of the reference formula summed pixel by pixel (the
   same operations in the same order, so to the bit; 1e-6 of the row's norm is
   allowed for another compiler's contractions).  Sums by 4 x 4-pixel cells differ
-  from them by 5e-5 to 2e-4."""
+  from them by 5e-5 to 2e-4.
+* A splat that no pixel blends has no influence on any gradient, whatever its
+  colour."""
 import random
 
 import pytest
 import torch
 
-from gpu_helpers import DEV
+from gpu_helpers import DEV, np_
 from gs_hip import camera as gcam
 from gs_hip import raster, scenes
 
@@ -47,3 +50,40 @@ def test_thin_splat_of_a_scene(i):
         want = torch.tensor([float.fromhex(x) for x in want], dtype=torch.float64)
         err = float((g[name][row].cpu().double() - want).norm() / want.norm())
         assert err <= 1e-6, (name, err)
+
+
+@pytest.mark.parametrize("posed", [False, True], ids=["no pose", "pose"])
+@pytest.mark.parametrize("det", [False, True], ids=["atomic", "fixed order"])
+def test_a_splat_that_no_pixel_blends(det, posed):
+    """The last splat's alpha is 1/255 only within 0.4 pixels of its centre, which
+    lies half a pixel off the next ones: the reach test lets it pass, no pixel
+    takes it.  A finite colour and an infinite one give the same gradients."""
+    print("splat that no pixel blends", det, posed, flush=True)
+    n, W, H = 40, 21, 18
+    sc = scenes.plain_scene(seed=5, P=n + 1, W=W, H=H)
+    g = torch.Generator().manual_seed(6)
+    sc["means"][:n] = torch.cat([(torch.rand((n, 2), generator=g) - 0.5) * 2, 2 + torch.rand((n, 1), generator=g)], 1)
+    sc["scales"][:n] = 0.3
+    sc["opacities"][:n] = 0.05
+    fx = W / (2 * sc["cam"].tanfovx)
+    sc["means"][n] = torch.tensor([0.5 * 2.5 / fx, 0.0, 2.5])  # column 10.5, row 8.5, between the others
+    sc["scales"][n] = 25.0 / fx  # 10 pixels
+    sc["opacities"][n] = 1.0005 / 255.0
+    v = {k: sc[k].to(DEV) for k in ("means", "opacities", "scales", "rotations")}
+    pose = torch.tensor([0.0, 0.0, 0.0, 0.0, 0.0, 0.0, 1.0], device=DEV) if posed else None
+    rs = gcam.raster_settings(sc["cam"].to(DEV), torch.zeros(3, device=DEV), 0)
+    dc = (torch.rand((3, H, W), generator=g) - 0.5).to(DEV)
+    got = []
+    for last in (0.5, float("inf")):
+        colors = torch.rand((n + 1, 3), generator=torch.Generator().manual_seed(7)).to(DEV)
+        colors[n] = last
+        args = (v["means"], None, colors, v["opacities"], v["scales"], v["rotations"], None)
+        color, radii, _, _, st = raster.forward(rs, *args, pose=pose)
+        assert int(radii[n]) > 0 and bool(torch.isfinite(color).all())
+        b = raster.backward(rs, st, *args, pose, dc, None, None, deterministic=det)
+        assert not np_(b["colors"][n]).any()  # no pixel took it
+        got.append({k: t for k, t in b.items() if t is not None})
+    for k, t in got[0].items():
+        assert bool(torch.isfinite(got[1][k]).all()), k
+        if det:
+            assert torch.equal(t, got[1][k]), k
