@@ -816,6 +816,7 @@ __device__ __forceinline__ void blend_block(const BlendArgs& a, uint32_t tile, i
     id = id_at(1);
     uint32_t have = 0;   // entries in the slots
     uint32_t count = 0;  // entries kept of this 256-entry batch
+    uint64_t odd = 0;    // a colour in the slots is not finite
     uint32_t w = 0;
     for (; w < nwin; ++w) {
       const float4 ea = sa, eb = sb, ec = sc;
@@ -846,8 +847,9 @@ __device__ __forceinline__ void blend_block(const BlendArgs& a, uint32_t tile, i
         s_ch[slot] = make_float4(ec.x, ec.y, ec.z, eb.z);
         s_pos[slot] = pos + 1u;
       }
-      // a colour that is not finite must not meet a weight of zero
-      const bool odd = __ballot(hit && !(fabsf(ec.x) + fabsf(ec.y) + fabsf(ec.z) < __builtin_inff())) != 0;
+      // a colour that is not finite must not meet a weight of zero: one of this
+      // window's, or of the entries left over from the last
+      odd = (have > 0 ? odd : 0ull) | __ballot(hit && !(fabsf(ec.x) + fabsf(ec.y) + fabsf(ec.z) < __builtin_inff()));
       have += (uint32_t)__popcll(hits);
       count += (uint32_t)__popcll(hits);
       const bool flush = (w & 3u) == 3u || w + 1 == nwin;
@@ -885,7 +887,7 @@ __device__ __forceinline__ void blend_block(const BlendArgs& a, uint32_t tile, i
           T = ok ? Ti : T;
         }
         done = done || !ok;
-        if (!odd) {
+        if (odd == 0) {
 #pragma unroll
           for (int i = 0; i < kGroup; ++i)
 #pragma unroll
