@@ -101,8 +101,8 @@ struct RBArgs {
 
 // One workgroup orders the backward's work items.  A tile's items are its
 // 256-entry chunks up to its last contributor; the forward's blend logged
-// them with a cost class from the longest per-wave list it had in the same
-// batch, which the render backward's time per chunk follows closely.  Items
+// them with a cost class from the entries its waves kept of the same batch,
+// which the render backward's time per chunk follows closely.  Items
 // are handed out longest first (longest-processing-time order): a large frame
 // has more items than fit on the GPU at once, and an item that starts late
 // and runs long keeps the launch going after the rest have drained.  This is
@@ -833,26 +833,16 @@ __global__ __launch_bounds__(256) void k_render_bwd_cells(RBArgs a) {
 
 // Many frames in one launch: frame f owns blocks [prefix[f], prefix[f + 1]),
 // an upper bound on its work items.
-__device__ __forceinline__ int frame_of_item(const uint32_t* prefix, int n, uint32_t b) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (prefix[mid] <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
 template <bool DET, bool DEP>
 __global__ __launch_bounds__(256) void k_render_bwd_multi(const uint32_t* prefix, const RBArgs* args, int n) {
-  const int f = frame_of_item(prefix, n, blockIdx.x);
+  const int f = frame_of_block(prefix, n, blockIdx.x);
   const RBArgs a = args[f];
   render_bwd_item<DET, DEP>(a, blockIdx.x - prefix[f]);
 }
 
 template <bool PO>
 __global__ __launch_bounds__(256) void k_render_bwd_cells_multi(const uint32_t* prefix, const RBArgs* args, int n) {
-  const int f = frame_of_item(prefix, n, blockIdx.x);
+  const int f = frame_of_block(prefix, n, blockIdx.x);
   const RBArgs a = args[f];
   render_bwd_cells_item<PO>(a, blockIdx.x - prefix[f]);
 }

@@ -235,45 +235,17 @@ __device__ __forceinline__ void tile_rect(float px, float py, int r, int gx, int
   y1 = min(gy, max(0, sat_i((((py + rr) + (float)kBY) - 1.0f) / (float)kBY)));
 }
 
-__device__ __forceinline__ float wave_sum(float v) {
-  v += dpp<0xB1>(v);   // quad_perm [1,0,3,2]
-  v += dpp<0x4E>(v);   // quad_perm [2,3,0,1]
-  v += dpp<0x141>(v);  // row_half_mirror
-  v += dpp<0x140>(v);  // row_mirror
-  const float r0 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 0));
-  const float r1 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 16));
-  const float r2 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 32));
-  const float r3 = __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, v), 48));
-  return (r0 + r1) + (r2 + r3);
-}
-
-// Block copies between global memory and LDS for 256-thread workgroups,
-// n16 16-byte vectors.  Every thread issues all of its (up to 12) loads
-// before its first store, so a workgroup has its whole block in flight at
-// once instead of one load-to-store round trip per vector (the SH rows of
-// 256 Gaussians at M = 16 are exactly 12 vectors per thread).
-// (The loads are unconditional, clamped to the last vector, so the staging
-// array is fully written and stays in registers.)  dst and src must not overlap.
-__device__ __forceinline__ void block_copy16(float4* __restrict__ dst, const float4* __restrict__ src, int n16) {
-  constexpr int kMax = 12;
-  if (n16 <= 0) return;
-  float4 v[kMax];
-#pragma unroll
-  for (int r = 0; r < kMax; ++r) v[r] = src[min((int)threadIdx.x + r * 256, n16 - 1)];
-  // stores clamped the same way: the duplicates write the last vector's own
-  // value to it again, and no store waits inside a branch for its load
-#pragma unroll
-  for (int r = 0; r < kMax; ++r) dst[min((int)threadIdx.x + r * 256, n16 - 1)] = v[r];
-  for (int k = (int)threadIdx.x + kMax * 256; k < n16; k += 256) dst[k] = src[k];
-}
-
 // Rows of `per4` 16-byte vectors, contiguous in global memory, into LDS rows
 // of `prow` floats.  A thread that then works on its own row reads
 // LDS at a stride of prow words across the wave: an odd prow puts the 64
 // lanes on 64 different banks (a stride of 48 puts them on 4).  The row /
 // column of vector k = threadIdx.x + 256 r advance by constant steps, so no
-// division per vector.  Loads come first, clamped to the last vector, as in
-// block_copy16.  256 threads.
+// division per vector.  Every thread issues all of its (up to 12) loads before
+// its first store, so a workgroup has its whole block in flight at once instead
+// of one load-to-store round trip per vector (the SH rows of 256 Gaussians at M
+// = 16 are exactly 12 vectors per thread); loads and stores are unconditional,
+// clamped to the last vector, so the staging array stays in registers.  256
+// threads; dst and src must not overlap.
 __device__ __forceinline__ void rows_to_lds(float* __restrict__ dst, const float4* __restrict__ src, int nrows,
                                             int per4, int prow) {
   constexpr int kMax = 12;
@@ -509,6 +481,19 @@ __device__ __forceinline__ int compact_wave_list(const uint32_t* s_mask, uint8_t
     n += __popcll(bal);
   }
   return n;
+}
+
+// Frame f of a set whose per-frame block counts have the exclusive prefix
+// `prefix`: the last f with prefix[f] <= b (frames owning no block share their
+// start with the next).
+__device__ __forceinline__ int frame_of_block(const uint32_t* prefix, int n, uint32_t b) {
+  int lo = 0, hi = n - 1;
+  while (lo < hi) {
+    const int mid = (lo + hi + 1) >> 1;
+    if (prefix[mid] <= b) lo = mid;
+    else hi = mid - 1;
+  }
+  return lo;
 }
 
 // Block id -> logical id so that each of the 8 XCDs (dispatch is round-robin

@@ -223,18 +223,6 @@ __global__ __launch_bounds__(256) void k_preprocess(PreArgs a) {
   preprocess_block(a, blockIdx.x, gridDim.x, s_sh);
 }
 
-// The block of many frames' launch that frame f owns: the last f with
-// prefix[f] <= b (frames owning no block share their start with the next).
-__device__ __forceinline__ int frame_of_block(const uint32_t* prefix, int n, uint32_t b) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (prefix[mid] <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
 // Many frames' preprocess in one launch: frame f owns workgroups [prefix[f],
 // prefix[f + 1]); the dynamic LDS covers the largest frame's SH rows.
 __global__ __launch_bounds__(256) void k_preprocess_multi(const uint32_t* prefix, const PreArgs* args, int n) {
@@ -982,7 +970,9 @@ __device__ __forceinline__ uint32_t blend_rank(uint32_t b, int& part) {
 // instructions count, of which the smaller blocks issue more.  8 x 8 / 4 x 4,
 // us: 46 / 26 at 256 tiles, 100 / 50 at 510, 87 / 50 at 858, 87 / 79 and
 // 100 / 77 at 1 170 - 1 450 (training scenes), but 73 / 82 at 920 and 71 / 109
-// at 2 040 for sparse views; 107 / 108 at 2 040, 270 / 564 at 8 160.
+// at 2 040 for sparse views; 107 / 108 at 2 040, 270 / 564 at 8 160.  (The tiles
+// alone do not tell: training scenes gain from 4 x 4 blocks beyond this line,
+// sparse views lose before it.  It lies where neither loses much.)
 constexpr int kCellTiles = 1024;
 inline unsigned blend_grid(unsigned tiles, int e) { return (tiles + 7u) / 8u * 32u * (unsigned)e; }
 
@@ -993,18 +983,6 @@ __global__ __launch_bounds__(64) void k_blend(BlendArgs a, uint32_t tiles) {
   if (r < tiles) blend_block<E>(a, a.tile_order[r], part);
 }
 
-// Frame f of a set whose per-frame block counts have the exclusive prefix
-// `prefix` (n + 1 entries): the last f with prefix[f] <= b.
-__device__ __forceinline__ int frame_of(const uint32_t* prefix, int n, uint32_t b) {
-  int lo = 0, hi = n - 1;
-  while (lo < hi) {
-    const int mid = (lo + hi + 1) >> 1;
-    if (prefix[mid] <= b) lo = mid;
-    else hi = mid - 1;
-  }
-  return lo;
-}
-
 // Blend of many frames in one launch: one workgroup per tile of every frame
 // (each frame's tiles in its longest-first order).
 template <int E>
@@ -1012,7 +990,7 @@ __global__ __launch_bounds__(64) void k_blend_multi(const uint32_t* prefix, cons
   int part;
   const uint32_t r = blend_rank<E>(blockIdx.x, part);
   if (r >= prefix[n]) return;
-  const int f = frame_of(prefix, n, r);
+  const int f = frame_of_block(prefix, n, r);
   const BlendArgs a = args[f];
   blend_block<E>(a, a.tile_order[r - prefix[f]], part);
 }

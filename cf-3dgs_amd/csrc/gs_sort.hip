@@ -11,13 +11,14 @@
 //
 // A sort of B bits takes ceil(B / 8) passes of near equal digits; a keys-only
 // sort of 9 or 10 bits (the lists of up to 1024 tiles) takes one pass.  Per pass:
-//   k_sort_upsweep  1024 or 2048 keys per workgroup (4096 with 10-bit digits),
-//                   4 waves x 4, 8 or 16 rounds x 64 lanes, all loaded up
+//   k_sort_upsweep  1024 or 2048 keys per workgroup (4096 with 10-bit digits and
+//                   past 2^24 keys), 4 waves x 4, 8 or 16 rounds x 64 lanes, all loaded up
 //                   front, counted with one LDS atomic each -> per-workgroup
 //                   digit counts
 //   k_sort_scan     one workgroup per digit: exclusive scan of its row, total.
 //                   Sorts of up to kDirectBlocks workgroups have no such
-//                   launch: each scatter workgroup adds the counts up itself
+//                   launch (kSegDirectBlocks in a segmented sort): each
+//                   scatter workgroup adds the counts up itself
 //   k_sort_scatter  recomputes the matches; rank = prior count of the digit in
 //                   this wave + lanes below with the same digit; waves are
 //                   ordered by an exclusive prefix over the 4 wave counts, so
